@@ -169,13 +169,14 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    cost model's tile, 256 x 96 on the role-split kernel); f32 x: the
  *    exact-code f32 GEMM;
  *  - Q4_K / Q6_K weights (f32 x only, any m; bf16 x fails with RQ_ERR_DTYPE):
- *    x is quantized to q8_K in scratch and the K-quant GEMV runs, the same two
- *    kernels as rq_quantize_act_q8k + rq_qmatmul_q8k and bit for bit their
+ *    x is quantized to q8_K in scratch and the K-quant matmul runs, the same
+ *    arithmetic as rq_quantize_act_q8k + rq_qmatmul_q8k and bit for bit their
  *    results (QMatrix apply of the built-in :q4_K / :q6_K formats,
- *    raster/quant/core.clj:55-75). The GEMV takes four activation rows per
- *    pass over the weight, so a call streams the weight ceil(m / 4) times:
- *    meant for decode (m <= 16); at prefill sizes (m = 512: 128 passes) its
- *    time grows with m.
+ *    raster/quant/core.clj:55-75). m <= 4 is one GEMV pass over the
+ *    weight, larger m the K-quant GEMM (int8 MFMA on the codes times their
+ *    integer sub-block scales, exact per super-block of 256). Weights with a
+ *    Q4_K aq above 63 or a scale that is not finite run the GEMV at every m,
+ *    four activation rows per pass.
  *
  * Numerics (all accumulation in f32):
  *  - v_dot4 GEMV and int8-level decode kernel: each 32-block of each
@@ -312,9 +313,10 @@ int rq_quantize_act_q8k(rq_ctx ctx, const float* x, int64_t m, int64_t in, int s
 
 /* y[m, out] = the K dot of a Q4_K / Q6_K weight with q8_K activations
  * (qmatmul-q4k-dp4a! / qmatmul-q6k-dp4a!, raster/quant/kernels_k.clj:186-297):
- * exact int32 sub-block dots, the scale terms added in f32 (Raster: double).
- * bsums must use the weight's sub-block size. Decode-oriented: four activation
- * rows per pass over the weights. xq 16-byte aligned. */
+ * exact int32 dots, per sub-block (m <= 4) or per super-block with its integer
+ * scales (larger m), the scale terms added in f32 (Raster: double). bsums must
+ * be the codes' sums over the weight's sub-block size (the Q6_K GEMM forms the
+ * term from the codes themselves). xq 16-byte aligned. */
 int rq_qmatmul_q8k(rq_ctx ctx, rq_weight w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
                    int y_dtype, int64_t m, void* stream);
 

@@ -6,6 +6,7 @@
 // thread-local string (rq_last_error).
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <mutex>
 #include <new>
 #include <string>
@@ -602,7 +603,8 @@ int rq_weight_destroy(rq_weight h) {
 // K-quant weight from host arrays already in the resident order: codes
 // (qbytes), super-block scales (sbytes), sub-block scales (ubytes).
 static int make_weight_k(Ctx* c, int format, int64_t out, int64_t in, const void* codes, size_t qbytes,
-                         const void* sup, size_t sbytes, const void* sub, size_t ubytes, rq_weight* wout) {
+                         const void* sup, size_t sbytes, const void* sub, size_t ubytes, bool kq_gemm,
+                         rq_weight* wout) {
   if (int s = set_device(c)) return s;
   const size_t total = align256(qbytes) + align256(sbytes) + align256(ubytes);
   void* base = nullptr;
@@ -628,6 +630,7 @@ static int make_weight_k(Ctx* c, int format, int64_t out, int64_t in, const void
   w->scales = static_cast<uint8_t*>(base) + align256(qbytes);
   w->scales_rb = nullptr;
   w->sub_scales = static_cast<uint8_t*>(base) + align256(qbytes) + align256(sbytes);
+  w->kq_gemm = kq_gemm;
   w->bytes = total;
   w->ctx = c;
   e = hipMemcpy(w->q, codes, qbytes, hipMemcpyHostToDevice);
@@ -671,14 +674,21 @@ int rq_weight_create_q4k(rq_ctx h, const uint8_t* wq, const float* da, const flo
   if (int s = check_shape_k(RQ_Q4_K, out, in)) return s;
   const int64_t nsb = out * (in / 256), nsub = out * (in / 32);
   std::vector<float> sup((size_t)(2 * nsb));
+  // the GEMM (kquant_gemm.hip) needs 6-bit aq, and folds aq into integers, where
+  // an infinite da would not meet a zero aq as it does in the GEMV
+  bool gemm = true;
   for (int64_t i = 0; i < nsb; i++) {
     sup[(size_t)(2 * i)] = da[i];
     sup[(size_t)(2 * i + 1)] = db[i];
+    gemm = gemm && std::isfinite(da[i]) && std::isfinite(db[i]);
   }
   std::vector<uint16_t> sub((size_t)nsub);
-  for (int64_t i = 0; i < nsub; i++) sub[(size_t)i] = (uint16_t)(aq[i] | ((uint16_t)(uint8_t)bq[i] << 8));
+  for (int64_t i = 0; i < nsub; i++) {
+    gemm = gemm && aq[i] <= 63;
+    sub[(size_t)i] = (uint16_t)(aq[i] | ((uint16_t)(uint8_t)bq[i] << 8));
+  }
   return make_weight_k(c, RQ_Q4_K, out, in, wq, (size_t)(out * in / 2), sup.data(), sup.size() * 4, sub.data(),
-                       sub.size() * 2, w);
+                       sub.size() * 2, gemm, w);
 }
 
 int rq_weight_create_q6k(rq_ctx h, const uint8_t* wq, const int8_t* sc, const float* ds, int64_t out, int64_t in,
@@ -707,7 +717,8 @@ int rq_weight_create_q6k(rq_ctx h, const uint8_t* wq, const int8_t* sc, const fl
   }
   if (bad & 0xC0) return fail(RQ_ERR_SHAPE, "Q6_K codes must lie in 0..63");
   return make_weight_k(c, RQ_Q6_K, out, in, packed.data(), packed.size(), ds, (size_t)(out * (in / 256)) * 4, sc,
-                       (size_t)(out * (in / 16)), w);
+                       (size_t)(out * (in / 16)),
+                       std::all_of(ds, ds + out * (in / 256), [](float d) { return std::isfinite(d); }), w);
 }
 
 int rq_weight_info(rq_weight h, int* format, int64_t* out, int64_t* in, int* scale_dtype, size_t* bytes) {
@@ -781,8 +792,9 @@ static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t 
 }
 
 // A K-quant weight with f32 x in one call: x quantized to q8_K in scratch,
-// then the K-quant GEMV -- rq_quantize_act_q8k + rq_qmatmul_q8k, with the
-// same kernels and so the same results (QMatrix apply of the built-in :q4_K /
+// then the K-quant GEMV or GEMM -- rq_quantize_act_q8k + rq_qmatmul_q8k, with
+// the same arithmetic and so the same results (for the GEMM the quantizer
+// writes its operand order, in buffers of the same sizes) (QMatrix apply of the built-in :q4_K /
 // :q6_K formats, raster/quant/core.clj:55-75).
 static int run_kquant_matmul(Ctx* c, const Weight& w, const float* x, void* y, int y_dtype, int64_t m,
                              hipStream_t stream, FixedScratch* fixed) {
@@ -795,14 +807,17 @@ static int run_kquant_matmul(Ctx* c, const Weight& w, const float* x, void* y, i
   int8_t* xq = static_cast<int8_t*>(buf);
   float* xs = reinterpret_cast<float*>(static_cast<uint8_t*>(buf) + xq_b);
   int32_t* bs = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(buf) + xq_b + xs_b);
-  hipError_t e = launch_quantize_act_q8k(x, m, w.in, sub, xq, xs, bs, stream);
+  const bool gemm = kquant_gemm_takes(w, m);
+  hipError_t e = gemm ? launch_quantize_act_q8k_packed(x, m, w.in, sub, xq, xs, bs, stream)
+                      : launch_quantize_act_q8k(x, m, w.in, sub, xq, xs, bs, stream);
   if (e != hipSuccess) return hip_fail(e, "quantizer launch");
   const EvSet ev = fixed ? EvSet{} : timing_set(c, stream);
   if (ev.n) (void)hipEventRecord(ev.e[0], stream);
-  e = launch_kquant_gemv(w, xq, xs, bs, y, y_dtype, m, c->cu_count, stream);
+  e = gemm ? launch_kquant_gemm(w, xq, xs, bs, true, y, y_dtype, m, c->cu_count, stream)
+           : launch_kquant_gemv(w, xq, xs, bs, y, y_dtype, m, c->cu_count, stream);
   if (ev.n && e == hipSuccess) (void)hipEventRecord(ev.e[1], stream);
   timing_done(c, ev, e == hipSuccess);
-  if (e != hipSuccess) return hip_fail(e, "K-quant GEMV launch");
+  if (e != hipSuccess) return hip_fail(e, "K-quant matmul launch");
   return RQ_OK;
 }
 
@@ -1059,10 +1074,12 @@ int rq_qmatmul_q8k(rq_ctx h, rq_weight wh, const int8_t* xq, const float* xs, co
   if (int s = set_device(c)) return s;
   const EvSet ev = timing_set(c, (hipStream_t)stream);
   if (ev.n) (void)hipEventRecord(ev.e[0], (hipStream_t)stream);
-  hipError_t e = launch_kquant_gemv(w, xq, xs, bsums, y, y_dtype, m, c->cu_count, (hipStream_t)stream);
+  hipError_t e = kquant_gemm_takes(w, m)
+                     ? launch_kquant_gemm(w, xq, xs, bsums, false, y, y_dtype, m, c->cu_count, (hipStream_t)stream)
+                     : launch_kquant_gemv(w, xq, xs, bsums, y, y_dtype, m, c->cu_count, (hipStream_t)stream);
   if (ev.n && e == hipSuccess) (void)hipEventRecord(ev.e[1], (hipStream_t)stream);
   timing_done(c, ev, e == hipSuccess);
-  if (e != hipSuccess) return hip_fail(e, "K-quant GEMV launch");
+  if (e != hipSuccess) return hip_fail(e, "K-quant matmul launch");
   return RQ_OK;
 }
 

@@ -39,13 +39,6 @@ namespace rq {
 
 namespace {
 
-// Buffer resources over whole arrays. Offsets are 32-bit: a per-lane part
-// fixed for the kernel (clamped once, at the start) in a VGPR and the k
-// offset of the step, uniform, in an SGPR, so a load costs no VALU work.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t wd_rsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
-
 // One 32-column x 32-k weight unit for one lane: 16 elements of its column
 struct WdCodes {
   u32x4 v;     // Q8: codes k = 16 g + 0..15 of the lane's column; Q4: the column's 16 packed bytes
@@ -161,7 +154,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
   // + 16 lane; this wave's m fragments are r32 = m0 / 32 + f, clamped to the
   // packed rows (rows past M only feed outputs that are never stored)
   const int r32_last = (M + 31) / 32 - 1;
-  const __amdgpu_buffer_rsrc_t xr = wd_rsrc(xf, xf_bytes);
+  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(xf, xf_bytes);
   const uint32_t a_lo = 16u * lane;
   uint32_t a_row[2];
 #pragma unroll
@@ -169,8 +162,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     a_row[f] = (uint32_t)__builtin_amdgcn_readfirstlane(min(m0 / 32 + f, r32_last) * nkb);
   // weights: codes of npad/16 * nkb chunks, block-major scales npad * nkb
   constexpr uint32_t CB = FMT == RQ_Q8_0 ? 512u : 256u, RB = FMT == RQ_Q8_0 ? 32u : 16u;
-  const __amdgpu_buffer_rsrc_t qr = wd_rsrc(q, (uint32_t)(npad / 16) * (uint32_t)nkb * CB);
-  const __amdgpu_buffer_rsrc_t sr = wd_rsrc(sc, (uint32_t)npad * (uint32_t)nkb * (uint32_t)sizeof(ST));
+  const __amdgpu_buffer_rsrc_t qr = buffer_rsrc(q, (uint32_t)(npad / 16) * (uint32_t)nkb * CB);
+  const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(sc, (uint32_t)npad * (uint32_t)nkb * (uint32_t)sizeof(ST));
   // this wave's dequant units u = wave + 4 i: n fragment u % NF, k-step u / NF.
   // The lane's column n0 + 32 c + lane % 32 is row lane % 16 of 16-row group
   // n0 / 16 + 2 c + (lane % 32) / 16 (clamped to the padded rows).
@@ -458,7 +451,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   if (wave < 4) {
     // ---- consumer ----
     const int r32_last = (M + 31) / 32 - 1;
-    const __amdgpu_buffer_rsrc_t xr = wd_rsrc(xf, xf_bytes);
+    const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(xf, xf_bytes);
     const uint32_t a_lo = 16u * lane;
     uint32_t a_row[2];
 #pragma unroll
@@ -626,8 +619,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   // ---- producer ----
   const int p = wave - 4;
   constexpr uint32_t CB = FMT == RQ_Q8_0 ? 512u : 256u, RB = FMT == RQ_Q8_0 ? 32u : 16u;
-  const __amdgpu_buffer_rsrc_t qr = wd_rsrc(q, (uint32_t)(npad / 16) * (uint32_t)nkb * CB);
-  const __amdgpu_buffer_rsrc_t sr = wd_rsrc(sc, (uint32_t)npad * (uint32_t)nkb * (uint32_t)sizeof(ST));
+  const __amdgpu_buffer_rsrc_t qr = buffer_rsrc(q, (uint32_t)(npad / 16) * (uint32_t)nkb * CB);
+  const __amdgpu_buffer_rsrc_t sr = buffer_rsrc(sc, (uint32_t)npad * (uint32_t)nkb * (uint32_t)sizeof(ST));
   const bool has2 = p + 4 < NU;  // the second unit (waves 4, 5 at NF 3; all at NF 4)
   const int g_last = npad / 16 - 1;
   int uu[2];

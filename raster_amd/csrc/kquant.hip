@@ -81,6 +81,70 @@ __global__ __launch_bounds__(kKqThreads) void quantize_act_q8k_kernel(const floa
   }
 }
 
+// The same codes in the operand order of the K-quant GEMM (kquant_gemm.hip):
+// per 16-row tile (the last one R = m % 16 rows if that is not 0) and 64-element
+// step one fragment, 16 bytes per (k group of 16, row); xs as [tile][super-block]
+// [row]; for SUB 32 the block sums as the f16 digits 64 h + l of the minimum
+// term's operand, 8 bytes per (slot group, row): slots 0..7 h, 8..15 l of the 8
+// sub-blocks (SUB 16: not stored, the GEMM does not use them). The buffers have
+// the sizes of the row-major form. A wave takes one super-block of 4 rows, 16
+// elements per lane, so every store instruction writes runs of 64 bytes.
+template <int SUB>
+__global__ __launch_bounds__(kKqThreads) void quantize_act_q8k_packed_kernel(const float* __restrict__ x,
+                                                                            int8_t* __restrict__ xq,
+                                                                            float* __restrict__ xs,
+                                                                            int32_t* __restrict__ bsums, int64_t M,
+                                                                            int nsb) {
+  const int lane = threadIdx.x & 63, ch = lane & 15;
+  const int64_t wv = (int64_t)blockIdx.x * (kKqThreads / 64) + (threadIdx.x >> 6);
+  const int64_t row = wv / nsb * 4 + (lane >> 4), sb = wv % nsb;
+  const bool live = row < M;
+  const float* src = x + ((live ? row : M - 1) * nsb + sb) * 256 + ch * 16;
+  f32x4 v[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) v[i] = reinterpret_cast<const f32x4*>(src)[i];
+  float a = 0.0f;
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    a = fmaxf(a, fmaxf(fmaxf(fabsf(v[i][0]), fabsf(v[i][1])), fmaxf(fabsf(v[i][2]), fabsf(v[i][3]))));
+#pragma unroll
+  for (int off = 8; off >= 1; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
+  const double d = (double)a / 127.0;
+  const double id = d == 0.0 ? 0.0 : 1.0 / d;
+  u32x4 w = {0u, 0u, 0u, 0u};
+  int s = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    const int q = java_round_clamp127((double)v[i / 4][i % 4] * id);
+    w[i / 4] |= (uint32_t)(q & 0xFF) << (8 * (i % 4));
+    s += q;
+  }
+  if (SUB == 32) s += __shfl_xor(s, 1, 64);
+  if (!live) return;
+  const int64_t t16 = row >> 4, R = M - 16 * t16 < 16 ? M - 16 * t16 : 16, r = row & 15;
+  *reinterpret_cast<u32x4*>(xq + t16 * 16 * nsb * 256 + (4 * sb + (ch >> 2)) * 64 * R + ((ch & 3) * R + r) * 16) = w;
+  if (ch == 0) xs[t16 * 16 * nsb + sb * R + r] = (float)d;
+  if (SUB == 32) {
+    const int slot = (ch & 1) * 8 + (ch >> 1);  // even lanes h, odd lanes l
+    reinterpret_cast<_Float16*>(bsums)[(t16 * 16 * nsb + sb * R) * 16 + ((slot >> 2) * R + r) * 4 + (slot & 3)] =
+        (_Float16)((ch & 1) ? s & 63 : s >> 6);
+  }
+}
+
+hipError_t launch_quantize_act_q8k_packed(const float* x, int64_t m, int64_t in, int sub, int8_t* xq, float* xs,
+                                          int32_t* bsums, hipStream_t stream) {
+  const int64_t waves = (m + 3) / 4 * (in / 256);
+  if (waves == 0) return hipSuccess;
+  const dim3 grid((unsigned)((waves + kKqThreads / 64 - 1) / (kKqThreads / 64)));
+  if (sub == 32)
+    hipLaunchKernelGGL((quantize_act_q8k_packed_kernel<32>), grid, dim3(kKqThreads), 0, stream, x, xq, xs, bsums, m,
+                       (int)(in / 256));
+  else
+    hipLaunchKernelGGL((quantize_act_q8k_packed_kernel<16>), grid, dim3(kKqThreads), 0, stream, x, xq, xs, bsums, m,
+                       (int)(in / 256));
+  return hipGetLastError();
+}
+
 hipError_t launch_quantize_act_q8k(const float* x, int64_t m, int64_t in, int sub, int8_t* xq, float* xs,
                                    int32_t* bsums, hipStream_t stream) {
   const int64_t nsb = m * (in / 256);

@@ -48,6 +48,7 @@ struct Weight {
   // K-quants (RQ_Q4_K / RQ_Q6_K) keep Raster's row-major codes in q, the
   // super-block scales in `scales` (Q4_K: da, db side by side) and these:
   void* sub_scales;  // per (row, sub-block): Q4_K aq, bq side by side; Q6_K sc
+  bool kq_gemm;      // scales the GEMM's digits hold: all finite, Q4_K: every aq <= 63
   size_t bytes;
   struct Ctx* ctx;
 };
@@ -197,6 +198,13 @@ hipError_t launch_quantize_act_q8k(const float* x, int64_t m, int64_t in, int su
 size_t kquant_gemv_lds(int format, int64_t k, int mt);
 hipError_t launch_kquant_gemv(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
                               int y_dtype, int64_t m, int cu_count, hipStream_t stream);
+// K-quant GEMM on int8 MFMA (kquant_gemm.hip): whether it takes a call, and the call
+bool kquant_gemm_takes(const Weight& w, int64_t m);
+hipError_t launch_kquant_gemm(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, bool packed,
+                              void* y, int y_dtype, int64_t m, int cu_count, hipStream_t stream);
+// q8_K activations in that kernel's operand order, in buffers of the row-major form's sizes
+hipError_t launch_quantize_act_q8k_packed(const float* x, int64_t m, int64_t in, int sub, int8_t* xq, float* xs,
+                                          int32_t* bsums, hipStream_t stream);
 hipError_t launch_kquant_dequant(const Weight& w, float* out, hipStream_t stream);
 // backward-data on f32 MFMA for m <= kDxFmMaxRows (dx.hip): the weight as
 // stored feeds the MFMA's B operand; column tiles x dy-row tiles x slices of
@@ -253,6 +261,13 @@ hipError_t launch_chunk_weight(int format, int scale_dtype, const uint8_t* q_rm,
 template <typename T>
 __device__ __forceinline__ const __attribute__((address_space(1))) T* as_global(const T* p) {
   return (const __attribute__((address_space(1))) T*)p;
+}
+
+// Buffer resource over a whole array. Offsets are 32-bit: a per-lane part
+// fixed for the kernel (clamped once, at the start) in a VGPR and the k
+// offset of the step, uniform, in an SGPR, so a load costs no VALU work.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_rsrc(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
 }
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b) { return __uint_as_float(b << 16); }
