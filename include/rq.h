@@ -207,6 +207,11 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  * do not share it):
  *  - bf16 x with m > 16, except in the weight-stream GEMM (which reads x as
  *    it is): the packed activation tile, ceil(m/32)*32*in*2 bytes;
+ *  - f32 x with m > 16 (Q8_0, Q4_0): the activations as bf16 hi + lo,
+ *    ceil(m/32)*32*in*4 bytes, at most RQ_NOALLOC_SCRATCH_MAX (a larger call
+ *    runs in row chunks). A call that cannot have it (captured before the
+ *    stream's scratch was grown, device memory full) reads x itself, slower,
+ *    with the same results;
  *  - K-slices' partial sums, m * out * 4 bytes per slice, added in slice
  *    order by a second kernel: the int8-level decode kernel when a row of x
  *    does not fit one workgroup's LDS (in above 17472 at m <= 4, 8704 at
@@ -219,7 +224,8 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    bytes (each part rounded up to 256), sub = 32 for Q4_K, 16 for Q6_K.
  * Under HIP graph capture nothing can be allocated: run the same (or a
  * larger) shape once on the capturing stream before capturing, otherwise the
- * call fails with RQ_ERR_SHAPE and a message saying so. A buffer that grows is
+ * call fails with RQ_ERR_SHAPE and a message saying so (except f32 x with
+ * m > 16, as above). A buffer that grows is
  * replaced but not freed until rq_ctx_destroy, so a graph captured before a
  * larger call still replays on its own (still allocated) buffers; graphs and
  * eager calls on one stream share a buffer only while it has not grown, and

@@ -931,6 +931,11 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
     // 16-row tile and 32-block
     const size_t bytes = (size_t)((m + 15) / 16) * (size_t)(w.in / 32) * 640;
     if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch)) return s;
+  } else if (!plan.ok) {
+    // bf16 hi + lo copy of the f32 activations; a call that cannot have the
+    // scratch (captured before it was grown, memory full) reads x itself
+    const size_t bytes = gemm_f32_pack_bytes(m, w.in);
+    if (bytes == 0 || call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch) != RQ_OK) a.scratch = nullptr;
   }
   a.part = static_cast<float*>(part);
   // no timing events for calls that allocate nothing (creating one allocates);

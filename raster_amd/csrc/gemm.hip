@@ -1,214 +1,666 @@
-// gemm.hip — prefill-regime (m > 16) block-quantized GEMM on CDNA4 MFMA.
+// gemm.hip — prefill-regime (m > 16) block-quantized GEMM for f32 activations on
+// CDNA4 MFMA.
 //
 // y[m, o] = sum_b scale[o, b] * P_b[m, o],  P_b = sum_{k in block b} x[m, k] * code[o, k]
 //
 // Raster's staged contraction (raster/compiler/ir/contract_stages.clj:25-31):
-// the inner sum over one 32-element block runs on v_mfma_f32_16x16x32_bf16 whose
-// K is exactly one quant block; the codes enter the MFMA as bf16 integers, which
-// is exact (|code| <= 128 needs 8 significand bits), so the dequantized tile in
-// LDS is bit-exact and every product is exact in f32. The f32 block scale then
-// multiplies the f32 partial (one FMA per output per block).
+// the codes enter v_mfma_f32_32x32x16_bf16 as bf16 integers, which is exact
+// (|code| <= 128 needs 8 significand bits), so every product is exact in f32;
+// the f32 block scale then multiplies the f32 partial of the block (one FMA per
+// output per block). x is carried as bf16 hi + lo (x = hi + lo + O(2^-17 |x|)),
+// two MFMAs per product.
 //
-// f32 activations are split into bf16 hi + lo (x = hi + lo + O(2^-17 |x|)) and
-// take two MFMAs per tile. This is the f32-activation path; bf16 activations
-// take gemm_bf16_kernel.
-//
-// Tiling: 256 threads = 4 waves (2 x 2), block tile 128 (m) x 128 (o), each wave
-// 64 x 64 = 4 x 4 MFMA tiles. Weights are the B operand so each lane's four
-// outputs of a tile share one column o and one scale. LDS is double-buffered:
-// the next block's global loads are in flight while the current one computes.
-// Block ids are remapped so the m-tiles that share a weight tile run on the same
-// XCD (one L2 fetch of the weight tile per XCD).
+// Bound: the MFMAs (twice the bf16 GEMM's) and, at the operand rates of a CU,
+// the activations: 4 bytes per element, so a fragment is loaded once per wave
+// and used for 96 or 192 columns. Measured (128 x 96 tile, per MFMA and wave):
+// 24 ns, of it 16.5 the MFMA itself, about 4 the activation loads and the
+// producers, 2 the LDS reads, 2 the block scaling.
+#include <algorithm>
+
 #include "rq_internal.h"
 
 namespace rq {
 
-constexpr int GBM = 128, GBN = 128;
-constexpr int LDA = 40;  // bf16 per LDS row: 32 + 8 padding (80 B stride spreads banks)
+namespace {
 
-__device__ __forceinline__ uint32_t pack_bf16_exact(float lo, float hi) {
-  // lo/hi are small integers: the bf16 is the top half of the f32, exactly
-  return (__float_as_uint(lo) >> 16) | (__float_as_uint(hi) & 0xFFFF0000u);
+constexpr int kGbBlocks = 4;  // 32-blocks per step
+
+// x = hi + lo, both RNE bf16, eight elements
+__device__ __forceinline__ void split8(const f32x4& v0, const f32x4& v1, u32x4& hi, u32x4& lo) {
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const float a = i < 2 ? v0[2 * i] : v1[2 * i - 4], b = i < 2 ? v0[2 * i + 1] : v1[2 * i - 3];
+    hi[i] = pack2_bf16(a, b);
+    lo[i] = pack2_bf16(a - __uint_as_float(hi[i] << 16), b - __uint_as_float(hi[i] & 0xFFFF0000u));
+  }
 }
 
-template <int FMT, typename ST, int XT>
-__global__ __launch_bounds__(256) void gemm_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc,
-                                                  const void* __restrict__ x, void* __restrict__ y, int M,
-                                                  int K, int N, int y_dtype, int tiles_m) {
-  constexpr int NA = XT == RQ_F32 ? 2 : 1;
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][NA][GBM * LDA];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[2][GBN * LDA];
-  __shared__ float Ss[2][GBN];
+}  // namespace
 
-  // XCD-aware order: block b runs on XCD b % 8; give each XCD a contiguous run.
-  const int nblk = gridDim.x, b = blockIdx.x;
-  const int xcd = b & 7, per = nblk >> 3, rem = nblk & 7;
-  const int tile = xcd * per + (xcd < rem ? xcd : rem) + (b >> 3);
-  const int tn = tile / tiles_m, tm = tile - tn * tiles_m;
-  const int m0 = tm * GBM, n0 = tn * GBN;
+// x[M][K] (f32) -> xf[M/32][K/32][hi, lo][2][64][8] bf16: fragment (tile, kb,
+// hl, j), lane l = row l % 32 of the tile, k = 32 kb + 16 (l / 32) + 8 j + 0..7.
+// Rows up to the next multiple of 32 are zero. A workgroup copies 32 rows x 64 k.
+__global__ __launch_bounds__(256) void pack_x32_split_kernel(const float* __restrict__ x, uint16_t* __restrict__ xf,
+                                                             int M, int K) {
+  const int nkb = K / 32, nq = (nkb + 1) / 2;
+  const int tile = blockIdx.x / nq, kb = (blockIdx.x % nq) * 2 + ((threadIdx.x & 7) >> 2);
+  if (kb >= nkb) return;
+  const int row = threadIdx.x >> 3, cc = threadIdx.x & 3;  // 8-k chunk cc of the k-step
+  const int m = tile * 32 + row;
+  f32x4 v0 = {0.0f, 0.0f, 0.0f, 0.0f}, v1 = v0;
+  if (m < M) {
+    const f32x4* p = reinterpret_cast<const f32x4*>(x + (int64_t)m * K + 32 * kb + 8 * cc);
+    v0 = p[0];
+    v1 = p[1];
+  }
+  u32x4 hi, lo;
+  split8(v0, v1, hi, lo);
+  const int j = cc & 1, lane = row + 32 * (cc >> 1);
+  u32x4* dst = reinterpret_cast<u32x4*>(xf) + (((int64_t)tile * nkb + kb) * 4 + j) * 64 + lane;
+  dst[0] = hi;
+  dst[128] = lo;
+}
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int nkb = K / 32;
-  const int lrow = tid >> 1, lhalf = tid & 1;
+// Workgroup: WM x KG waves; tile 32 MF WM rows x 32 NF columns, a wave 32 MF x
+// 32 NF of it over the steps s (of four 32-blocks) with s % KG = its kg (their
+// sums are added in kg order at the end). All waves convert the next KG steps'
+// codes to bf16 (16 codes per thread and task) into the other half of a
+// double-buffered LDS ring while the current ones compute; one barrier per KG
+// steps. Activation fragments go straight into registers, a block ahead: from
+// the packed copy, or (PK false: calls that have no scratch) from x itself,
+// split in registers, with the same result.
+template <int FMT, typename ST, bool PK, int MF, int NF, int WM, int KG>
+__global__ __attribute__((amdgpu_flat_work_group_size(64 * WM * KG, 64 * WM * KG), amdgpu_waves_per_eu(1))) void
+gemm_f32_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x,
+                void* __restrict__ y, int M, int K, int N, int npad, int y_dtype, int tiles_m, uint32_t x_bytes) {
+  constexpr int T = 64 * WM * KG, NB = kGbBlocks;
+  constexpr int BM = 32 * MF * WM, BN = 32 * NF;
+  constexpr int G = BN / 16;                 // 16-row weight groups of the tile
+  constexpr int NT = G * KG * NB * 32 / T;   // conversion tasks per thread and step
+  constexpr int NS = (BN * KG * NB + T - 1) / T;  // scales per thread and step
+  static_assert(NT * T == G * KG * NB * 32, "whole tasks");
+  struct Lds {
+    u32x4 w[2][KG][NB][2][NF][64];  // code fragments [buffer][kg][block][half j][32-column fragment][lane]
+    float s[2][KG][NB][BN];
+  };
+  constexpr int kRed = KG > 1 ? (KG - 1) * BM * BN * 4 : 16;
+  __shared__ __attribute__((aligned(16))) uint8_t smem[sizeof(Lds) > kRed ? sizeof(Lds) : kRed];
+  Lds& L = *reinterpret_cast<Lds*>(smem);
 
-  // staging registers
-  uint4 a_raw[XT == RQ_F32 ? 4 : 2];
-  uint4 b_raw;
-  float s_raw = 0.0f;
+  const int nblk = (int)gridDim.x, bid = (int)blockIdx.x;
+  // the row tiles of a column tile adjacent, each XCD a contiguous run
+  const int xcd = bid & 7, per = nblk >> 3, rem = nblk & 7;
+  const int tord = xcd * per + (xcd < rem ? xcd : rem) + (bid >> 3);
+  const int tm = tord % tiles_m, tn = tord / tiles_m;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wm = wave % WM, kg = wave / WM;
+  const int l32 = lane & 31, g = lane >> 5;
+  const int nkb = K / 32, steps = (nkb + NB - 1) / NB, turns = (steps + KG - 1) / KG;
+  const int n0 = tn * BN, m0 = tm * BM + wm * 32 * MF;
 
-  auto gload = [&](int kb) {
-    const int am = m0 + lrow;
-    if (am < M) {
-      if (XT == RQ_F32) {
-        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const float*>(x) + (int64_t)am * K +
-                                                        (int64_t)kb * 32 + 16 * lhalf);
+  // ---- conversion tasks: task t = tid + T i is row t % 16, half t / 16 % 2 of
+  // block t / 32 % NB of kg t / 32 / NB % KG of the tile's 16-row group
+  // t / 32 / NB / KG (clamped to the padded rows; blocks past the last one
+  // reread it and get zero scales)
+  constexpr uint32_t CB = FMT == RQ_Q8_0 ? 512u : 256u, RB = FMT == RQ_Q8_0 ? 32u : 16u;
+  constexpr uint32_t HB = RB / 2;
+  // the tile's own groups: 32-bit offsets whatever the weight's size
+  const int g0 = n0 / 16, g_last = min(G, npad / 16 - g0) - 1;
+  const __amdgpu_buffer_rsrc_t qr =
+      buffer_rsrc(q + (int64_t)g0 * nkb * CB, (uint32_t)(g_last + 1) * (uint32_t)nkb * CB);
+  const __amdgpu_buffer_rsrc_t sr =
+      buffer_rsrc(sc + (int64_t)g0 * nkb * 16, (uint32_t)(g_last + 1) * (uint32_t)nkb * 16 * (uint32_t)sizeof(ST));
+  const int tr = tid & 15, th = (tid >> 4) & 1;
+  u32x4 raw[NT];
+  uint32_t rs[NS];
+  auto wload = [&](int turn) {
 #pragma unroll
-        for (int i = 0; i < (XT == RQ_F32 ? 4 : 2); i++) a_raw[i] = p[i];
+    for (int i = 0; i < NT; i++) {
+      const int u = (tid + T * i) >> 5, b = u % NB, k = u / NB % KG;
+      const uint32_t grp = (uint32_t)min(u / NB / KG, g_last);
+      const uint32_t kb = (uint32_t)min((turn * KG + k) * NB + b, nkb - 1);
+      const uint32_t off = (grp * (uint32_t)nkb + kb) * CB + (uint32_t)tr * RB + (uint32_t)th * HB;
+      if (FMT == RQ_Q8_0) {
+        raw[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(qr, (int)off, 0, 0));
       } else {
-        const uint4* p = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(x) + (int64_t)am * K +
-                                                        (int64_t)kb * 32 + 16 * lhalf);
-#pragma unroll
-        for (int i = 0; i < 2; i++) a_raw[i] = p[i];
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(qr, (int)off, 0, 0));
+        raw[i] = u32x4{v[0], v[1], 0u, 0u};
       }
-    } else {
-#pragma unroll
-      for (int i = 0; i < (XT == RQ_F32 ? 4 : 2); i++) a_raw[i] = make_uint4(0, 0, 0, 0);
     }
-    const int bn = n0 + lrow;
-    if (bn < N) {
-      const int64_t off = code_off<FMT>(bn, kb, nkb) + (FMT == RQ_Q8_0 ? 16 * lhalf : 0);
-      b_raw = *reinterpret_cast<const uint4*>(q + off);
-      s_raw = load_scale<ST>(sc, scale_off(bn, kb, nkb));
-    } else {
-      b_raw = make_uint4(0, 0, 0, 0);
-      s_raw = 0.0f;
+#pragma unroll
+    for (int i = 0; i < NS; i++) {
+      // scale t = tid + T i: row t % 16 of block t / 16 % NB, kg, group as above
+      const int t = tid + T * i, b = (t >> 4) % NB, k = (t >> 4) / NB % KG;
+      const uint32_t grp = (uint32_t)min((t >> 4) / NB / KG, g_last);
+      const int kb = (turn * KG + k) * NB + b;
+      const uint32_t off = ((grp * (uint32_t)nkb + (uint32_t)min(kb, nkb - 1)) * 16 + (uint32_t)(t & 15)) * sizeof(ST);
+      if (sizeof(ST) == 4)
+        rs[i] = __builtin_amdgcn_raw_buffer_load_b32(sr, (int)off, 0, 0);
+      else
+        rs[i] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)off, 0, 0);
+      if (kb >= nkb) rs[i] = 0u;
     }
   };
-
-  auto lstore = [&](int buf) {
-    // A -> bf16 (hi[/lo]) rows
-    if (XT == RQ_F32) {
-      uint32_t hi[8], lo[8];
+  auto wstore = [&](int buf) {
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float v[4] = {__uint_as_float(a_raw[i].x), __uint_as_float(a_raw[i].y),
-                            __uint_as_float(a_raw[i].z), __uint_as_float(a_raw[i].w)};
-        uint32_t h[4], l[4];
+    for (int i = 0; i < NT; i++) {
+      const int u = (tid + T * i) >> 5, b = u % NB, k = u / NB % KG, grp = u / NB / KG;
+      const int n = 16 * (grp & 1) + tr;
+      if (FMT == RQ_Q8_0) {
+        // 16 codes k = 16 th + 0..15: half j = 0 the first eight, j = 1 the rest
+        u32x2 p[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          h[j] = f32_to_bf16_bits(v[j]);
-          l[j] = f32_to_bf16_bits(v[j] - bf16_bits_to_f32(h[j]));
+        for (int d = 0; d < 4; d++) p[d] = q8_dword_bf16(raw[i][d], 1.0f);
+        L.w[buf][k][b][0][grp >> 1][n + 32 * th] = u32x4{p[0][0], p[0][1], p[1][0], p[1][1]};
+        L.w[buf][k][b][1][grp >> 1][n + 32 * th] = u32x4{p[2][0], p[2][1], p[3][0], p[3][1]};
+      } else {
+        // bytes 8 th + 0..7: low nibbles k = 8 th + 0..7 (lanes of half 0),
+        // high nibbles 16 + 8 th + 0..7 (half 1), both j = th
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+          uint32_t d[2] = {(raw[i][0] >> (4 * h)) & 0x0F0F0F0Fu, (raw[i][1] >> (4 * h)) & 0x0F0F0F0Fu};
+          asm("" : "+v"(d[0]), "+v"(d[1]));  // byte-select conversions instead of a bit-field extract per nibble
+          uint32_t o[4];
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            o[2 * e] = pack2_bf16((float)(d[e] & 0xFFu) - 8.0f, (float)((d[e] >> 8) & 0xFFu) - 8.0f);
+            o[2 * e + 1] = pack2_bf16((float)((d[e] >> 16) & 0xFFu) - 8.0f, (float)(d[e] >> 24) - 8.0f);
+          }
+          L.w[buf][k][b][th][grp >> 1][n + 32 * h] = u32x4{o[0], o[1], o[2], o[3]};
         }
-        hi[2 * i] = h[0] | (h[1] << 16);
-        hi[2 * i + 1] = h[2] | (h[3] << 16);
-        lo[2 * i] = l[0] | (l[1] << 16);
-        lo[2 * i + 1] = l[2] | (l[3] << 16);
       }
-      uint4* dh = reinterpret_cast<uint4*>(&As[buf][0][lrow * LDA + 16 * lhalf]);
-      dh[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-      dh[1] = make_uint4(hi[4], hi[5], hi[6], hi[7]);
-      uint4* dl = reinterpret_cast<uint4*>(&As[buf][NA - 1][lrow * LDA + 16 * lhalf]);
-      dl[0] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-      dl[1] = make_uint4(lo[4], lo[5], lo[6], lo[7]);
-    } else {
-      uint4* d = reinterpret_cast<uint4*>(&As[buf][0][lrow * LDA + 16 * lhalf]);
-      d[0] = a_raw[0];
-      d[1] = a_raw[1];
     }
-    // B -> exact bf16 codes, elements [16*lhalf, 16*lhalf + 16) of the block
-    const uint32_t w[4] = {b_raw.x, b_raw.y, b_raw.z, b_raw.w};
-    uint32_t o[8];
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      float c[4];
-#pragma unroll
-      for (int j = 0; j < 4; j++)
-        c[j] = FMT == RQ_Q8_0 ? q8_code(w[i], j) : q4_nib(w[i], j, lhalf != 0) - 8.0f;
-      o[2 * i] = pack_bf16_exact(c[0], c[1]);
-      o[2 * i + 1] = pack_bf16_exact(c[2], c[3]);
+    for (int i = 0; i < NS; i++) {
+      const int t = tid + T * i, b = (t >> 4) % NB, k = (t >> 4) / NB % KG, grp = (t >> 4) / NB / KG;
+      if (NS * T == BN * KG * NB || grp < G) L.s[buf][k][b][16 * grp + (t & 15)] = scale_from_bits<ST>(rs[i]);
     }
-    uint4* db = reinterpret_cast<uint4*>(&Bs[buf][lrow * LDA + 16 * lhalf]);
-    db[0] = make_uint4(o[0], o[1], o[2], o[3]);
-    db[1] = make_uint4(o[4], o[5], o[6], o[7]);
-    if (lhalf == 0) Ss[buf][lrow] = s_raw;
   };
 
-  f32x4 acc[4][4];
+  // ---- this wave's activation fragments: rows m0 + 32 f + lane % 32
+  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
+  const int r32_last = (M + 31) / 32 - 1;
+  uint32_t xo[MF];
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+  for (int f = 0; f < MF; f++)
+    xo[f] = PK ? (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
+               : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
+  u32x4 a[2][MF][4];  // PK: hi j 0, 1, lo j 0, 1; else the 16 f32
+  auto aload = [&](int slot, int kb) {
+    kb = min(kb, nkb - 1);
 #pragma unroll
-    for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int f = 0; f < MF; f++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        a[slot][f][i] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
+                                                         (int)((uint32_t)kb * (PK ? 4096u : 128u)), 0));
+  };
 
-  gload(0);
-  lstore(0);
+  f32x16 acc[MF][NF];
+#pragma unroll
+  for (int f = 0; f < MF; f++)
+#pragma unroll
+    for (int c = 0; c < NF; c++)
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[f][c][e] = 0.0f;
+  f32x16 zero;
+#pragma unroll
+  for (int e = 0; e < 16; e++) zero[e] = 0.0f;
+
+  wload(0);
+  aload(0, kg * NB);
+  wstore(0);
+  wload(1);
   __syncthreads();
-  const int fr = lane & 15, fk = 8 * (lane >> 4);
-  for (int kb = 0; kb < nkb; kb++) {
-    const int buf = kb & 1;
-    if (kb + 1 < nkb) gload(kb + 1);
-    bf16x8 af[NA][4], bfr[4];
-    float sj[4];
+  for (int t = 0; t < turns; t++) {
+    const int buf = t & 1, kb0 = (t * KG + kg) * NB;
+    wstore(buf ^ 1);
+    wload(t + 2);
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int b = 0; b < NB; b++) {
+      aload((b + 1) & 1, b + 1 < NB ? kb0 + b + 1 : kb0 + KG * NB);
+      bf16x8 h[MF][2], l[MF][2];
 #pragma unroll
-      for (int h = 0; h < NA; h++)
-        af[h][i] = *reinterpret_cast<const bf16x8*>(&As[buf][h][(wm * 64 + i * 16 + fr) * LDA + fk]);
+      for (int f = 0; f < MF; f++) {
+        const u32x4* r = a[b & 1][f];
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      bfr[j] = *reinterpret_cast<const bf16x8*>(&Bs[buf][(wn * 64 + j * 16 + fr) * LDA + fk]);
-      sj[j] = Ss[buf][wn * 64 + j * 16 + fr];
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) {
-        f32x4 p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[0][i], bfr[j], zero, 0, 0, 0);
-        if (NA == 2) p = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[NA - 1][i], bfr[j], p, 0, 0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; r++) acc[i][j][r] = fmaf(sj[j], p[r], acc[i][j][r]);
+        for (int j = 0; j < 2; j++) {
+          u32x4 hv, lv;
+          if (PK) {
+            hv = r[j];
+            lv = r[2 + j];
+          } else {
+            split8(__builtin_bit_cast(f32x4, r[2 * j]), __builtin_bit_cast(f32x4, r[2 * j + 1]), hv, lv);
+          }
+          h[f][j] = __builtin_bit_cast(bf16x8, hv);
+          l[f][j] = __builtin_bit_cast(bf16x8, lv);
+        }
       }
-    if (kb + 1 < nkb) lstore(buf ^ 1);
+#pragma unroll
+      for (int c = 0; c < NF; c++) {
+        const bf16x8 w0 = __builtin_bit_cast(bf16x8, L.w[buf][kg][b][0][c][lane]);
+        const bf16x8 w1 = __builtin_bit_cast(bf16x8, L.w[buf][kg][b][1][c][lane]);
+        const float s = L.s[buf][kg][b][32 * c + l32];
+#pragma unroll
+        for (int f = 0; f < MF; f++) {
+          f32x16 p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][0], w0, zero, 0, 0, 0);
+          p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][1], w1, p, 0, 0, 0);
+          p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[f][0], w0, p, 0, 0, 0);
+          p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[f][1], w1, p, 0, 0, 0);
+#pragma unroll
+          for (int e = 0; e < 16; e++) acc[f][c][e] = fmaf(s, p[e], acc[f][c][e]);
+        }
+      }
+    }
     __syncthreads();
   }
 
-  // epilogue: lane holds column fr of each 16x16 tile, rows 4*(lane>>4) + r
+  if (KG > 1) {
+    // the kg waves' sums through LDS, added in kg order
+    f32x16* red = reinterpret_cast<f32x16*>(smem);
+    constexpr int W = WM * MF * NF * 64;
+    const int at = wm * MF * NF * 64 + lane;
+    if (kg > 0) {
 #pragma unroll
-  for (int i = 0; i < 4; i++)
+      for (int f = 0; f < MF; f++)
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const int n = n0 + wn * 64 + j * 16 + fr;
+        for (int c = 0; c < NF; c++) red[(kg - 1) * W + at + (f * NF + c) * 64] = acc[f][c];
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int k = 0; k < KG - 1; k++)
+#pragma unroll
+      for (int f = 0; f < MF; f++)
+#pragma unroll
+        for (int c = 0; c < NF; c++) acc[f][c] += red[k * W + at + (f * NF + c) * 64];
+  }
+
+  // acc[f][c] register e: m = m0 + 32 f + 8 (e / 4) + 4 g + e % 4, n = n0 + 32 c + lane % 32
+#pragma unroll
+  for (int f = 0; f < MF; f++)
+#pragma unroll
+    for (int c = 0; c < NF; c++) {
+      const int n = n0 + 32 * c + l32;
       if (n >= N) continue;
 #pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const int m = m0 + wm * 64 + i * 16 + 4 * (lane >> 4) + r;
+      for (int e = 0; e < 16; e++) {
+        const int m = m0 + 32 * f + 8 * (e >> 2) + 4 * g + (e & 3);
         if (m >= M) continue;
         if (y_dtype == RQ_F32)
-          static_cast<float*>(y)[(int64_t)m * N + n] = acc[i][j][r];
+          static_cast<float*>(y)[(int64_t)m * N + n] = acc[f][c][e];
         else
-          static_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)f32_to_bf16_bits(acc[i][j][r]);
+          static_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)f32_to_bf16_bits(acc[f][c][e]);
       }
     }
 }
 
-// f32 activations only: bf16 activations take gemm_bf16_kernel (gemm_bf16.hip).
-template <int FMT, typename ST>
-static hipError_t launch_x(const MatmulArgs& a) {
-  if (a.x_dtype != RQ_F32) return hipErrorInvalidValue;
-  const int tiles_m = (int)((a.m + GBM - 1) / GBM), tiles_n = (int)((a.n + GBN - 1) / GBN);
-  dim3 grid((unsigned)(tiles_m * tiles_n));
-  hipExtLaunchKernelGGL((gemm_kernel<FMT, ST, RQ_F32>), grid, dim3(256), 0, a.stream, a.ev_main[0], a.ev_main[1],
-                        0, a.q, static_cast<const ST*>(a.scales), a.x, a.y, (int)a.m, (int)a.k, (int)a.n,
-                        a.y_dtype, tiles_m);
+// Role-split form for the larger tiles: eight waves, waves 0..3 (consumers) 32 MF
+// rows x 32 NF columns each, waves 4..7 (producers) load the codes RW - 1 steps
+// ahead and convert step s + 2 into LDS buffer (s + 2) % 3 while the consumers
+// run step s. A wave's loads complete in issue order, so a wave that loads both
+// would wait for its codes (HBM) whenever it waits for activations (L2).
+template <int FMT, typename ST, bool PK, int MF, int NF, int RA>
+__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void gemm_f32_rs_kernel(
+    const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x, void* __restrict__ y, int M,
+    int K, int N, int npad, int y_dtype, int tiles_m, uint32_t x_bytes) {
+  constexpr int NB = kGbBlocks, RW = 3;
+  constexpr int BM = 128 * MF, BN = 32 * NF, G = BN / 16;
+  constexpr int NT = G * NB * 32 / 256;
+  constexpr int NS = (BN * NB + 255) / 256;
+  constexpr int TPS = NB * NF * MF, PR = TPS % 3 == 0 ? 3 : 4;  // tiles per step, block sums in flight
+  static_assert(NB % RA == 0 && NB * NF % 3 == 0 && NB * NF % 4 == 0 && TPS % PR == 0, "rings turn whole in a step");
+  struct Lds {
+    u32x4 w[3][NB][2][NF][64];
+    float s[3][NB][BN];
+  };
+  __shared__ __attribute__((aligned(16))) Lds L;
+  const int nblk = (int)gridDim.x, bid = (int)blockIdx.x;
+  const int xcd = bid & 7, per = nblk >> 3, rem = nblk & 7;
+  const int tord = xcd * per + (xcd < rem ? xcd : rem) + (bid >> 3);
+  const int tm = tord % tiles_m, tn = tord / tiles_m;
+  const int tid = threadIdx.x & 255, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nkb = K / 32, steps = (nkb + NB - 1) / NB;
+  const int n0 = tn * BN;
+
+  if (wave >= 4) {
+    // ---- producer
+    constexpr uint32_t CB = FMT == RQ_Q8_0 ? 512u : 256u, RB = FMT == RQ_Q8_0 ? 32u : 16u;
+    constexpr uint32_t HB = RB / 2;
+    const int g0 = n0 / 16, g_last = min(G, npad / 16 - g0) - 1;
+    const __amdgpu_buffer_rsrc_t qr =
+        buffer_rsrc(q + (int64_t)g0 * nkb * CB, (uint32_t)(g_last + 1) * (uint32_t)nkb * CB);
+    const __amdgpu_buffer_rsrc_t sr =
+        buffer_rsrc(sc + (int64_t)g0 * nkb * 16, (uint32_t)(g_last + 1) * (uint32_t)nkb * 16 * (uint32_t)sizeof(ST));
+    const int tr = tid & 15, th = (tid >> 4) & 1;
+    u32x4 raw[RW][NT];
+    uint32_t rs[RW][NS];
+    auto wload = [&](int slot, int step) {
+#pragma unroll
+      for (int i = 0; i < NT; i++) {
+        const int u = (tid + 256 * i) >> 5, b = u % NB;
+        const uint32_t grp = (uint32_t)min(u / NB, g_last);
+        const uint32_t kb = (uint32_t)min(step * NB + b, nkb - 1);
+        const uint32_t off = (grp * (uint32_t)nkb + kb) * CB + (uint32_t)tr * RB + (uint32_t)th * HB;
+        if (FMT == RQ_Q8_0) {
+          raw[slot][i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(qr, (int)off, 0, 0));
+        } else {
+          const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(qr, (int)off, 0, 0));
+          raw[slot][i] = u32x4{v[0], v[1], 0u, 0u};
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NS; i++) {
+        const int t = tid + 256 * i, b = (t >> 4) % NB;
+        const uint32_t grp = (uint32_t)min((t >> 4) / NB, g_last);
+        const uint32_t kb = (uint32_t)min(step * NB + b, nkb - 1);
+        const uint32_t off = ((grp * (uint32_t)nkb + kb) * 16 + (uint32_t)(t & 15)) * sizeof(ST);
+        if (sizeof(ST) == 4)
+          rs[slot][i] = __builtin_amdgcn_raw_buffer_load_b32(sr, (int)off, 0, 0);
+        else
+          rs[slot][i] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)off, 0, 0);
+      }
+    };
+    auto wstore = [&](int slot, int buf, int step) {
+#pragma unroll
+      for (int i = 0; i < NT; i++) {
+        const int u = (tid + 256 * i) >> 5, b = u % NB, grp = u / NB;
+        const int n = 16 * (grp & 1) + tr;
+        if (FMT == RQ_Q8_0) {
+          u32x2 p[4];
+#pragma unroll
+          for (int d = 0; d < 4; d++) p[d] = q8_dword_bf16(raw[slot][i][d], 1.0f);
+          L.w[buf][b][0][grp >> 1][n + 32 * th] = u32x4{p[0][0], p[0][1], p[1][0], p[1][1]};
+          L.w[buf][b][1][grp >> 1][n + 32 * th] = u32x4{p[2][0], p[2][1], p[3][0], p[3][1]};
+        } else {
+#pragma unroll
+          for (int h = 0; h < 2; h++) {
+            uint32_t d[2] = {(raw[slot][i][0] >> (4 * h)) & 0x0F0F0F0Fu, (raw[slot][i][1] >> (4 * h)) & 0x0F0F0F0Fu};
+            asm("" : "+v"(d[0]), "+v"(d[1]));
+            uint32_t o[4];
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+              o[2 * e] = pack2_bf16((float)(d[e] & 0xFFu) - 8.0f, (float)((d[e] >> 8) & 0xFFu) - 8.0f);
+              o[2 * e + 1] = pack2_bf16((float)((d[e] >> 16) & 0xFFu) - 8.0f, (float)(d[e] >> 24) - 8.0f);
+            }
+            L.w[buf][b][th][grp >> 1][n + 32 * h] = u32x4{o[0], o[1], o[2], o[3]};
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < NS; i++) {
+        const int t = tid + 256 * i, b = (t >> 4) % NB, grp = (t >> 4) / NB;
+        if (grp < G) L.s[buf][b][16 * grp + (t & 15)] = step * NB + b < nkb ? scale_from_bits<ST>(rs[slot][i]) : 0.0f;
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < RW; s++) wload(s, s);
+    wstore(0, 0, 0);
+    wload(0, 3);
+    wstore(1, 1, 1);
+    wload(1, 4);
+    __syncthreads();
+    for (int s0 = 0; s0 < steps; s0 += 3) {
+#pragma unroll
+      for (int u = 0; u < 3; u++) {
+        if (s0 + u < steps) {
+          wstore((u + 2) % 3, (u + 2) % 3, s0 + u + 2);
+          wload((u + 2) % 3, s0 + u + 5);
+          __syncthreads();
+        }
+      }
+    }
+    return;
+  }
+
+  // ---- consumer
+  const int l32 = lane & 31, g = lane >> 5;
+  const int m0 = tm * BM + wave * 32 * MF;
+  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
+  const int r32_last = (M + 31) / 32 - 1;
+  uint32_t xo[MF];
+#pragma unroll
+  for (int f = 0; f < MF; f++)
+    xo[f] = PK ? (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
+               : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
+  u32x4 a[RA][MF][4];
+  auto aload = [&](int slot, int kb) {
+    kb = min(kb, nkb - 1);
+#pragma unroll
+    for (int f = 0; f < MF; f++)
+#pragma unroll
+      for (int i = 0; i < 4; i++)
+        a[slot][f][i] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
+                                                         (int)((uint32_t)kb * (PK ? 4096u : 128u)), 0));
+  };
+  f32x16 zero;
+#pragma unroll
+  for (int e = 0; e < 16; e++) zero[e] = 0.0f;
+  f32x16 acc[MF][NF], p[PR];
+#pragma unroll
+  for (int f = 0; f < MF; f++)
+#pragma unroll
+    for (int c = 0; c < NF; c++) acc[f][c] = zero;
+#pragma unroll
+  for (int i = 0; i < PR; i++) p[i] = zero;
+  bf16x8 w[3][2];
+  float ws[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // scales of the column fragments j - 2 .. j + 1
+  bf16x8 h[MF][2], l[MF][2], lp[2];  // the block's hi and lo fragments; the last tile's lo of the block before
+  const bf16x8 none = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+  w[2][0] = w[2][1] = lp[0] = lp[1] = none;
+  auto wread = [&](int j, int buf, int b, int c) {
+    w[j % 3][0] = __builtin_bit_cast(bf16x8, L.w[buf][b][0][c][lane]);
+    w[j % 3][1] = __builtin_bit_cast(bf16x8, L.w[buf][b][1][c][lane]);
+    ws[j % 4] = L.s[buf][b][32 * c + l32];
+  };
+#pragma unroll
+  for (int i = 0; i < RA - 1; i++) aload(i, i);
+  __syncthreads();
+  wread(0, 0, 0, 0);
+  int buf = 0;
+  for (int s = 0; s < steps; s++) {
+    const int nbuf = buf == 2 ? 0 : buf + 1;
+    // tile i of the step: column fragment j = i / MF, row fragment i % MF. Its
+    // four MFMAs (hi, hi, lo, lo of the two 16-k halves) are spread over two
+    // turns, so that two chains alternate, and the block sums are scaled in
+    // the turn after, beside the MFMAs of the next two tiles
+#pragma unroll
+    for (int i = 0; i < TPS; i++) {
+      const int j = i / MF, f = i % MF, b = j / NF, c = j % NF;
+      const int q1 = (i + TPS - 1) % TPS, j1 = q1 / MF, f1 = q1 % MF;  // the tile before
+      const int q2 = (i + TPS - 2) % TPS, j2 = q2 / MF, f2 = q2 % MF;  // and the one before it
+      if (c == 0 && f == 0) {
+#pragma unroll
+        for (int ff = 0; ff < MF; ff++)
+#pragma unroll
+          for (int e = 0; e < 2; e++) {
+            const u32x4* r = a[b % RA][ff];
+            u32x4 hv, lv;
+            if (PK) {
+              hv = r[e];
+              lv = r[2 + e];
+            } else {
+              split8(__builtin_bit_cast(f32x4, r[2 * e]), __builtin_bit_cast(f32x4, r[2 * e + 1]), hv, lv);
+            }
+            h[ff][e] = __builtin_bit_cast(bf16x8, hv);
+            l[ff][e] = __builtin_bit_cast(bf16x8, lv);
+          }
+      }
+      if (f == 0) wread(j + 1, j + 1 < NB * NF ? buf : nbuf, (j + 1) / NF % NB, (j + 1) % NF);
+      const bool head = c == 0 && f == 0;  // the tile before is of the block before
+      p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][0], w[j % 3][0], zero, 0, 0, 0);
+      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[0] : l[f1][0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
+      p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][1], w[j % 3][1], p[i % PR], 0, 0, 0);
+      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[1] : l[f1][1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
+      if (c == 0 && f == 0) aload((b + RA - 1) % RA, s * NB + b + RA - 1);
+      if (c == NF - 1 && f == MF - 1) {
+        lp[0] = l[f][0];
+        lp[1] = l[f][1];
+      }
+      if (PK) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+    buf = nbuf;
+  }
+  {
+    constexpr int q1 = TPS - 1, j1 = q1 / MF, f1 = q1 % MF, q2 = TPS - 2, j2 = q2 / MF, f2 = q2 % MF;
+    p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
+    p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
+#pragma unroll
+    for (int e = 0; e < 16; e++) acc[f1][j1 % NF][e] = fmaf(ws[j1 % 4], p[q1 % PR][e], acc[f1][j1 % NF][e]);
+  }
+
+#pragma unroll
+  for (int f = 0; f < MF; f++)
+#pragma unroll
+    for (int c = 0; c < NF; c++) {
+      const int n = n0 + 32 * c + l32;
+      if (n >= N) continue;
+#pragma unroll
+      for (int e = 0; e < 16; e++) {
+        const int m = m0 + 32 * f + 8 * (e >> 2) + 4 * g + (e & 3);
+        if (m >= M) continue;
+        if (y_dtype == RQ_F32)
+          static_cast<float*>(y)[(int64_t)m * N + n] = acc[f][c][e];
+        else
+          static_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)f32_to_bf16_bits(acc[f][c][e]);
+      }
+    }
+}
+
+template <int FMT, typename ST, bool PK, int MF, int NF, int RA>
+static hipError_t launch_rs_t(const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
+                           hipEvent_t done) {
+  constexpr int BM = 128 * MF, BN = 32 * NF;
+  const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
+  if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
+  const int64_t bytes = std::min<int64_t>((PK ? (m + 31) / 32 * 32 : m) * a.k * 4, UINT32_MAX);
+  hipExtLaunchKernelGGL((gemm_f32_rs_kernel<FMT, ST, PK, MF, NF, RA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0,
+                        a.stream, begin, done, 0, a.q, static_cast<const ST*>(a.scales), x, y, (int)m, (int)a.k,
+                        (int)a.n, (int)a.npad, a.y_dtype, (int)tiles_m, (uint32_t)bytes);
   return hipGetLastError();
 }
 
+template <int FMT, typename ST, bool PK, int MF, int NF, int WM, int KG>
+static hipError_t launch_t(const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
+                           hipEvent_t done) {
+  constexpr int BM = 32 * MF * WM, BN = 32 * NF;
+  const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
+  if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
+  const int64_t bytes = std::min<int64_t>((PK ? (m + 31) / 32 * 32 : m) * a.k * 4, UINT32_MAX);
+  hipExtLaunchKernelGGL((gemm_f32_kernel<FMT, ST, PK, MF, NF, WM, KG>), dim3((unsigned)(tiles_m * tiles_n)),
+                        dim3(64 * WM * KG), 0, a.stream, begin, done, 0, a.q, static_cast<const ST*>(a.scales), x, y,
+                        (int)m, (int)a.k, (int)a.n, (int)a.npad, a.y_dtype, (int)tiles_m, (uint32_t)bytes);
+  return hipGetLastError();
+}
+
+namespace {
+
+// The tiles. Time of a call, fitted to an MI355X with c = workgroups per CU
+// (rounded up): K-blocks / kg x max(one_ns, c block_ns) + c round_ns. Measured,
+// us a call with the packing pass, Q8_0, f32 y:
+//                        32x32  64x32  128x64  128x96  128x192
+//   11008 x 4096  m = 32  22.8   31.3    53.0    45.1    73.6
+//                 m = 64  33.7   35.1    53.6    45.8    73.6
+//                 m = 256 99.1   86.9    65.6    54.6    77.8
+//                 m = 333 136    127     93.3    93.8    79.4
+//                 m = 512 222    164     105     102     94.5
+//   4096 x 4096   m = 256 45.8   38.1    55.3    48.2    76.8
+//                 m = 768 190    108     70.9    99.2    80.3
+// The kernel before these (one 128 x 128 tile, both operands converted in every
+// workgroup, two barriers per 32-block) took 275 us at m = 333, 11008 x 4096
+// (Q4_0).
+struct F32Tile {
+  int bm, bn, kg, one_ns, block_ns, round_ns;
+};
+constexpr F32Tile kF32Tiles[] = {{32, 32, 4, 310, 262, 0},
+                                 {64, 32, 4, 500, 440, 0},
+                                 {128, 64, 1, 360, 245, 0},
+                                 {128, 96, 1, 315, 315, 4000},
+                                 {128, 192, 1, 570, 570, 5000}};
+
+int pick_tile(int64_t m, int64_t k, int64_t n, int cu_count) {
+  int best = 0;
+  int64_t best_cost = INT64_MAX;
+  for (int i = 0; i < (int)(sizeof(kF32Tiles) / sizeof(kF32Tiles[0])); i++) {
+    const F32Tile& t = kF32Tiles[i];
+    const int64_t tiles = (m + t.bm - 1) / t.bm * ((n + t.bn - 1) / t.bn), c = (tiles + cu_count - 1) / cu_count;
+    const int64_t cost = k / 32 * std::max<int64_t>(t.one_ns, c * t.block_ns) / t.kg + c * t.round_ns;
+    if (cost < best_cost) best_cost = cost, best = i;
+  }
+  return best;
+}
+
+template <int FMT, typename ST, bool PK>
+hipError_t launch_tile(int tile, const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
+                           hipEvent_t done) {
+  switch (tile) {
+    case 0: return launch_t<FMT, ST, PK, 1, 1, 1, 4>(a, x, y, m, begin, done);
+    case 1: return launch_t<FMT, ST, PK, 2, 1, 1, 4>(a, x, y, m, begin, done);
+    case 2: return launch_t<FMT, ST, PK, 1, 2, 4, 1>(a, x, y, m, begin, done);
+    case 3: return launch_rs_t<FMT, ST, PK, 1, 3, 4>(a, x, y, m, begin, done);
+    default: return launch_rs_t<FMT, ST, PK, 1, 6, 2>(a, x, y, m, begin, done);
+  }
+}
+
+// Rows per launch: the packed copy within rq_qmatmul_noalloc's scratch, x within
+// the 32-bit buffer offsets
+int64_t chunk_rows(int64_t k, bool packed) {
+  const int64_t rows = (packed ? (int64_t)RQ_NOALLOC_SCRATCH_MAX : (int64_t)UINT32_MAX) / (4 * k);
+  return rows >= 256 ? rows / 256 * 256 : packed ? rows / 32 * 32 : std::max<int64_t>(rows, 1);
+}
+}  // namespace
+
+size_t gemm_f32_pack_bytes(int64_t m, int64_t k) {
+  return (size_t)(std::min((m + 31) / 32 * 32, chunk_rows(k, true)) * k * 4);
+}
+
+template <int FMT, typename ST>
+static hipError_t launch_x(const MatmulArgs& a, int cu_count) {
+  const bool pk = a.scratch != nullptr;
+  // of the whole call, whatever its chunks; a tile's weights within 32-bit offsets
+  const int tile = a.k > (int64_t)1 << 24 ? 0 : pick_tile(a.m, a.k, a.n, cu_count);
+  const int64_t chunk = chunk_rows(a.k, pk);
+  for (int64_t m0 = 0; m0 < a.m; m0 += chunk) {
+    const int64_t m = std::min(chunk, a.m - m0);
+    const float* x = static_cast<const float*>(a.x) + m0 * a.k;
+    void* y = static_cast<uint8_t*>(a.y) + m0 * a.n * (a.y_dtype == RQ_F32 ? 4 : 2);
+    const hipEvent_t done = m0 + chunk >= a.m ? a.ev_main[1] : nullptr;
+    if (pk) {
+      const int64_t blocks = (m + 31) / 32 * ((a.k / 32 + 1) / 2);
+      hipExtLaunchKernelGGL(pack_x32_split_kernel, dim3((unsigned)blocks), dim3(256), 0, a.stream, nullptr,
+                            m0 == 0 ? a.ev_main[0] : nullptr, 0, x, static_cast<uint16_t*>(a.scratch), (int)m,
+                            (int)a.k);
+      if (hipError_t e = hipGetLastError()) return e;
+    }
+    const hipError_t e = pk ? launch_tile<FMT, ST, true>(tile, a, a.scratch, y, m, nullptr, done)
+                            : launch_tile<FMT, ST, false>(tile, a, x, y, m, m0 == 0 ? a.ev_main[0] : nullptr, done);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
 hipError_t launch_gemm(const MatmulArgs& a, int cu_count) {
-  (void)cu_count;
-  if (a.format == RQ_Q8_0) return launch_x<RQ_Q8_0, float>(a);
-  if (a.scale_dtype == RQ_F16) return launch_x<RQ_Q4_0, uint16_t>(a);
-  return launch_x<RQ_Q4_0, float>(a);
+  if (a.x_dtype != RQ_F32) return hipErrorInvalidValue;
+  if (a.format == RQ_Q8_0) return launch_x<RQ_Q8_0, float>(a, cu_count);
+  if (a.scale_dtype == RQ_F16) return launch_x<RQ_Q4_0, uint16_t>(a, cu_count);
+  return launch_x<RQ_Q4_0, float>(a, cu_count);
 }
 
 }  // namespace rq

@@ -165,6 +165,9 @@ hipError_t launch_split_reduce(const float* part, void* y, int64_t n, int ks, in
 
 // Kernel launchers (each returns a hipError_t from hipGetLastError after launch).
 hipError_t launch_gemv(const MatmulArgs& a, const DecodePlan& p);
+// f32 x, m > 16 (gemm.hip): with gemm_f32_pack_bytes of scratch (0: it has no
+// use for any) the packed activations, without (a.scratch NULL) slower, same results
+size_t gemm_f32_pack_bytes(int64_t m, int64_t k);
 hipError_t launch_gemm(const MatmulArgs& a, int cu_count);
 hipError_t launch_gemm_bf16(const MatmulArgs& a, int cu_count);
 // bf16 x, 16 < m <= 64, weight-stream GEMM with LDS-staged activations
