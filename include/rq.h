@@ -354,7 +354,10 @@ int rq_quantize_act_i8(rq_ctx ctx, const float* x, int64_t m, int64_t in, int8_t
  * in double). Q4_0 needs xsum (qmatmul-q4-composable,
  * raster/quant/kernels.clj:140-184); Q8_0 ignores it (qmatmul-i8-gemm!,
  * raster/quant/kernels_k.clj:357-370). m <= 16 runs the decode kernel, larger
- * m an int8-MFMA GEMM. xq 16-byte aligned. */
+ * m a bf16-MFMA GEMM on the exact codes (per-stream scratch, 2.125 bytes per
+ * element of at most 64 MiB of rows at a time, grown outside capture only).
+ * xq 16-byte aligned; xsum the codes' sums, as the quantizer gives them (the
+ * GEMM forms the zero-point term from the codes themselves). */
 int rq_qmatmul_i8(rq_ctx ctx, rq_weight w, const int8_t* xq, const float* xs, const int32_t* xsum, void* y,
                   int y_dtype, int64_t m, void* stream);
 

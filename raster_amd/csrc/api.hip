@@ -927,9 +927,8 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
     const size_t bytes = std::max((size_t)((m + 15) / 16 * 16) * (size_t)w.in * 2, pack_x32_bytes(m, w.in));
     if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch)) return s;
   } else if (!plan.ok && x_dtype == kXtI8) {
-    // fragment-major int8 activations with their scales and sums: 640 B per
-    // 16-row tile and 32-block
-    const size_t bytes = (size_t)((m + 15) / 16) * (size_t)(w.in / 32) * 640;
+    // the int8 activations as bf16 fragments, with their scales
+    const size_t bytes = gemm_i8_pack_bytes(m, w.in);
     if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch)) return s;
   } else if (!plan.ok) {
     // bf16 hi + lo copy of the f32 activations; a call that cannot have the

@@ -1,5 +1,6 @@
-// gemm.hip — prefill-regime (m > 16) block-quantized GEMM for f32 activations on
-// CDNA4 MFMA.
+// gemm.hip — prefill-regime (m > 16) block-quantized GEMMs whose block sums are
+// scaled in f32, on CDNA4 MFMA: f32 activations, and int8 activations
+// (rq_quantize_act_i8).
 //
 // y[m, o] = sum_b scale[o, b] * P_b[m, o],  P_b = sum_{k in block b} x[m, k] * code[o, k]
 //
@@ -10,7 +11,14 @@
 // output per block). x is carried as bf16 hi + lo (x = hi + lo + O(2^-17 |x|)),
 // two MFMAs per product.
 //
-// Bound: the MFMAs (twice the bf16 GEMM's) and, at the operand rates of a CU,
+// int8 activations (qmatmul-i8-gemm!, raster/quant/kernels_k.clj:357-370, and the
+// Q4_0 form of qmatmul-q4-composable, raster/quant/kernels.clj:140-184):
+//   y[t, o] = sum_b ws[o, b] * xs[t, b] * dot_b(code[o] [- 8], xq[t])
+// The codes of both sides enter the bf16 MFMA as exact integers (the Q4_0 zero
+// point subtracted from the code, which is the -8 xsum fold) and a block's sum,
+// below 2^19, is exact in f32: no int32 result to convert, and no sums to fold.
+//
+// Bound, f32 activations: the MFMAs (twice the bf16 GEMM's) and, at the operand rates of a CU,
 // the activations: 4 bytes per element, so a fragment is loaded once per wave
 // and used for 96 or 192 columns. Measured (128 x 96 tile, per MFMA and wave):
 // 24 ns, of it 16.5 the MFMA itself, about 4 the activation loads and the
@@ -23,6 +31,8 @@ namespace rq {
 
 namespace {
 
+typedef float f32x32 __attribute__((ext_vector_type(32)));
+
 constexpr int kGbBlocks = 4;  // 32-blocks per step
 
 // x = hi + lo, both RNE bf16, eight elements
@@ -33,6 +43,12 @@ __device__ __forceinline__ void split8(const f32x4& v0, const f32x4& v1, u32x4& 
     hi[i] = pack2_bf16(a, b);
     lo[i] = pack2_bf16(a - __uint_as_float(hi[i] << 16), b - __uint_as_float(hi[i] & 0xFFFF0000u));
   }
+}
+
+// bytes of the packed activations: bf16 hi + lo, or (int8) bf16 codes and f32 block scales
+int64_t packed_bytes(int x_dtype, int64_t m, int64_t k) {
+  const int64_t m32 = (m + 31) / 32 * 32;
+  return x_dtype == kXtI8 ? m32 * k * 2 + m32 * (k / 32) * 4 : m32 * k * 4;
 }
 
 }  // namespace
@@ -61,6 +77,25 @@ __global__ __launch_bounds__(256) void pack_x32_split_kernel(const float* __rest
   dst[128] = lo;
 }
 
+// int8 codes xq[M][K] and their block scales xs[M][K/32] -> the same fragments
+// (codes as bf16, exact) and, after them, the scales as [M/32][K/32][32].
+__global__ __launch_bounds__(256) void pack_x32_i8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xs,
+                                                          uint16_t* __restrict__ xf, int M, int K) {
+  const int nkb = K / 32, nq = (nkb + 1) / 2;
+  const int tile = blockIdx.x / nq, kb = (blockIdx.x % nq) * 2 + ((threadIdx.x & 7) >> 2);
+  if (kb >= nkb) return;
+  const int row = threadIdx.x >> 3, cc = threadIdx.x & 3;  // 8-k chunk cc of the k-step
+  const int m = tile * 32 + row;
+  u32x2 v = {0u, 0u};
+  if (m < M) v = *reinterpret_cast<const u32x2*>(xq + (int64_t)m * K + 32 * kb + 8 * cc);
+  const u32x2 p = q8_dword_bf16(v[0], 1.0f), q = q8_dword_bf16(v[1], 1.0f);
+  const int64_t at = (int64_t)tile * nkb + kb;
+  reinterpret_cast<u32x4*>(xf)[(at * 2 + (cc & 1)) * 64 + row + 32 * (cc >> 1)] = u32x4{p[0], p[1], q[0], q[1]};
+  if (cc == 0)
+    reinterpret_cast<float*>(xf + (int64_t)((M + 31) / 32) * nkb * 1024)[at * 32 + row] =
+        m < M ? xs[(int64_t)m * nkb + kb] : 0.0f;
+}
+
 // Workgroup: WM x KG waves; tile 32 MF WM rows x 32 NF columns, a wave 32 MF x
 // 32 NF of it over the steps s (of four 32-blocks) with s % KG = its kg (their
 // sums are added in kg order at the end). All waves convert the next KG steps'
@@ -69,15 +104,17 @@ __global__ __launch_bounds__(256) void pack_x32_split_kernel(const float* __rest
 // steps. Activation fragments go straight into registers, a block ahead: from
 // the packed copy, or (PK false: calls that have no scratch) from x itself,
 // split in registers, with the same result.
-template <int FMT, typename ST, bool PK, int MF, int NF, int WM, int KG>
+template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int WM, int KG>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * WM * KG, 64 * WM * KG), amdgpu_waves_per_eu(1))) void
-gemm_f32_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x,
+gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x,
                 void* __restrict__ y, int M, int K, int N, int npad, int y_dtype, int tiles_m, uint32_t x_bytes) {
   constexpr int T = 64 * WM * KG, NB = kGbBlocks;
   constexpr int BM = 32 * MF * WM, BN = 32 * NF;
   constexpr int G = BN / 16;                 // 16-row weight groups of the tile
   constexpr int NT = G * KG * NB * 32 / T;   // conversion tasks per thread and step
   constexpr int NS = (BN * KG * NB + T - 1) / T;  // scales per thread and step
+  constexpr bool I8 = XT == kXtI8;
+  constexpr int AF = I8 ? 2 : 4;             // 16-byte pieces of an activation fragment
   static_assert(NT * T == G * KG * NB * 32, "whole tasks");
   struct Lds {
     u32x4 w[2][KG][NB][2][NF][64];  // code fragments [buffer][kg][block][half j][32-column fragment][lane]
@@ -181,21 +218,32 @@ gemm_f32_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
   // ---- this wave's activation fragments: rows m0 + 32 f + lane % 32
   const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
   const int r32_last = (M + 31) / 32 - 1;
-  uint32_t xo[MF];
+  const uint32_t xs_base = (uint32_t)(r32_last + 1) * (uint32_t)nkb * 2048u;  // I8: the scales' region
+  uint32_t xo[MF], so[MF];
 #pragma unroll
-  for (int f = 0; f < MF; f++)
-    xo[f] = PK ? (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
+  for (int f = 0; f < MF; f++) {
+    const uint32_t r32 = (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb;
+    xo[f] = PK ? r32 * (1024u * AF) + 16u * (uint32_t)lane
                : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
-  u32x4 a[2][MF][4];  // PK: hi j 0, 1, lo j 0, 1; else the 16 f32
+    so[f] = xs_base + r32 * 128u + 16u * (uint32_t)g;
+  }
+  u32x4 a[2][MF][AF];     // PK: hi j 0, 1, f32: lo j 0, 1; else the 16 f32
+  f32x4 xs[2][I8 ? MF : 1][4];  // I8: the scales of rows 8 q + 4 g + 0..3
   auto aload = [&](int slot, int kb) {
     kb = min(kb, nkb - 1);
 #pragma unroll
-    for (int f = 0; f < MF; f++)
+    for (int f = 0; f < MF; f++) {
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < AF; i++)
         a[slot][f][i] = __builtin_bit_cast(
             u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
-                                                         (int)((uint32_t)kb * (PK ? 4096u : 128u)), 0));
+                                                         (int)((uint32_t)kb * (PK ? 1024u * AF : 128u)), 0));
+      if (I8)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          xs[slot][f][i] = __builtin_bit_cast(
+              f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(so[f] + 32u * i), (int)((uint32_t)kb * 128u), 0));
+    }
   };
 
   f32x16 acc[MF][NF];
@@ -227,12 +275,11 @@ gemm_f32_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
         const u32x4* r = a[b & 1][f];
 #pragma unroll
         for (int j = 0; j < 2; j++) {
-          u32x4 hv, lv;
+          u32x4 hv = r[j], lv = r[j];
           if (PK) {
-            hv = r[j];
-            lv = r[2 + j];
+            if (!I8) lv = r[AF - 2 + j];
           } else {
-            split8(__builtin_bit_cast(f32x4, r[2 * j]), __builtin_bit_cast(f32x4, r[2 * j + 1]), hv, lv);
+            split8(__builtin_bit_cast(f32x4, r[2 * j % AF]), __builtin_bit_cast(f32x4, r[(2 * j + 1) % AF]), hv, lv);
           }
           h[f][j] = __builtin_bit_cast(bf16x8, hv);
           l[f][j] = __builtin_bit_cast(bf16x8, lv);
@@ -247,10 +294,13 @@ gemm_f32_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
         for (int f = 0; f < MF; f++) {
           f32x16 p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][0], w0, zero, 0, 0, 0);
           p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][1], w1, p, 0, 0, 0);
-          p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[f][0], w0, p, 0, 0, 0);
-          p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[f][1], w1, p, 0, 0, 0);
+          if (!I8) {
+            p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[f][0], w0, p, 0, 0, 0);
+            p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(l[f][1], w1, p, 0, 0, 0);
+          }
 #pragma unroll
-          for (int e = 0; e < 16; e++) acc[f][c][e] = fmaf(s, p[e], acc[f][c][e]);
+          for (int e = 0; e < 16; e++)
+            acc[f][c][e] = fmaf(I8 ? s * xs[b & 1][I8 ? f : 0][e / 4][e % 4] : s, p[e], acc[f][c][e]);
         }
       }
     }
@@ -302,8 +352,8 @@ gemm_f32_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
 // ahead and convert step s + 2 into LDS buffer (s + 2) % 3 while the consumers
 // run step s. A wave's loads complete in issue order, so a wave that loads both
 // would wait for its codes (HBM) whenever it waits for activations (L2).
-template <int FMT, typename ST, bool PK, int MF, int NF, int RA>
-__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void gemm_f32_rs_kernel(
+template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int RA>
+__global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void gemm_blk_rs_kernel(
     const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x, void* __restrict__ y, int M,
     int K, int N, int npad, int y_dtype, int tiles_m, uint32_t x_bytes) {
   constexpr int NB = kGbBlocks, RW = 3;
@@ -311,7 +361,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   constexpr int NT = G * NB * 32 / 256;
   constexpr int NS = (BN * NB + 255) / 256;
   constexpr int TPS = NB * NF * MF, PR = TPS % 3 == 0 ? 3 : 4;  // tiles per step, block sums in flight
-  static_assert(NB % RA == 0 && NB * NF % 3 == 0 && NB * NF % 4 == 0 && TPS % PR == 0, "rings turn whole in a step");
+  static_assert(XT == kXtI8 ? NB % RA == 0 && NF % 2 == 0 && MF == 1
+                            : NB % RA == 0 && NB * NF % 3 == 0 && NB * NF % 4 == 0 && TPS % PR == 0,
+                "rings turn whole in a step");
   struct Lds {
     u32x4 w[3][NB][2][NF][64];
     float s[3][NB][BN];
@@ -421,109 +473,189 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   const int m0 = tm * BM + wave * 32 * MF;
   const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
   const int r32_last = (M + 31) / 32 - 1;
-  uint32_t xo[MF];
-#pragma unroll
-  for (int f = 0; f < MF; f++)
-    xo[f] = PK ? (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
-               : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
-  u32x4 a[RA][MF][4];
-  auto aload = [&](int slot, int kb) {
-    kb = min(kb, nkb - 1);
-#pragma unroll
-    for (int f = 0; f < MF; f++)
-#pragma unroll
-      for (int i = 0; i < 4; i++)
-        a[slot][f][i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
-                                                         (int)((uint32_t)kb * (PK ? 4096u : 128u)), 0));
-  };
-  f32x16 zero;
+  f32x16 zero, acc[MF][NF];
 #pragma unroll
   for (int e = 0; e < 16; e++) zero[e] = 0.0f;
-  f32x16 acc[MF][NF], p[PR];
 #pragma unroll
   for (int f = 0; f < MF; f++)
 #pragma unroll
     for (int c = 0; c < NF; c++) acc[f][c] = zero;
+  if constexpr (XT == kXtI8) {
+    f32x32 zero2;
 #pragma unroll
-  for (int i = 0; i < PR; i++) p[i] = zero;
-  bf16x8 w[3][2];
-  float ws[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // scales of the column fragments j - 2 .. j + 1
-  bf16x8 h[MF][2], l[MF][2], lp[2];  // the block's hi and lo fragments; the last tile's lo of the block before
-  const bf16x8 none = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-  w[2][0] = w[2][1] = lp[0] = lp[1] = none;
-  auto wread = [&](int j, int buf, int b, int c) {
-    w[j % 3][0] = __builtin_bit_cast(bf16x8, L.w[buf][b][0][c][lane]);
-    w[j % 3][1] = __builtin_bit_cast(bf16x8, L.w[buf][b][1][c][lane]);
-    ws[j % 4] = L.s[buf][b][32 * c + l32];
-  };
+    for (int e = 0; e < 32; e++) zero2[e] = 0.0f;
+    // int8 activations. Tiles in pairs of column fragments; the scales of a pair's
+    // outputs, xs[row] ws[column], come from one 32x32x1 two-block f32 MFMA (one
+    // rounding, as a multiply; 32 cycles a tile where 16 multiplies on the VALU
+    // cost about 70 beside the FMAs that wait for them), issued ahead of the next
+    // pair's MFMAs, beside which the pair before is scaled
+    const uint32_t r32 = (uint32_t)min(m0 / 32, r32_last) * (uint32_t)nkb;
+    const uint32_t xo = r32 * 2048u + 16u * (uint32_t)lane;
+    const uint32_t so = ((uint32_t)(r32_last + 1) * (uint32_t)nkb * 512u + r32 * 32u + (uint32_t)l32) * 4u;
+    constexpr int NP = NF / 2, TP = NB * NP;  // pairs per block and step
+    u32x4 a[RA][2];
+    float xs[RA];
+    auto aload = [&](int slot, int kb) {
+      kb = min(kb, nkb - 1);
 #pragma unroll
-  for (int i = 0; i < RA - 1; i++) aload(i, i);
-  __syncthreads();
-  wread(0, 0, 0, 0);
-  int buf = 0;
-  for (int s = 0; s < steps; s++) {
-    const int nbuf = buf == 2 ? 0 : buf + 1;
-    // tile i of the step: column fragment j = i / MF, row fragment i % MF. Its
-    // four MFMAs (hi, hi, lo, lo of the two 16-k halves) are spread over two
-    // turns, so that two chains alternate, and the block sums are scaled in
-    // the turn after, beside the MFMAs of the next two tiles
+      for (int i = 0; i < 2; i++)
+        a[slot][i] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo + 1024u * i), (int)((uint32_t)kb * 2048u), 0));
+      xs[slot] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)so, (int)((uint32_t)kb * 128u), 0));
+    };
+    f32x16 p[2][2];
 #pragma unroll
-    for (int i = 0; i < TPS; i++) {
-      const int j = i / MF, f = i % MF, b = j / NF, c = j % NF;
-      const int q1 = (i + TPS - 1) % TPS, j1 = q1 / MF, f1 = q1 % MF;  // the tile before
-      const int q2 = (i + TPS - 2) % TPS, j2 = q2 / MF, f2 = q2 % MF;  // and the one before it
-      if (c == 0 && f == 0) {
+    for (int i = 0; i < 2; i++) p[1][i] = zero;
+    bf16x8 w[2][2][2];  // [slot][tile of the pair][half]
+    float ws[2];        // lanes 0..31 the pair's first column fragment, 32..63 its second
+    f32x32 sc2[2];      // scales of the pair's outputs
+    sc2[1] = zero2;
+    auto wread = [&](int slot, int buf, int b, int q) {
 #pragma unroll
-        for (int ff = 0; ff < MF; ff++)
+      for (int i = 0; i < 2; i++)
 #pragma unroll
-          for (int e = 0; e < 2; e++) {
-            const u32x4* r = a[b % RA][ff];
-            u32x4 hv, lv;
-            if (PK) {
-              hv = r[e];
-              lv = r[2 + e];
-            } else {
-              split8(__builtin_bit_cast(f32x4, r[2 * e]), __builtin_bit_cast(f32x4, r[2 * e + 1]), hv, lv);
-            }
-            h[ff][e] = __builtin_bit_cast(bf16x8, hv);
-            l[ff][e] = __builtin_bit_cast(bf16x8, lv);
-          }
-      }
-      if (f == 0) wread(j + 1, j + 1 < NB * NF ? buf : nbuf, (j + 1) / NF % NB, (j + 1) % NF);
-      const bool head = c == 0 && f == 0;  // the tile before is of the block before
-      p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][0], w[j % 3][0], zero, 0, 0, 0);
-      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[0] : l[f1][0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
-      p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][1], w[j % 3][1], p[i % PR], 0, 0, 0);
-      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[1] : l[f1][1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+        for (int j = 0; j < 2; j++) w[slot][i][j] = __builtin_bit_cast(bf16x8, L.w[buf][b][j][2 * q + i][lane]);
+      ws[slot] = L.s[buf][b][64 * q + lane];
+    };
 #pragma unroll
-      for (int e = 0; e < 16; e++)
-        acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
-      if (c == 0 && f == 0) aload((b + RA - 1) % RA, s * NB + b + RA - 1);
-      if (c == NF - 1 && f == MF - 1) {
-        lp[0] = l[f][0];
-        lp[1] = l[f][1];
-      }
-      if (PK) {
+    for (int i = 0; i < RA - 1; i++) aload(i, i);
+    __syncthreads();
+    wread(0, 0, 0, 0);
+    int buf = 0;
+    for (int s = 0; s < steps; s++) {
+      const int nbuf = buf == 2 ? 0 : buf + 1;
+#pragma unroll
+      for (int i = 0; i < TP; i++) {
+        const int b = i / NP, q = i % NP, cur = i & 1, q1 = (i + TP - 1) % TP % NP;
+        if (q == 0) aload((b + RA - 1) % RA, s * NB + b + RA - 1);
+        wread(cur ^ 1, i + 1 < TP ? buf : nbuf, (i + 1) / NP % NB, (i + 1) % NP);
+        sc2[cur] = __builtin_amdgcn_mfma_f32_32x32x1f32(xs[b % RA], ws[cur], zero2, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 2; j++)
+#pragma unroll
+          for (int t = 0; t < 2; t++)
+            p[cur][t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a[b % RA][j]), w[cur][t][j],
+                                                                j > 0 ? p[cur][t] : zero, 0, 0, 0);
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+          for (int e = 0; e < 16; e++)
+            acc[0][2 * q1 + t][e] = fmaf(sc2[cur ^ 1][16 * t + e], p[cur ^ 1][t][e], acc[0][2 * q1 + t][e]);
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
       }
-      __builtin_amdgcn_sched_barrier(0);
+      __syncthreads();
+      buf = nbuf;
     }
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int e = 0; e < 16; e++)
+        acc[0][NF - 2 + t][e] = fmaf(sc2[1][16 * t + e], p[1][t][e], acc[0][NF - 2 + t][e]);
+  } else {
+    uint32_t xo[MF];
+#pragma unroll
+    for (int f = 0; f < MF; f++)
+      xo[f] = PK ? (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
+                 : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
+    u32x4 a[RA][MF][4];
+    auto aload = [&](int slot, int kb) {
+      kb = min(kb, nkb - 1);
+#pragma unroll
+      for (int f = 0; f < MF; f++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          a[slot][f][i] = __builtin_bit_cast(
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
+                                                           (int)((uint32_t)kb * (PK ? 4096u : 128u)), 0));
+    };
+    f32x16 p[PR];
+#pragma unroll
+    for (int i = 0; i < PR; i++) p[i] = zero;
+    bf16x8 w[3][2];
+    float ws[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // scales of the column fragments j - 2 .. j + 1
+    bf16x8 h[MF][2], l[MF][2], lp[2];  // the block's hi and lo fragments; the last tile's lo of the block before
+    const bf16x8 none = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
+    w[2][0] = w[2][1] = lp[0] = lp[1] = none;
+    auto wread = [&](int j, int buf, int b, int c) {
+      w[j % 3][0] = __builtin_bit_cast(bf16x8, L.w[buf][b][0][c][lane]);
+      w[j % 3][1] = __builtin_bit_cast(bf16x8, L.w[buf][b][1][c][lane]);
+      ws[j % 4] = L.s[buf][b][32 * c + l32];
+    };
+#pragma unroll
+    for (int i = 0; i < RA - 1; i++) aload(i, i);
     __syncthreads();
-    buf = nbuf;
-  }
-  {
-    constexpr int q1 = TPS - 1, j1 = q1 / MF, f1 = q1 % MF, q2 = TPS - 2, j2 = q2 / MF, f2 = q2 % MF;
-    p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
-    p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+    wread(0, 0, 0, 0);
+    int buf = 0;
+    for (int s = 0; s < steps; s++) {
+      const int nbuf = buf == 2 ? 0 : buf + 1;
+      // tile i of the step: column fragment j = i / MF, row fragment i % MF. Its
+      // four MFMAs (hi, hi, lo, lo of the two 16-k halves) are spread over two
+      // turns, so that two chains alternate, and the block sums are scaled in
+      // the turn after, beside the MFMAs of the next two tiles
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
+      for (int i = 0; i < TPS; i++) {
+        const int j = i / MF, f = i % MF, b = j / NF, c = j % NF;
+        const int q1 = (i + TPS - 1) % TPS, j1 = q1 / MF, f1 = q1 % MF;  // the tile before
+        const int q2 = (i + TPS - 2) % TPS, j2 = q2 / MF, f2 = q2 % MF;  // and the one before it
+        if (c == 0 && f == 0) {
 #pragma unroll
-    for (int e = 0; e < 16; e++) acc[f1][j1 % NF][e] = fmaf(ws[j1 % 4], p[q1 % PR][e], acc[f1][j1 % NF][e]);
+          for (int ff = 0; ff < MF; ff++)
+#pragma unroll
+            for (int e = 0; e < 2; e++) {
+              const u32x4* r = a[b % RA][ff];
+              u32x4 hv, lv;
+              if (PK) {
+                hv = r[e];
+                lv = r[2 + e];
+              } else {
+                split8(__builtin_bit_cast(f32x4, r[2 * e]), __builtin_bit_cast(f32x4, r[2 * e + 1]), hv, lv);
+              }
+              h[ff][e] = __builtin_bit_cast(bf16x8, hv);
+              l[ff][e] = __builtin_bit_cast(bf16x8, lv);
+            }
+        }
+        if (f == 0) wread(j + 1, j + 1 < NB * NF ? buf : nbuf, (j + 1) / NF % NB, (j + 1) % NF);
+        const bool head = c == 0 && f == 0;  // the tile before is of the block before
+        p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][0], w[j % 3][0], zero, 0, 0, 0);
+        p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[0] : l[f1][0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
+        p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][1], w[j % 3][1], p[i % PR], 0, 0, 0);
+        p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[1] : l[f1][1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 16; e++)
+          acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
+        if (c == 0 && f == 0) aload((b + RA - 1) % RA, s * NB + b + RA - 1);
+        if (c == NF - 1 && f == MF - 1) {
+          lp[0] = l[f][0];
+          lp[1] = l[f][1];
+        }
+        if (PK) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
+          }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __syncthreads();
+      buf = nbuf;
+    }
+    {
+      constexpr int q1 = TPS - 1, j1 = q1 / MF, f1 = q1 % MF, q2 = TPS - 2, j2 = q2 / MF, f2 = q2 % MF;
+      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
+      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[f1][j1 % NF][e] = fmaf(ws[j1 % 4], p[q1 % PR][e], acc[f1][j1 % NF][e]);
+    }
   }
 
 #pragma unroll
@@ -544,27 +676,27 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     }
 }
 
-template <int FMT, typename ST, bool PK, int MF, int NF, int RA>
+template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int RA>
 static hipError_t launch_rs_t(const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
                            hipEvent_t done) {
   constexpr int BM = 128 * MF, BN = 32 * NF;
   const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
   if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
-  const int64_t bytes = std::min<int64_t>((PK ? (m + 31) / 32 * 32 : m) * a.k * 4, UINT32_MAX);
-  hipExtLaunchKernelGGL((gemm_f32_rs_kernel<FMT, ST, PK, MF, NF, RA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0,
+  const int64_t bytes = std::min<int64_t>(PK ? packed_bytes(XT, m, a.k) : m * a.k * 4, UINT32_MAX);
+  hipExtLaunchKernelGGL((gemm_blk_rs_kernel<FMT, ST, XT, PK, MF, NF, RA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0,
                         a.stream, begin, done, 0, a.q, static_cast<const ST*>(a.scales), x, y, (int)m, (int)a.k,
                         (int)a.n, (int)a.npad, a.y_dtype, (int)tiles_m, (uint32_t)bytes);
   return hipGetLastError();
 }
 
-template <int FMT, typename ST, bool PK, int MF, int NF, int WM, int KG>
+template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int WM, int KG>
 static hipError_t launch_t(const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
                            hipEvent_t done) {
   constexpr int BM = 32 * MF * WM, BN = 32 * NF;
   const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
   if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
-  const int64_t bytes = std::min<int64_t>((PK ? (m + 31) / 32 * 32 : m) * a.k * 4, UINT32_MAX);
-  hipExtLaunchKernelGGL((gemm_f32_kernel<FMT, ST, PK, MF, NF, WM, KG>), dim3((unsigned)(tiles_m * tiles_n)),
+  const int64_t bytes = std::min<int64_t>(PK ? packed_bytes(XT, m, a.k) : m * a.k * 4, UINT32_MAX);
+  hipExtLaunchKernelGGL((gemm_blk_kernel<FMT, ST, XT, PK, MF, NF, WM, KG>), dim3((unsigned)(tiles_m * tiles_n)),
                         dim3(64 * WM * KG), 0, a.stream, begin, done, 0, a.q, static_cast<const ST*>(a.scales), x, y,
                         (int)m, (int)a.k, (int)a.n, (int)a.npad, a.y_dtype, (int)tiles_m, (uint32_t)bytes);
   return hipGetLastError();
@@ -586,20 +718,33 @@ namespace {
 // The kernel before these (one 128 x 128 tile, both operands converted in every
 // workgroup, two barriers per 32-block) took 275 us at m = 333, 11008 x 4096
 // (Q4_0).
-struct F32Tile {
+struct BlkTile {
   int bm, bn, kg, one_ns, block_ns, round_ns;
 };
-constexpr F32Tile kF32Tiles[] = {{32, 32, 4, 310, 262, 0},
+constexpr BlkTile kF32Tiles[] = {{32, 32, 4, 310, 262, 0},
                                  {64, 32, 4, 500, 440, 0},
                                  {128, 64, 1, 360, 245, 0},
                                  {128, 96, 1, 315, 315, 4000},
                                  {128, 192, 1, 570, 570, 5000}};
 
-int pick_tile(int64_t m, int64_t k, int64_t n, int cu_count) {
+// int8 activations, fitted alike. Measured, us a call with the packing pass, Q8_0,
+// f32 y, against the kernel before (int8 MFMA, every int32 dot converted and
+// scaled by the product of its two scales on the VALU; 32 x 64 to 64 x 128 tiles):
+//                        before  32x32  128x64  128x128
+//   11008 x 4096  m = 17   59.8   25.9    31.7    48.9
+//                 m = 128  60.7   64      33.4    52
+//                 m = 256  83.3  109      58.9    51.3
+//                 m = 512 107.6  205      87.4    99.9
+//                 m = 1024 227.5 429     170     150
+//   4096 x 4096   m = 512  62.1   83.3    35.2    51.8
+//   28672 x 2048  m = 512 141.5  306     115     111
+constexpr BlkTile kI8Tiles[] = {{32, 32, 4, 340, 300, 0}, {128, 64, 1, 200, 200, 2500}, {128, 128, 1, 315, 315, 3500}};
+
+int pick_tile(const BlkTile* table, int count, int64_t m, int64_t k, int64_t n, int cu_count) {
   int best = 0;
   int64_t best_cost = INT64_MAX;
-  for (int i = 0; i < (int)(sizeof(kF32Tiles) / sizeof(kF32Tiles[0])); i++) {
-    const F32Tile& t = kF32Tiles[i];
+  for (int i = 0; i < count; i++) {
+    const BlkTile& t = table[i];
     const int64_t tiles = (m + t.bm - 1) / t.bm * ((n + t.bn - 1) / t.bn), c = (tiles + cu_count - 1) / cu_count;
     const int64_t cost = k / 32 * std::max<int64_t>(t.one_ns, c * t.block_ns) / t.kg + c * t.round_ns;
     if (cost < best_cost) best_cost = cost, best = i;
@@ -607,15 +752,15 @@ int pick_tile(int64_t m, int64_t k, int64_t n, int cu_count) {
   return best;
 }
 
-template <int FMT, typename ST, bool PK>
+template <int FMT, typename ST, int XT, bool PK>
 hipError_t launch_tile(int tile, const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
                            hipEvent_t done) {
   switch (tile) {
-    case 0: return launch_t<FMT, ST, PK, 1, 1, 1, 4>(a, x, y, m, begin, done);
-    case 1: return launch_t<FMT, ST, PK, 2, 1, 1, 4>(a, x, y, m, begin, done);
-    case 2: return launch_t<FMT, ST, PK, 1, 2, 4, 1>(a, x, y, m, begin, done);
-    case 3: return launch_rs_t<FMT, ST, PK, 1, 3, 4>(a, x, y, m, begin, done);
-    default: return launch_rs_t<FMT, ST, PK, 1, 6, 2>(a, x, y, m, begin, done);
+    case 0: return launch_t<FMT, ST, XT, PK, 1, 1, 1, 4>(a, x, y, m, begin, done);
+    case 1: return launch_t<FMT, ST, XT, PK, 2, 1, 1, 4>(a, x, y, m, begin, done);
+    case 2: return launch_t<FMT, ST, XT, PK, 1, 2, 4, 1>(a, x, y, m, begin, done);
+    case 3: return launch_rs_t<FMT, ST, XT, PK, 1, 3, 4>(a, x, y, m, begin, done);
+    default: return launch_rs_t<FMT, ST, XT, PK, 1, 6, 2>(a, x, y, m, begin, done);
   }
 }
 
@@ -625,6 +770,13 @@ int64_t chunk_rows(int64_t k, bool packed) {
   const int64_t rows = (packed ? (int64_t)RQ_NOALLOC_SCRATCH_MAX : (int64_t)UINT32_MAX) / (4 * k);
   return rows >= 256 ? rows / 256 * 256 : packed ? rows / 32 * 32 : std::max<int64_t>(rows, 1);
 }
+
+// int8: the packed copy within 64 MiB, at least 32 rows
+int64_t i8_chunk_rows(int64_t k) {
+  const int64_t rows = (int64_t)(64 << 20) / (2 * k + k / 8);
+  return rows >= 256 ? rows / 256 * 256 : std::max<int64_t>(rows / 32 * 32, 32);
+}
+
 }  // namespace
 
 size_t gemm_f32_pack_bytes(int64_t m, int64_t k) {
@@ -635,7 +787,7 @@ template <int FMT, typename ST>
 static hipError_t launch_x(const MatmulArgs& a, int cu_count) {
   const bool pk = a.scratch != nullptr;
   // of the whole call, whatever its chunks; a tile's weights within 32-bit offsets
-  const int tile = a.k > (int64_t)1 << 24 ? 0 : pick_tile(a.m, a.k, a.n, cu_count);
+  const int tile = a.k > (int64_t)1 << 24 ? 0 : pick_tile(kF32Tiles, 5, a.m, a.k, a.n, cu_count);
   const int64_t chunk = chunk_rows(a.k, pk);
   for (int64_t m0 = 0; m0 < a.m; m0 += chunk) {
     const int64_t m = std::min(chunk, a.m - m0);
@@ -649,11 +801,43 @@ static hipError_t launch_x(const MatmulArgs& a, int cu_count) {
                             (int)a.k);
       if (hipError_t e = hipGetLastError()) return e;
     }
-    const hipError_t e = pk ? launch_tile<FMT, ST, true>(tile, a, a.scratch, y, m, nullptr, done)
-                            : launch_tile<FMT, ST, false>(tile, a, x, y, m, m0 == 0 ? a.ev_main[0] : nullptr, done);
+    const hipError_t e = pk ? launch_tile<FMT, ST, RQ_F32, true>(tile, a, a.scratch, y, m, nullptr, done)
+                            : launch_tile<FMT, ST, RQ_F32, false>(tile, a, x, y, m, m0 == 0 ? a.ev_main[0] : nullptr, done);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+template <int FMT, typename ST>
+static hipError_t launch_i8(const MatmulArgs& a, int cu_count) {
+  const int64_t chunk = i8_chunk_rows(a.k), nb = a.k / 32;
+  const int tile = a.k > (int64_t)1 << 24 ? 0 : pick_tile(kI8Tiles, 3, a.m, a.k, a.n, cu_count);
+  for (int64_t m0 = 0; m0 < a.m; m0 += chunk) {
+    const int64_t m = std::min(chunk, a.m - m0);
+    void* y = static_cast<uint8_t*>(a.y) + m0 * a.n * (a.y_dtype == RQ_F32 ? 4 : 2);
+    const int64_t blocks = (m + 31) / 32 * ((nb + 1) / 2);
+    hipExtLaunchKernelGGL(pack_x32_i8_kernel, dim3((unsigned)blocks), dim3(256), 0, a.stream, nullptr,
+                          m0 == 0 ? a.ev_main[0] : nullptr, 0, static_cast<const int8_t*>(a.x) + m0 * a.k,
+                          a.ops.act_scale + m0 * nb, static_cast<uint16_t*>(a.scratch), (int)m, (int)a.k);
+    if (hipError_t e = hipGetLastError()) return e;
+    const hipEvent_t done = m0 + chunk >= a.m ? a.ev_main[1] : nullptr;
+    const hipError_t e =
+        tile == 0   ? launch_t<FMT, ST, kXtI8, true, 1, 1, 1, 4>(a, a.scratch, y, m, nullptr, done)
+        : tile == 1 ? launch_rs_t<FMT, ST, kXtI8, true, 1, 2, 4>(a, a.scratch, y, m, nullptr, done)
+                    : launch_rs_t<FMT, ST, kXtI8, true, 1, 4, 4>(a, a.scratch, y, m, nullptr, done);
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+size_t gemm_i8_pack_bytes(int64_t m, int64_t k) {
+  return (size_t)packed_bytes(kXtI8, std::min(m, i8_chunk_rows(k)), k);
+}
+
+hipError_t launch_gemm_i8(const MatmulArgs& a, int cu_count) {
+  if (a.format == RQ_Q8_0) return launch_i8<RQ_Q8_0, float>(a, cu_count);
+  if (a.scale_dtype == RQ_F16) return launch_i8<RQ_Q4_0, uint16_t>(a, cu_count);
+  return launch_i8<RQ_Q4_0, float>(a, cu_count);
 }
 
 hipError_t launch_gemm(const MatmulArgs& a, int cu_count) {

@@ -175,7 +175,9 @@ hipError_t launch_gemm_bf16(const MatmulArgs& a, int cu_count);
 int gemm_sm_slices(int format, int64_t m, int64_t k, int64_t npad, int cu_count);
 bool gemm_sm_takes(int format, int64_t m, int64_t k);
 hipError_t launch_gemm_sm(const MatmulArgs& a, int ks);
-// int8 activations (x_dtype kXtI8, scales / sums in a.ops), m > 16 (gemm_i8.hip)
+// int8 activations (x_dtype kXtI8, scales in a.ops), m > 16 (gemm.hip), with
+// gemm_i8_pack_bytes of scratch
+size_t gemm_i8_pack_bytes(int64_t m, int64_t k);
 hipError_t launch_gemm_i8(const MatmulArgs& a, int cu_count);
 // bf16 x, m > 128: 256 x 192 tiles on 32x32x16 MFMA, one wave per SIMD
 // (gemm_wide.hip), where its tiles fill their rounds of the CUs

@@ -1,0 +1,39 @@
+"""The int8-activation GEMM (csrc/gemm.hip, m > 16) against 64-bit products of
+the quantized activations and the dequantized weight: the block dots are exact,
+each block adds its product of scales (one rounding), its product with the dot
+and the sum's rounding: |y - ref| <= (in / 32 + 8) 2^-23 sum_b |ws xs dot_b|, and
+2^-8 |y| more for bf16 y.
+"""
+import numpy as np
+import pytest
+from test_gpu_gemm_f32 import ctx, rows, torch, weight  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+# the tiles (32 x 32, 128 x 64, 128 x 128) with row, column and K-step remainders
+SHAPES = [(17, 3, 32), (18, 4100, 96), (40, 300, 1056), (129, 4099, 416), (300, 2050, 224), (256, 11008, 160),
+          (200, 30001, 288)]
+
+
+@pytest.mark.parametrize("fmt,ydt", [("q8", "f32"), ("q4h", "f32"), ("q4f", "bf16")])
+@pytest.mark.parametrize("m,out,in_", SHAPES)
+def test_gemm_i8(torch, ctx, m, out, in_, fmt, ydt):  # noqa: F811
+    import raster_amd
+
+    print(f"[gpu] int8 GEMM {fmt} m={m} {out}x{in_} y={ydt}", flush=True)
+    w = weight(ctx, fmt, out, in_, m)
+    x = rows(torch, m, in_, out)
+    x[2] = 0.0
+    xq, xs, xsum = raster_amd.quantize_act_i8(ctx, x, in_)
+    y = w.matmul_i8(xq, xs, xsum, out_dtype=torch.bfloat16 if ydt == "bf16" else torch.float32).double()
+    W = w.dequant().double()
+    w.destroy()
+    ref, mag = torch.zeros_like(y), torch.zeros_like(y)
+    for b in range(in_ // 32):
+        k = slice(32 * b, 32 * b + 32)
+        d = (xq[:, k].double() * xs[:, b:b + 1].double()) @ W[:, k].T
+        ref += d
+        mag += d.abs()
+    bound = (in_ / 32 + 8) * 2.0 ** -23 * mag + (2.0 ** -8 * ref.abs() if ydt == "bf16" else 0.0)
+    # the dequantized weight is scale * code rounded to f32: one more rounding of the operands
+    assert bool(((y - ref).abs() <= bound + 2.0 ** -23 * (x.abs().double() @ W.abs().T)).all())
