@@ -147,6 +147,7 @@ constexpr int kMaxDims = 512;
 // head_dim weighted values.
 constexpr int kAttnRec = 4;
 constexpr int kMaxSplits = 64;
+constexpr int kGqaRows = 8;  // cached rows per lane and chunk of the grouped-query kernel
 
 template <int TPR, int NV, int NP, int THREADS>
 __global__ __launch_bounds__(THREADS) void decode_attention_chunk_kernel(
@@ -350,21 +351,65 @@ __global__ __launch_bounds__(THREADS) void decode_attention_chunk_kernel(
   }
 }
 
+namespace {
+
+// v from lane ^ D (D 1, 2, 8: DPP), lane ^ 7 for D = 4
+template <int D>
+__device__ __forceinline__ float lane_pair(float v) {
+  const int i = __float_as_int(v);
+  if (D == 1) return __int_as_float(dpp_xor1(i));
+  if (D == 2) return __int_as_float(dpp_xor2(i));
+  if (D == 4) return __int_as_float(dpp_half_mirror(i));
+  if (D == 8) return __int_as_float(__builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, false));  // row_ror:8
+  return __shfl_xor(v, D, 64);
+}
+
+// Sums over TPR lanes of N values at once: every step adds the halves of the
+// values between lane pairs, a lane keeping one half (the upper one where its
+// bit is set), so N values cost about N exchanges in all instead of log2(TPR)
+// each. Value i ends in the lanes whose top bits (of the TPR-lane index) are i's
+// top bits; v[0 .. max(1, N / TPR)) hold what is left.
+template <int N, int D>
+__device__ __forceinline__ void reduce_scatter(float* v, int lane) {
+  if constexpr (D >= 1) {
+    if constexpr (N > 1) {
+      const bool up = (lane & D) != 0;
+#pragma unroll
+      for (int i = 0; i < N / 2; i++) {
+        const float give = up ? v[i] : v[i + N / 2], keep = up ? v[i + N / 2] : v[i];
+        v[i] = keep + lane_pair<D>(give);
+      }
+      reduce_scatter<N / 2, D / 2>(v, lane);
+    } else {
+      v[0] += lane_pair<D>(v[0]);
+      reduce_scatter<1, D / 2>(v, lane);
+    }
+  }
+}
+
+}  // namespace
+
 // Grouped-query form of the chunk kernel: one workgroup per (KV head, row
 // range) serves all G query heads that read that KV head, so each cached row
-// is loaded once instead of G times. Per row a lane forms the G partial dot
-// products of its dimensions; each head keeps its own online softmax state.
-// G query heads hkv G .. hkv G + G - 1; 4 waves; 2 rows per lane per chunk.
-// LDS (dynamic): qr[G][hd], kr[hd], vn[hd], wacc[WAVES][G][hd], wm / wl[WAVES][G].
+// is loaded once instead of G times. Eight rows per lane per chunk, the chunk's
+// K and V in flight together; a lane forms the 8 G partial dot products of its
+// dimensions, which reduce_scatter sums to one score per lane (8 / TPR G);
+// the softmax weights go back to all lanes through LDS. Each head keeps its own
+// online softmax state per wave.
+// G query heads hkv G .. hkv G + G - 1; 4 waves.
+// LDS (dynamic): qr[G][hd], kr[hd], vn[hd], wacc[WAVES][G][hd], wm / wl / al[WAVES][G], sp[WAVES 64/TPR][8][G].
 template <int TPR, int NV, int G>
 __global__ __launch_bounds__(kAttnThreads) void decode_attention_gqa_kernel(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ v, float* __restrict__ kcache,
     float* __restrict__ vcache, int pos, int n_q, int n_kv, int head_dim, double theta, float scale,
     float* __restrict__ out, int nsplit, int rps, float* __restrict__ part) {
   constexpr int WAVES = kAttnThreads / 64;
-  constexpr int NP = 2;
+  constexpr int NP = kGqaRows;
   constexpr int RW = 64 / TPR;         // rows per wave per load
   constexpr int CH = WAVES * RW * NP;  // rows per chunk
+  constexpr int V = NP * G;            // scores per row group and chunk
+  constexpr int H = V > TPR ? V / TPR : 1;  // held by a lane
+  constexpr int DUP = V < TPR ? TPR / V : 1;  // lanes that hold the same score
   extern __shared__ __attribute__((aligned(16))) float gsm[];
   float* qr = gsm;                         // [G][head_dim]
   float* kr = qr + G * head_dim;           // [head_dim]
@@ -372,6 +417,8 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_gqa_kernel(
   float* wacc = vn + head_dim;             // [WAVES][G][head_dim]
   float* wm = wacc + WAVES * G * head_dim;  // [WAVES][G]
   float* wl = wm + WAVES * G;               // [WAVES][G]
+  float* al = wl + WAVES * G;               // [WAVES][G]
+  float* sp = al + WAVES * G;               // [WAVES * RW][NP][G]
   const int hkv = (int)blockIdx.x % n_kv, split = (int)blockIdx.x / n_kv, hq0 = hkv * G;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -379,23 +426,31 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_gqa_kernel(
   const int half = head_dim / 2, kvd = n_kv * head_dim;
   const int r0 = min(split * rps, pos), r1 = min(r0 + rps, pos);
   const int nch = (r1 - r0 + CH - 1) / CH;
+  int dc[NV];
+  bool dlive[NV];
+#pragma unroll
+  for (int nv = 0; nv < NV; nv++) {
+    const int d = 4 * sub + 4 * TPR * nv;
+    dlive[nv] = d < head_dim;
+    dc[nv] = min(d, head_dim - 4);
+  }
   const float* kb = kcache + hkv * head_dim;
   const float* vb = vcache + hkv * head_dim;
 
-  f32x4 kx[2][NP][NV], vx[2][NP][NV];
-  auto load = [&](int slot, int c) {
+  f32x4 kx[NP][NV], vx[NP][NV];
+  auto load = [&](f32x4 (&x)[NP][NV], const float* base, int c) {
 #pragma unroll
     for (int p = 0; p < NP; p++) {
-      const int row = min(r0 + c * CH + p * WAVES * RW + wave * RW + rg, r1 - 1);
+      const int row = min(r0 + c * CH + (p * WAVES + wave) * RW + rg, r1 - 1);
 #pragma unroll
-      for (int nv = 0; nv < NV; nv++) {
-        const int d = min(4 * sub + 4 * TPR * nv, head_dim - 4);
-        kx[slot][p][nv] = *reinterpret_cast<const f32x4*>(kb + (int64_t)row * kvd + d);
-        vx[slot][p][nv] = *reinterpret_cast<const f32x4*>(vb + (int64_t)row * kvd + d);
-      }
+      for (int nv = 0; nv < NV; nv++)
+        x[p][nv] = *reinterpret_cast<const f32x4*>(base + (int64_t)row * kvd + dc[nv]);
     }
   };
-  if (nch > 0) load(0, 0);
+  if (nch > 0) {
+    load(kx, kb, 0);
+    load(vx, vb, 0);
+  }
 
   // RoPE of the G queries and of the KV head's new key (the angle depends on
   // the dimension only); the value as is
@@ -421,141 +476,130 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_gqa_kernel(
       vcache[(int64_t)pos * kvd + hkv * head_dim + d] = vn[d];
     }
   }
-  f32x4 q4[G][NV];
-  bool dlive[NV];
+  f32x4 q4[G][NV], acc[G][NV];
 #pragma unroll
-  for (int nv = 0; nv < NV; nv++) {
-    const int d = 4 * sub + 4 * TPR * nv;
-    dlive[nv] = d < head_dim;
+  for (int g = 0; g < G; g++)
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-      const f32x4 t = *reinterpret_cast<const f32x4*>(qr + g * head_dim + min(d, head_dim - 4));
+    for (int nv = 0; nv < NV; nv++) {
+      const f32x4 t = *reinterpret_cast<const f32x4*>(qr + g * head_dim + dc[nv]);
       q4[g][nv] = dlive[nv] ? t : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      acc[g][nv] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     }
-  }
+  // the score(s) this lane ends with: value i = NP g + p, its head and rows
+  const int i0 = sub * V / TPR;
+  const int myg = i0 / NP, myp = i0 % NP;
+  float m = -INFINITY, l = 0.0f;  // of head myg, in this wave (l: of this lane's scores)
+  float* wsp = sp + (wave * RW + rg) * V;
 
-  float m[G], l[G];
-  f32x4 acc[G][NV];
+  for (int c = 0; c < nch; c++) {
+    float s[V];
 #pragma unroll
-  for (int g = 0; g < G; g++) {
-    m[g] = -INFINITY;
-    l[g] = 0.0f;
-#pragma unroll
-    for (int nv = 0; nv < NV; nv++) acc[g][nv] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  // fold the scores s[g][p] of NP rows (values vv) into head g's state
-  auto fold = [&](int g, const float (&s)[NP], const f32x4 (&vv)[NP][NV]) {
-    float mc = s[0];
-#pragma unroll
-    for (int p = 1; p < NP; p++) mc = fmaxf(mc, s[p]);
-#pragma unroll
-    for (int off = TPR; off < 64; off <<= 1) mc = fmaxf(mc, __shfl_xor(mc, off, 64));
-    const float mn = fmaxf(m[g], mc);
-    const float alpha = m[g] == -INFINITY ? 0.0f : expf(m[g] - mn);
-    l[g] *= alpha;
-#pragma unroll
-    for (int nv = 0; nv < NV; nv++) acc[g][nv] *= alpha;
-#pragma unroll
-    for (int p = 0; p < NP; p++) {
-      const float e = s[p] == -INFINITY ? 0.0f : expf(s[p] - mn);
-      l[g] += e;
-#pragma unroll
-      for (int nv = 0; nv < NV; nv++) acc[g][nv] += e * vv[p][nv];
-    }
-    m[g] = mn;
-  };
-  auto compute = [&](int slot, int c) {
-#pragma unroll
-    for (int g = 0; g < G; g++) {
-      float s[NP];
+    for (int g = 0; g < G; g++)
 #pragma unroll
       for (int p = 0; p < NP; p++) {
         float dot = 0.0f;
 #pragma unroll
         for (int nv = 0; nv < NV; nv++) {
-          const f32x4 kk = kx[slot][p][nv];
+          const f32x4 kk = kx[p][nv];
           dot += q4[g][nv][0] * kk[0] + q4[g][nv][1] * kk[1] + q4[g][nv][2] * kk[2] + q4[g][nv][3] * kk[3];
         }
-#pragma unroll
-        for (int off = TPR / 2; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
-        const int row = r0 + c * CH + p * WAVES * RW + wave * RW + rg;
-        s[p] = row < r1 ? dot * scale : -INFINITY;
+        s[g * NP + p] = dot;
       }
-      fold(g, s, vx[slot]);
+    if (c + 1 < nch) load(kx, kb, c + 1);
+    reduce_scatter<V, TPR / 2>(s, lane);
+    float mc = -INFINITY;
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+      const int row = r0 + c * CH + ((myp + h) * WAVES + wave) * RW + rg;
+      s[h] = row < r1 ? s[h] * scale : -INFINITY;
+      mc = fmaxf(mc, s[h]);
     }
-  };
-  for (int c = 0; c < nch; c += 2) {
-    if (c + 1 < nch) load(1, c + 1);
-    compute(0, c);
-    if (c + 1 >= nch) break;
-    if (c + 2 < nch) load(0, c + 2);
-    compute(1, c + 1);
+    // over the lanes of head myg, and the row groups
+#pragma unroll
+    for (int off = TPR / G / 2; off >= 1; off >>= 1) mc = fmaxf(mc, __shfl_xor(mc, off, 64));
+#pragma unroll
+    for (int off = TPR; off < 64; off <<= 1) mc = fmaxf(mc, __shfl_xor(mc, off, 64));
+    const float mn = fmaxf(m, mc);
+    const float alpha = m == -INFINITY ? 0.0f : expf(m - mn);
+    m = mn;
+    l *= alpha;
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+      const float e = s[h] == -INFINITY ? 0.0f : expf(s[h] - mn);
+      l += e;
+      wsp[(myp + h) * G + myg] = e;
+    }
+    al[wave * G + myg] = alpha;
+    // the wave's own exchange through LDS
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int g = 0; g < G; g++)
+#pragma unroll
+      for (int nv = 0; nv < NV; nv++) acc[g][nv] *= al[wave * G + g];
+#pragma unroll
+    for (int p = 0; p < NP; p++)
+#pragma unroll
+      for (int g = 0; g < G; g++)
+#pragma unroll
+        for (int nv = 0; nv < NV; nv++) acc[g][nv] += wsp[p * G + g] * vx[p][nv];
+    if (c + 1 < nch) load(vx, vb, c + 1);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
 
-  // the new row (pos) from LDS, folded into wave 0's states by its row group
-  // 0 (of the last range)
-  if (wave == 0 && split == nsplit - 1) {
-    f32x4 vv[NP][NV], kk[NV];
+  // each head: the wave's row groups
 #pragma unroll
-    for (int nv = 0; nv < NV; nv++) {
-      const int d = min(4 * sub + 4 * TPR * nv, head_dim - 4);
-      kk[nv] = *reinterpret_cast<const f32x4*>(kr + d);
-      vv[0][nv] = *reinterpret_cast<const f32x4*>(vn + d);
+  for (int off = TPR / G / 2; off >= DUP; off >>= 1) l += __shfl_xor(l, off, 64);
 #pragma unroll
-      for (int p = 1; p < NP; p++) vv[p][nv] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+  for (int off = TPR; off < 64; off <<= 1) {
+    l += __shfl_xor(l, off, 64);
 #pragma unroll
-    for (int g = 0; g < G; g++) {
-      float dot = 0.0f;
-#pragma unroll
-      for (int nv = 0; nv < NV; nv++)
-        dot += q4[g][nv][0] * kk[nv][0] + q4[g][nv][1] * kk[nv][1] + q4[g][nv][2] * kk[nv][2] +
-               q4[g][nv][3] * kk[nv][3];
-#pragma unroll
-      for (int off = TPR / 2; off >= 1; off >>= 1) dot += __shfl_xor(dot, off, 64);
-      float s[NP];
-      s[0] = rg == 0 ? dot * scale : -INFINITY;
-#pragma unroll
-      for (int p = 1; p < NP; p++) s[p] = -INFINITY;
-      fold(g, s, vv);
-    }
-  }
-
-  // each head: the wave's row groups, then the waves
-#pragma unroll
-  for (int g = 0; g < G; g++) {
-#pragma unroll
-    for (int off = TPR; off < 64; off <<= 1) {
-      l[g] += __shfl_xor(l[g], off, 64);
+    for (int g = 0; g < G; g++)
 #pragma unroll
       for (int nv = 0; nv < NV; nv++)
 #pragma unroll
         for (int e = 0; e < 4; e++) acc[g][nv][e] += __shfl_xor(acc[g][nv][e], off, 64);
-    }
-    if (rg == 0) {
-#pragma unroll
-      for (int nv = 0; nv < NV; nv++)
-        if (dlive[nv])
-          *reinterpret_cast<f32x4*>(&wacc[(wave * G + g) * head_dim + 4 * sub + 4 * TPR * nv]) = acc[g][nv];
-    }
-    if (lane == 0) {
-      wm[wave * G + g] = m[g];
-      wl[wave * G + g] = l[g];
-    }
   }
+#pragma unroll
+  for (int g = 0; g < G; g++)
+#pragma unroll
+    for (int nv = 0; nv < NV; nv++)
+      if (rg == 0 && dlive[nv]) *reinterpret_cast<f32x4*>(&wacc[(wave * G + g) * head_dim + dc[nv]]) = acc[g][nv];
+  wm[wave * G + myg] = m;
+  wl[wave * G + myg] = l;
+  // the new row's score (last range), one head after another over the waves
+  float* ns = al;  // [G], free after the barrier
   __syncthreads();
+  if (split == nsplit - 1) {
+    for (int g = wave; g < G; g += WAVES) {
+      float dot = 0.0f;
+      for (int d = lane; d < head_dim; d += 64) dot += qr[g * head_dim + d] * kr[d];
+      dot = wave_sum(dot);
+      if (lane == 0) ns[g] = dot * scale;
+    }
+    __syncthreads();
+  }
   const int rstride = kAttnRec + head_dim;
   for (int idx = tid; idx < G * head_dim; idx += kAttnThreads) {
     const int g = idx / head_dim, d = idx - g * head_dim;
-    float mx = wm[g];
+    const float sn = split == nsplit - 1 ? ns[g] : -INFINITY;
+    float mx = sn;
 #pragma unroll
-    for (int w = 1; w < WAVES; w++) mx = fmaxf(mx, wm[w * G + g]);
+    for (int w = 0; w < WAVES; w++) mx = fmaxf(mx, wm[w * G + g]);
     float a = 0.0f, sum = 0.0f;
 #pragma unroll
     for (int w = 0; w < WAVES; w++) {
       const float f = wm[w * G + g] == -INFINITY ? 0.0f : expf(wm[w * G + g] - mx);
       sum += f * wl[w * G + g];
       a += f * wacc[(w * G + g) * head_dim + d];
+    }
+    if (split == nsplit - 1) {
+      const float e = expf(sn - mx);
+      sum += e;
+      a += e * vn[d];
     }
     const int hq = hq0 + g;
     if (nsplit == 1) {
@@ -572,7 +616,8 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_gqa_kernel(
 }
 
 size_t decode_attention_gqa_lds(int64_t head_dim, int g) {
-  return (size_t)((g + 2) * head_dim + (kAttnThreads / 64) * (g * head_dim + 2 * g)) * sizeof(float);
+  const int64_t waves = kAttnThreads / 64, groups = waves * 64 / chunk_tpr(head_dim);
+  return (size_t)((g + 2) * head_dim + waves * (g * head_dim + 3 * g) + groups * kGqaRows * g) * sizeof(float);
 }
 
 // Merge of the nsplit range records of each head (one workgroup per head), in
@@ -610,6 +655,58 @@ __global__ __launch_bounds__(kAttnThreads) void decode_attention_merge_kernel(co
   }
 }
 
+// The same for more than kWideMerge ranges, where walking them one after another
+// is what takes the time: thread t adds dimensions 4 (t % DL) .. + 3 of the ranges
+// r = t / DL, + RG, ... (their loads in flight together), and the RG sums are added
+// in order (64 ranges, 32 heads, hd 128: the call 15.4 -> 12.5 us; at 8 ranges the
+// walk is 0.7 us the faster).
+__global__ __launch_bounds__(kAttnThreads) void decode_attention_merge_wide_kernel(const float* __restrict__ part,
+                                                                              int nsplit, int head_dim,
+                                                                              float* __restrict__ out) {
+  __shared__ float fac[kMaxSplits];
+  __shared__ float inv;
+  __shared__ __attribute__((aligned(16))) float sums[kAttnThreads * 4];
+  const int hq = (int)blockIdx.x, tid = (int)threadIdx.x;
+  const int rstride = kAttnRec + head_dim, dl = head_dim / 4;  // head_dim % 4 == 0
+  const int ngrp = kAttnThreads / dl, d = tid % dl, grp = tid / dl;
+  const float* hrec = part + (int64_t)hq * nsplit * rstride;
+  constexpr int U = 8;
+  f32x4 x[U];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int r = min(grp + u * ngrp, nsplit - 1);
+    x[u] = *reinterpret_cast<const f32x4*>(hrec + (int64_t)r * rstride + kAttnRec + 4 * d);
+  }
+  if (tid < 64) {
+    const float rm = tid < nsplit ? hrec[(int64_t)tid * rstride] : -INFINITY;
+    const float rl = tid < nsplit ? hrec[(int64_t)tid * rstride + 1] : 0.0f;
+    float gm = rm;
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) gm = fmaxf(gm, __shfl_xor(gm, off, 64));
+    const float fr = rm == -INFINITY ? 0.0f : expf(rm - gm);
+    fac[tid] = fr;
+    const float gs = wave_sum(tid < nsplit ? fr * rl : 0.0f);
+    if (tid == 0) inv = 1.0f / gs;
+  }
+  __syncthreads();
+  f32x4 a = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (grp < ngrp) {
+#pragma unroll
+    for (int u = 0; u < U; u++)
+      if (grp + u * ngrp < nsplit) a += fac[grp + u * ngrp] * x[u];
+    for (int r = grp + U * ngrp; r < nsplit; r += ngrp)
+      a += fac[r] * *reinterpret_cast<const f32x4*>(hrec + (int64_t)r * rstride + kAttnRec + 4 * d);
+    *reinterpret_cast<f32x4*>(&sums[4 * tid]) = a;
+  }
+  __syncthreads();
+  if (tid < dl) {
+    for (int g = 1; g < ngrp; g++) a += *reinterpret_cast<const f32x4*>(&sums[4 * (g * dl + tid)]);
+    float* o = out + hq * head_dim + 4 * tid;
+#pragma unroll
+    for (int e = 0; e < 4; e++) o[e] = a[e] * inv;
+  }
+}
+
 size_t decode_attention_lds(int64_t pos, int64_t head_dim) {
   if (chunk_tpr(head_dim)) return (size_t)(3 + kAttnThreads / 64) * kMaxDims * sizeof(float);
   return (size_t)(3 * head_dim + pos + 1 + 8) * sizeof(float);
@@ -628,22 +725,28 @@ constexpr int kAttnThreads1 = 512;  // threads of the single-range workgroup
 }  // namespace
 
 AttnSplit plan_decode_attention(int64_t pos, int64_t n_q, int64_t n_kv, int64_t head_dim, int cu_count) {
-  AttnSplit p{1, (int)pos, kAttnThreads1, 2, 1, 0};
+  AttnSplit p{1, (int)pos, kAttnThreads1, 2, 0, 0};
   if (!chunk_tpr(head_dim)) return p;
-  // grouped-query heads (4 or 8 per KV head) on long caches: one workgroup
-  // per KV head serves its G query heads, about two workgroups per CU.
-  // Measured (hd 128, 256 CUs): 32 heads over 8, 2048 / 4096 rows 18.0 / 27.2
-  // -> 15.6 / 19.5 us; 64 over 8, 4096 / 16384 rows 46.0 / 158 -> 27.8 / 64.2;
-  // 32 over 4, 8192 rows 45.9 -> 35.9. Shorter caches and pairs of heads stay
-  // with a workgroup per query head (1024 rows: 10.6 against 14.4; 16 over 8,
-  // 2048 rows: 11.0 against 12.7).
+  // 1, 2, 4 or 8 query heads per KV head on long caches: one workgroup per KV
+  // head and range serves the G query heads, about one workgroup per CU. The line
+  // is n_q head_dim pos = 4 Mi (8 heads: 6 Mi), where the two cross; below it the
+  // launches bound and a workgroup per query head has more of them in flight.
+  // Measured (us a call in a graph, heads / KV heads / hd, rows; this kernel
+  // against the one it replaces there):
+  //   32/8/128   734 11.1 / 9.4   1024 9.7 / 10.6   4096 12.5 / 20.3  16383 27.5 / 41.9
+  //   64/8/128   734 14.7 / 15.6  1024 12.8 / 18.0  4096 16.5 / 28.8  16383 33.4 / 64.0
+  //   16/2/128  2048 12.9 / 11.0  4096 13.4 / 25.0  16383 21.8 / 56.3
+  //   16/16/128 1024  8.0 / 8.0   2048 10.0 / 11.4  4096 16.7 / 19.2  16383 44.9 / 48.3
+  //   32/16/64  1024  8.8 / 7.7   2048  9.0 / 10.7  4096 10.7 / 18.0  16383 25.7 / 47.2
+  // (two workgroups per CU: 64/8/128 4096 22.7, 16383 42.0.)
   const int64_t g = n_q / n_kv;
-  const bool gqa = (g == 4 || g == 8) && g * head_dim <= 1024 && pos >= 2048;
+  const bool gqa = (g == 1 || g == 2 || g == 4 || g == 8) && g * head_dim <= 1024 &&
+                   n_q * head_dim * pos >= (int64_t)(g == 8 ? 6 : 4) << 20;
   if (gqa) p.group = (int)g;
-  const int64_t want = gqa ? (2 * (int64_t)std::max(cu_count, 1) + n_kv - 1) / n_kv
-                           : ((int64_t)std::max(cu_count, 1) + n_q - 1) / n_q;
+  const int64_t want = ((int64_t)std::max(cu_count, 1) + (gqa ? n_kv : n_q) - 1) / (gqa ? n_kv : n_q);
   const int64_t ns = std::min<int64_t>({want, pos / kMinSplitRows, (int64_t)kMaxSplits});
-  if (ns < 4) {
+  if (gqa && ns < 2) return p;
+  if (!gqa && ns < 4) {
     // one range per head: beyond two chunks of 2 rows per lane, 8 rows per
     // lane keep more of the cache in flight (16 heads, hd 128, graph
     // replays: 128 rows 6.9 -> 6.2 us, 255 rows 9.3 -> 8.1; at two chunks
@@ -662,6 +765,13 @@ AttnSplit plan_decode_attention(int64_t pos, int64_t n_q, int64_t n_kv, int64_t 
 
 namespace {
 
+constexpr int kWideMerge = 16;
+
+void launch_merge(const float* part, int ns, int64_t n_q, int64_t head_dim, float* out, hipStream_t stream) {
+  hipLaunchKernelGGL(ns > kWideMerge ? decode_attention_merge_wide_kernel : decode_attention_merge_kernel,
+                     dim3((unsigned)n_q), dim3(kAttnThreads), 0, stream, part, ns, (int)head_dim, out);
+}
+
 template <int TPR, int NV, int NP, int THREADS>
 hipError_t launch_chunk(const float* q, const float* k, const float* v, float* kcache, float* vcache, int64_t pos,
                         int64_t n_q, int64_t n_kv, int64_t head_dim, double theta, double scale, float* out,
@@ -672,8 +782,7 @@ hipError_t launch_chunk(const float* q, const float* k, const float* v, float* k
                      theta, (float)scale, out, ns, sp.rps, part);
   if (hipError_t e = hipGetLastError()) return e;
   if (ns > 1)
-    hipLaunchKernelGGL(decode_attention_merge_kernel, dim3((unsigned)n_q), dim3(kAttnThreads), 0, stream, part, ns,
-                       (int)head_dim, out);
+    launch_merge(part, ns, n_q, head_dim, out, stream);
   return hipGetLastError();
 }
 
@@ -705,8 +814,7 @@ hipError_t launch_gqa(const float* q, const float* k, const float* v, float* kca
                      (int)n_q, (int)n_kv, (int)head_dim, theta, (float)scale, out, ns, sp.rps, part);
   if (hipError_t e = hipGetLastError()) return e;
   if (ns > 1)
-    hipLaunchKernelGGL(decode_attention_merge_kernel, dim3((unsigned)n_q), dim3(kAttnThreads), 0, stream, part, ns,
-                       (int)head_dim, out);
+    launch_merge(part, ns, n_q, head_dim, out, stream);
   return hipGetLastError();
 }
 
@@ -715,6 +823,7 @@ hipError_t launch_gqa_g(const float* q, const float* k, const float* v, float* k
                         int64_t n_q, int64_t n_kv, int64_t head_dim, double theta, double scale, float* out,
                         const AttnSplit& sp, float* part, hipStream_t stream) {
 #define RQ_GQA_ARGS q, k, v, kcache, vcache, pos, n_q, n_kv, head_dim, theta, scale, out, sp, part, stream
+  if (sp.group == 1) return launch_gqa<TPR, NV, 1>(RQ_GQA_ARGS);
   if (sp.group == 2) return launch_gqa<TPR, NV, 2>(RQ_GQA_ARGS);
   if (sp.group == 4) return launch_gqa<TPR, NV, 4>(RQ_GQA_ARGS);
   return launch_gqa<TPR, NV, 8>(RQ_GQA_ARGS);
@@ -728,7 +837,7 @@ hipError_t launch_decode_attention(const float* q, const float* k, const float* 
                                    double scale, float* out, const AttnSplit& sp, void* scratch, hipStream_t stream) {
   float* part = static_cast<float*>(scratch);
 #define RQ_ATTN_ARGS q, k, v, kcache, vcache, pos, n_q, n_kv, head_dim, theta, scale, out, sp, part, stream
-  if (sp.group > 1) {
+  if (sp.group > 0) {
     switch (chunk_tpr(head_dim)) {
       case 16:
         return launch_gqa_g<16, 1>(RQ_ATTN_ARGS);
