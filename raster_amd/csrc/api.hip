@@ -6,7 +6,7 @@
 // thread-local string (rq_last_error).
 #include <algorithm>
 #include <atomic>
-#include <cmath>
+#include <cstring>
 #include <mutex>
 #include <new>
 #include <string>
@@ -655,6 +655,17 @@ static int make_weight_k(Ctx* c, int format, int64_t out, int64_t in, const void
   return RQ_OK;
 }
 
+// Branch-free, so that the scan runs at memory speed
+static bool all_finite(const float* v, int64_t n) {
+  uint32_t bad = 0;
+  for (int64_t i = 0; i < n; i++) {
+    uint32_t u;
+    std::memcpy(&u, v + i, 4);
+    bad |= (uint32_t)((u & 0x7F800000u) == 0x7F800000u);
+  }
+  return bad == 0;
+}
+
 static int check_shape_k(int format, int64_t out, int64_t in) {
   if (int s = check_shape(out, in)) return s;
   if (in % 256 != 0) return fail(RQ_ERR_SHAPE, "K-quants need in % 256 == 0 (super-blocks of 256)");
@@ -674,19 +685,19 @@ int rq_weight_create_q4k(rq_ctx h, const uint8_t* wq, const float* da, const flo
   if (int s = check_shape_k(RQ_Q4_K, out, in)) return s;
   const int64_t nsb = out * (in / 256), nsub = out * (in / 32);
   std::vector<float> sup((size_t)(2 * nsb));
-  // the GEMM (kquant_gemm.hip) needs 6-bit aq, and folds aq into integers, where
-  // an infinite da would not meet a zero aq as it does in the GEMV
-  bool gemm = true;
   for (int64_t i = 0; i < nsb; i++) {
     sup[(size_t)(2 * i)] = da[i];
     sup[(size_t)(2 * i + 1)] = db[i];
-    gemm = gemm && std::isfinite(da[i]) && std::isfinite(db[i]);
   }
   std::vector<uint16_t> sub((size_t)nsub);
+  // the GEMM (kquant_gemm.hip) needs 6-bit aq, and folds aq into integers, where
+  // an infinite da would not meet a zero aq as it does in the GEMV
+  uint8_t any = 0;
   for (int64_t i = 0; i < nsub; i++) {
-    gemm = gemm && aq[i] <= 63;
+    any |= aq[i];
     sub[(size_t)i] = (uint16_t)(aq[i] | ((uint16_t)(uint8_t)bq[i] << 8));
   }
+  const bool gemm = any <= 63 && all_finite(sup.data(), 2 * nsb);
   return make_weight_k(c, RQ_Q4_K, out, in, wq, (size_t)(out * in / 2), sup.data(), sup.size() * 4, sub.data(),
                        sub.size() * 2, gemm, w);
 }
@@ -718,7 +729,7 @@ int rq_weight_create_q6k(rq_ctx h, const uint8_t* wq, const int8_t* sc, const fl
   if (bad & 0xC0) return fail(RQ_ERR_SHAPE, "Q6_K codes must lie in 0..63");
   return make_weight_k(c, RQ_Q6_K, out, in, packed.data(), packed.size(), ds, (size_t)(out * (in / 256)) * 4, sc,
                        (size_t)(out * (in / 16)),
-                       std::all_of(ds, ds + out * (in / 256), [](float d) { return std::isfinite(d); }), w);
+                       all_finite(ds, out * (in / 256)), w);
 }
 
 int rq_weight_info(rq_weight h, int* format, int64_t* out, int64_t* in, int* scale_dtype, size_t* bytes) {
