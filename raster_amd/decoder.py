@@ -31,10 +31,12 @@ A whole step can be captured in one HIP graph (no call allocates).
 from __future__ import annotations
 
 import math
+from ctypes import byref
 
 import numpy as np
 
-from .quant import Context, QWeight, decode_attention
+from ._lib import RQ_F32, FusedOps, call
+from .quant import Context, QWeight, _current_stream, _need, _t
 
 
 def rms_norm(torch, x, weight, eps: float, gain_offset: float = 0.0):
@@ -120,16 +122,10 @@ class DecoderLayer:
         """x: f32 [d] on the device; kcache / vcache: f32 [>= pos+1, n_kv*head_dim].
         Appends this token's k / v at `pos`, attends positions 0..pos and
         returns the layer output [d]."""
-        import torch
-
-        qd, kvd = self.n_q * self.hd, self.n_kv * self.hd
         if self.fused:
-            qkv = self.w_qkv.matmul_fused(x.view(1, -1), norm_gain=self.g1, norm_eps=self.eps).view(-1)
-            at = decode_attention(self.ctx, qkv[:qd], qkv[qd:qd + kvd], qkv[qd + kvd:], kcache, vcache, pos,
-                                  self.n_q, self.n_kv, self.hd, self.theta, 1.0 / math.sqrt(self.hd))
-            x1 = self.w_o.matmul_fused(at.view(1, -1), residual=x.view(1, -1))
-            h = self.w_gu.matmul_fused(x1, norm_gain=self.g2, norm_eps=self.eps, swiglu=True)
-            return self.w_d.matmul_fused(h, residual=x1).view(-1)
+            return self._step_fused(x, kcache, vcache, pos)
+        torch = _t()
+        qd, kvd = self.n_q * self.hd, self.n_kv * self.hd
         if pos not in self._rope:
             self._rope[pos] = rope_tables(torch, self.hd, self.theta, pos, x.device)
         cos, sin = self._rope[pos]
@@ -144,6 +140,41 @@ class DecoderLayer:
         gu = self.w_gu.matmul(rms_norm(torch, x1, self.g2, self.eps).view(1, -1)).view(-1)
         h = silu_mul(torch, gu[:self.ffn], gu[self.ffn:])
         return residual_add(x1, self.w_d.matmul(h.view(1, -1)).view(-1))
+
+    def _step_fused(self, x, kcache, vcache, pos: int):
+        """The five fused calls on raw pointers into one workspace of this step
+        (matmul_fused and decode_attention on tensors would allocate five and
+        cut seven views: about half of the step's host time, which is longer
+        than its kernels')."""
+        torch = _t()
+        d, qd, kvd = self.d, self.n_q * self.hd, self.n_kv * self.hd
+        for t, n in ((x, d), (self.g1, d), (self.g2, d)):
+            _need(t.is_cuda and t.is_contiguous() and t.dtype == torch.float32 and t.numel() == n,
+                  f"x and the norm gains must be contiguous f32 CUDA tensors of {n} elements")
+        for t in (kcache, vcache):
+            _need(t.is_cuda and t.is_contiguous() and t.dtype == torch.float32 and t.numel() >= (pos + 1) * kvd,
+                  "kcache / vcache must be contiguous f32 CUDA tensors of at least pos+1 rows")
+        # qkv | attention | x1 | h, each on a 16-byte boundary
+        sizes = [(n + 3) & ~3 for n in (qd + 2 * kvd, qd, d, self.ffn)]
+        work = torch.empty(sum(sizes), dtype=torch.float32, device=x.device)
+        out = torch.empty(d, dtype=torch.float32, device=x.device)
+        qkv = work.data_ptr()
+        at = qkv + 4 * sizes[0]
+        x1 = at + 4 * sizes[1]
+        h = x1 + 4 * sizes[2]
+        stream, ctx, x0 = _current_stream(x), self.ctx.handle, x.data_ptr()
+
+        def linear(w, src, dst, gain=None, residual=None, swiglu=0):
+            ops = FusedOps(gain, self.eps if gain else 0.0, residual, swiglu, 0)
+            call("rq_qmatmul_fused", ctx, w.handle, src, RQ_F32, dst, RQ_F32, 1, byref(ops), stream)
+
+        linear(self.w_qkv, x0, qkv, gain=self.g1.data_ptr())
+        call("rq_decode_attention", ctx, qkv, qkv + 4 * qd, qkv + 4 * (qd + kvd), kcache.data_ptr(), vcache.data_ptr(),
+             pos, self.n_q, self.n_kv, self.hd, float(self.theta), 1.0 / math.sqrt(self.hd), at, stream)
+        linear(self.w_o, at, x1, residual=x0)
+        linear(self.w_gu, x1, h, gain=self.g2.data_ptr(), swiglu=1)
+        linear(self.w_d, h, out.data_ptr(), residual=x1)
+        return out
 
     def matmul_bytes(self) -> int:
         """Algorithmic weight bytes the step streams (codes + f32 scales)."""

@@ -90,6 +90,26 @@ def context(device: int = 0) -> Context:
         return c
 
 
+_torch = None  # torch, once a device call has needed it (host arrays alone do not)
+_dtypes: dict = {}
+
+
+def _t():
+    global _torch
+    if _torch is None:
+        import torch
+
+        _dtypes[torch.float32], _dtypes[torch.bfloat16] = RQ_F32, RQ_BF16
+        _torch = torch
+    return _torch
+
+
+def _current_stream(t) -> int:
+    """The raw current stream of a CUDA tensor's device (building a
+    torch.cuda.Stream object for it takes 1.9 us of a call's 9, this 0.1)."""
+    return _torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
 def _stream_ptr(stream):
     if stream is None:
         return None
@@ -99,13 +119,29 @@ def _stream_ptr(stream):
 
 
 def _dtype_code(t) -> int:
-    import torch
+    code = _dtypes.get(t.dtype)
+    if code is None:
+        raise TypeError(f"activations/outputs must be float32 or bfloat16, got {t.dtype}")
+    return code
 
-    if t.dtype == torch.float32:
-        return RQ_F32
-    if t.dtype == torch.bfloat16:
-        return RQ_BF16
-    raise TypeError(f"activations/outputs must be float32 or bfloat16, got {t.dtype}")
+
+def _cuda_rows(x, in_: int, msg: str = "x") -> int:
+    """Rows of `in_` elements in a contiguous CUDA tensor."""
+    if not (x.is_cuda and x.is_contiguous()):
+        raise ValueError(f"{msg} must be a contiguous CUDA tensor")
+    n = x.numel()
+    if n % in_:
+        raise ValueError(f"{msg}.numel() must be a multiple of in")
+    return n // in_
+
+
+def _out_rows(y, x, m: int, n: int, dtype, msg: str):
+    """A caller's y checked, or a new [m, n] one on x's device."""
+    if y is None:
+        return _torch.empty((m, n), dtype=dtype or _torch.float32, device=x.device)
+    if not (y.is_cuda and y.is_contiguous() and y.numel() == m * n):
+        raise ValueError(msg)
+    return y
 
 
 class QWeight:
@@ -199,18 +235,11 @@ class QWeight:
         """y[m, out] = x[m, in] . dequant(W)^T on the device (x: torch f32/bf16 CUDA tensor).
         K-quant weights (Q4_K, Q6_K) take f32 x, quantized to q8_K inside the
         call: the same bits as quantize_act_q8k + matmul_q8k."""
-        import torch
-
-        _need(x.is_cuda and x.is_contiguous(), "x must be a contiguous CUDA tensor")
-        _need(x.numel() % self.in_ == 0, "x.numel() must be a multiple of in")
-        m = x.numel() // self.in_
-        if y is None:
-            y = torch.empty((m, self.out), dtype=out_dtype or torch.float32, device=x.device)
-        _need(y.is_cuda and y.is_contiguous() and y.numel() == m * self.out, "y must be a contiguous [m, out] CUDA tensor")
-        if stream is None:
-            stream = torch.cuda.current_stream(x.device)
-        call("rq_qmatmul", self.ctx.handle, self.handle, C.c_void_p(x.data_ptr()), _dtype_code(x),
-             C.c_void_p(y.data_ptr()), _dtype_code(y), m, _stream_ptr(stream))
+        _t()
+        m = _cuda_rows(x, self.in_)
+        y = _out_rows(y, x, m, self.out, out_dtype, "y must be a contiguous [m, out] CUDA tensor")
+        call("rq_qmatmul", self.ctx.handle, self.handle, x.data_ptr(), _dtype_code(x), y.data_ptr(), _dtype_code(y), m,
+             _current_stream(x) if stream is None else _stream_ptr(stream))
         return y
 
     def matmul_fused(self, x, y=None, out_dtype=None, norm_gain=None, norm_eps: float = 0.0, residual=None,
@@ -220,15 +249,10 @@ class QWeight:
         of row pairs (rows 2i / 2i+1 = gate / up; y is [m, out/2]) or a
         residual add (residual [m, out], y's dtype) after it. act_i8 quantizes
         the activations to Raster's int8 blocks in the kernel."""
-        import torch
-
-        _need(x.is_cuda and x.is_contiguous(), "x must be a contiguous CUDA tensor")
-        _need(x.numel() % self.in_ == 0, "x.numel() must be a multiple of in")
-        m = x.numel() // self.in_
+        torch = _t()
+        m = _cuda_rows(x, self.in_)
         ny = self.out // 2 if swiglu else self.out
-        if y is None:
-            y = torch.empty((m, ny), dtype=out_dtype or torch.float32, device=x.device)
-        _need(y.is_cuda and y.is_contiguous() and y.numel() == m * ny, "y must be a contiguous CUDA tensor of m rows")
+        y = _out_rows(y, x, m, ny, out_dtype, "y must be a contiguous CUDA tensor of m rows")
         ops = _lib.FusedOps(None, float(norm_eps), None, 1 if swiglu else 0, 1 if act_i8 else 0)
         if norm_gain is not None:
             _need(norm_gain.is_cuda and norm_gain.dtype == torch.float32 and norm_gain.is_contiguous()
@@ -238,18 +262,15 @@ class QWeight:
             _need(residual.is_cuda and residual.is_contiguous() and residual.dtype == y.dtype
                   and residual.numel() == m * ny, "residual must match y")
             ops.residual = residual.data_ptr()
-        if stream is None:
-            stream = torch.cuda.current_stream(x.device)
-        call("rq_qmatmul_fused", self.ctx.handle, self.handle, C.c_void_p(x.data_ptr()), _dtype_code(x),
-             C.c_void_p(y.data_ptr()), _dtype_code(y), m, C.byref(ops), _stream_ptr(stream))
+        call("rq_qmatmul_fused", self.ctx.handle, self.handle, x.data_ptr(), _dtype_code(x), y.data_ptr(),
+             _dtype_code(y), m, C.byref(ops), _current_stream(x) if stream is None else _stream_ptr(stream))
         return y
 
     def matmul_i8(self, xq, xs, xsum=None, y=None, out_dtype=None, stream=None):
         """rq_qmatmul_i8: y[m, out] from int8 activations (xq int8 [m, in],
         xs f32 [m, in/32], xsum int32 [m, in/32], needed for Q4_0), as
         produced by quantize_act_i8."""
-        import torch
-
+        torch = _t()
         _need(xq.is_cuda and xq.is_contiguous() and xq.dtype == torch.int8, "xq must be a contiguous int8 CUDA tensor")
         _need(xq.numel() % self.in_ == 0, "xq.numel() must be a multiple of in")
         m = xq.numel() // self.in_
@@ -261,18 +282,15 @@ class QWeight:
         if y is None:
             y = torch.empty((m, self.out), dtype=out_dtype or torch.float32, device=xq.device)
         _need(y.is_cuda and y.is_contiguous() and y.numel() == m * self.out, "y must be a contiguous [m, out] CUDA tensor")
-        if stream is None:
-            stream = torch.cuda.current_stream(xq.device)
-        call("rq_qmatmul_i8", self.ctx.handle, self.handle, C.c_void_p(xq.data_ptr()), C.c_void_p(xs.data_ptr()),
-             C.c_void_p(xsum.data_ptr() if xsum is not None else None), C.c_void_p(y.data_ptr()), _dtype_code(y), m,
-             _stream_ptr(stream))
+        stream = _current_stream(xq) if stream is None else _stream_ptr(stream)
+        call("rq_qmatmul_i8", self.ctx.handle, self.handle, xq.data_ptr(), xs.data_ptr(),
+             xsum.data_ptr() if xsum is not None else None, y.data_ptr(), _dtype_code(y), m, stream)
         return y
 
     def matmul_q8k(self, xq, xs, bsums, y=None, out_dtype=None, stream=None):
         """rq_qmatmul_q8k: y[m, out] for a K-quant weight from q8_K activations
         (xq int8 [m, in], xs f32 [m, in/256], bsums int32 [m, in/sub])."""
-        import torch
-
+        torch = _t()
         _need(self.format in (_lib.RQ_Q4_K, _lib.RQ_Q6_K), "matmul_q8k needs a Q4_K or Q6_K weight")
         sub = 32 if self.format == _lib.RQ_Q4_K else 16
         _need(xq.is_cuda and xq.is_contiguous() and xq.dtype == torch.int8 and xq.numel() % self.in_ == 0,
@@ -285,16 +303,14 @@ class QWeight:
         if y is None:
             y = torch.empty((m, self.out), dtype=out_dtype or torch.float32, device=xq.device)
         _need(y.is_cuda and y.is_contiguous() and y.numel() == m * self.out, "y must be a contiguous [m, out] CUDA tensor")
-        if stream is None:
-            stream = torch.cuda.current_stream(xq.device)
-        call("rq_qmatmul_q8k", self.ctx.handle, self.handle, C.c_void_p(xq.data_ptr()), C.c_void_p(xs.data_ptr()),
-             C.c_void_p(bsums.data_ptr()), C.c_void_p(y.data_ptr()), _dtype_code(y), m, _stream_ptr(stream))
+        stream = _current_stream(xq) if stream is None else _stream_ptr(stream)
+        call("rq_qmatmul_q8k", self.ctx.handle, self.handle, xq.data_ptr(), xs.data_ptr(),
+             bsums.data_ptr(), y.data_ptr(), _dtype_code(y), m, stream)
         return y
 
     def matmul_dx(self, dy, dx=None, stream=None):
         """rq_qmatmul_dx (qlinear-q8-dx): dx[m, in] = dy[m, out] . dequant(W), f32."""
-        import torch
-
+        torch = _t()
         _need(dy.is_cuda and dy.is_contiguous() and dy.dtype == torch.float32 and dy.numel() % self.out == 0,
               "dy must be a contiguous f32 CUDA tensor of m*out elements")
         m = dy.numel() // self.out
@@ -302,20 +318,16 @@ class QWeight:
             dx = torch.empty((m, self.in_), dtype=torch.float32, device=dy.device)
         _need(dx.is_cuda and dx.is_contiguous() and dx.dtype == torch.float32 and dx.numel() == m * self.in_,
               "dx must be a contiguous f32 [m, in] CUDA tensor")
-        if stream is None:
-            stream = torch.cuda.current_stream(dy.device)
-        call("rq_qmatmul_dx", self.ctx.handle, self.handle, C.c_void_p(dy.data_ptr()), C.c_void_p(dx.data_ptr()), m,
-             _stream_ptr(stream))
+        stream = _current_stream(dy) if stream is None else _stream_ptr(stream)
+        call("rq_qmatmul_dx", self.ctx.handle, self.handle, dy.data_ptr(), dx.data_ptr(), m, stream)
         return dx
 
     def dequant(self, stream=None):
         """Dequantized f32 W[out, in] computed on the device."""
-        import torch
-
+        torch = _t()
         w = torch.empty((self.out, self.in_), dtype=torch.float32, device=f"cuda:{self.ctx.device}")
-        if stream is None:
-            stream = torch.cuda.current_stream(w.device)
-        call("rq_dequant", self.ctx.handle, self.handle, C.c_void_p(w.data_ptr()), _stream_ptr(stream))
+        stream = _current_stream(w) if stream is None else _stream_ptr(stream)
+        call("rq_dequant", self.ctx.handle, self.handle, w.data_ptr(), stream)
         return w
 
     def device_ptrs(self):
@@ -333,8 +345,7 @@ def quantize_act_i8(ctx: Context, x, in_: int, out=None, stream=None):
     """rq_quantize_act_i8 (quantize-act-i8): x f32 [m*in] on the device ->
     (xq int8 [m, in], xs f32 [m, in/32], xsum int32 [m, in/32]), written into
     `out` when given."""
-    import torch
-
+    torch = _t()
     _need(x.is_cuda and x.is_contiguous() and x.dtype == torch.float32, "x must be a contiguous f32 CUDA tensor")
     _need(in_ % 32 == 0 and x.numel() % in_ == 0, "x.numel() must be a multiple of in, in a multiple of 32")
     m = x.numel() // in_
@@ -347,10 +358,9 @@ def quantize_act_i8(ctx: Context, x, in_: int, out=None, stream=None):
         _need(xq.numel() == m * in_ and xs.numel() == m * (in_ // 32) and xsum.numel() == xs.numel()
               and xq.dtype == torch.int8 and xs.dtype == torch.float32 and xsum.dtype == torch.int32
               and all(t.is_cuda and t.is_contiguous() for t in (xq, xs, xsum)), "out tensors do not match x")
-    if stream is None:
-        stream = torch.cuda.current_stream(x.device)
-    call("rq_quantize_act_i8", ctx.handle, C.c_void_p(x.data_ptr()), m, in_, C.c_void_p(xq.data_ptr()),
-         C.c_void_p(xs.data_ptr()), C.c_void_p(xsum.data_ptr()), _stream_ptr(stream))
+    stream = _current_stream(x) if stream is None else _stream_ptr(stream)
+    call("rq_quantize_act_i8", ctx.handle, x.data_ptr(), m, in_, xq.data_ptr(),
+         xs.data_ptr(), xsum.data_ptr(), stream)
     return xq, xs, xsum
 
 
@@ -358,8 +368,7 @@ def quantize_act_q8k(ctx: Context, x, in_: int, sub: int, out=None, stream=None)
     """rq_quantize_act_q8k (quantize-act-q8k): x f32 [m*in] on the device ->
     (xq int8 [m, in], xs f32 [m, in/256], bsums int32 [m, in/sub]); sub 32 for
     Q4_K, 16 for Q6_K."""
-    import torch
-
+    torch = _t()
     _need(x.is_cuda and x.is_contiguous() and x.dtype == torch.float32, "x must be a contiguous f32 CUDA tensor")
     _need(in_ % 256 == 0 and x.numel() % in_ == 0 and sub in (16, 32), "in % 256 == 0, sub 16 or 32")
     m = x.numel() // in_
@@ -368,10 +377,9 @@ def quantize_act_q8k(ctx: Context, x, in_: int, sub: int, out=None, stream=None)
                torch.empty((m, in_ // 256), dtype=torch.float32, device=x.device),
                torch.empty((m, in_ // sub), dtype=torch.int32, device=x.device))
     xq, xs, bsums = out
-    if stream is None:
-        stream = torch.cuda.current_stream(x.device)
-    call("rq_quantize_act_q8k", ctx.handle, C.c_void_p(x.data_ptr()), m, in_, sub, C.c_void_p(xq.data_ptr()),
-         C.c_void_p(xs.data_ptr()), C.c_void_p(bsums.data_ptr()), _stream_ptr(stream))
+    stream = _current_stream(x) if stream is None else _stream_ptr(stream)
+    call("rq_quantize_act_q8k", ctx.handle, x.data_ptr(), m, in_, sub, xq.data_ptr(),
+         xs.data_ptr(), bsums.data_ptr(), stream)
     return xq, xs, bsums
 
 
@@ -379,18 +387,16 @@ def i8gemv_dp4a(ctx: Context, wp, xp, kw: int, out: int, y=None, stream=None):
     """rq_i8gemv_dp4a (i8gemv-dp4a!, raster/quant/kernels_k.clj:141-150):
     y[o] = (float) sum_w dp4a(wp[o*kw + w], xp[w]); wp int32 [out*kw], xp int32
     [kw] CUDA tensors (four little-endian int8 lanes per word) -> y f32 [out]."""
-    import torch
-
+    torch = _t()
     _need(wp.is_cuda and xp.is_cuda and wp.dtype == torch.int32 and xp.dtype == torch.int32,
           "wp and xp must be int32 CUDA tensors")
     _need(wp.is_contiguous() and xp.is_contiguous() and wp.numel() == out * kw and xp.numel() == kw,
           "wp must hold out*kw words and xp kw words, contiguous")
     if y is None:
         y = torch.empty(out, dtype=torch.float32, device=wp.device)
-    if stream is None:
-        stream = torch.cuda.current_stream(wp.device)
-    call("rq_i8gemv_dp4a", ctx.handle, C.c_void_p(wp.data_ptr()), C.c_void_p(xp.data_ptr()),
-         C.c_void_p(y.data_ptr()), kw, out, _stream_ptr(stream))
+    stream = _current_stream(wp) if stream is None else _stream_ptr(stream)
+    call("rq_i8gemv_dp4a", ctx.handle, wp.data_ptr(), xp.data_ptr(),
+         y.data_ptr(), kw, out, stream)
     return y
 
 
@@ -400,8 +406,7 @@ def decode_attention(ctx: Context, q, k, v, kcache, vcache, pos: int, n_q: int, 
     `pos`, append of the rotated k and of v to row pos of kcache / vcache
     ([rows, n_kv*head_dim] f32), and single-query attention over rows 0..pos.
     Returns out [n_q*head_dim] f32."""
-    import torch
-
+    torch = _t()
     kvd = n_kv * head_dim
     for t, n in ((q, n_q * head_dim), (k, kvd), (v, kvd)):
         _need(t.is_cuda and t.is_contiguous() and t.dtype == torch.float32 and t.numel() == n,
@@ -413,11 +418,9 @@ def decode_attention(ctx: Context, q, k, v, kcache, vcache, pos: int, n_q: int, 
         out = torch.empty(n_q * head_dim, dtype=torch.float32, device=q.device)
     _need(out.is_cuda and out.is_contiguous() and out.dtype == torch.float32 and out.numel() == n_q * head_dim,
           "out must be a contiguous f32 CUDA tensor of n_q*head_dim elements")
-    if stream is None:
-        stream = torch.cuda.current_stream(q.device)
-    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
-    call("rq_decode_attention", ctx.handle, ptr(q), ptr(k), ptr(v), ptr(kcache), ptr(vcache), pos, n_q, n_kv,
-         head_dim, float(theta), float(scale), ptr(out), _stream_ptr(stream))
+    stream = _current_stream(q) if stream is None else _stream_ptr(stream)
+    call("rq_decode_attention", ctx.handle, q.data_ptr(), k.data_ptr(), v.data_ptr(), kcache.data_ptr(),
+         vcache.data_ptr(), pos, n_q, n_kv, head_dim, float(theta), float(scale), out.data_ptr(), stream)
     return out
 
 
@@ -431,16 +434,14 @@ def nextpad(in_: int) -> int:
 def q8_quantize(ctx: Context, W, out: int, in_: int, stream=None):
     """raster.quant.train/q8-quantize on the device (rq_q8_quantize): W f32
     [out*in] CUDA tensor -> (codes int8 [out, in], scales f32 [out, in/32])."""
-    import torch
-
+    torch = _t()
     _need(W.is_cuda and W.is_contiguous() and W.dtype == torch.float32 and W.numel() == out * in_,
           "W must be a contiguous f32 CUDA tensor of out*in elements")
     codes = torch.empty((out, in_), dtype=torch.int8, device=W.device)
     scales = torch.empty((out, in_ // 32), dtype=torch.float32, device=W.device)
-    if stream is None:
-        stream = torch.cuda.current_stream(W.device)
-    call("rq_q8_quantize", ctx.handle, C.c_void_p(W.data_ptr()), out, in_, C.c_void_p(codes.data_ptr()),
-         C.c_void_p(scales.data_ptr()), _stream_ptr(stream))
+    stream = _current_stream(W) if stream is None else _stream_ptr(stream)
+    call("rq_q8_quantize", ctx.handle, W.data_ptr(), out, in_, codes.data_ptr(),
+         scales.data_ptr(), stream)
     return codes, scales
 
 
@@ -448,8 +449,7 @@ def q4k_of(ctx: Context, W, out: int, in_: int, stream=None):
     """raster.quant.pack/q4k-of on the device (rq_q4k_of): W f32 [out*in] CUDA
     tensor, rows zero-padded to inp = nextpad(in) -> dict(wq, da, db, aq, bq,
     in=inp, out=out) of CUDA tensors, the arrays QWeight.q4k takes."""
-    import torch
-
+    torch = _t()
     _need(W.is_cuda and W.is_contiguous() and W.dtype == torch.float32 and W.numel() == out * in_,
           "W must be a contiguous f32 CUDA tensor of out*in elements")
     inp = nextpad(in_)
@@ -459,29 +459,25 @@ def q4k_of(ctx: Context, W, out: int, in_: int, stream=None):
     da, db = torch.empty(n // 256, device=dev), torch.empty(n // 256, device=dev)
     aq, bq = torch.empty(n // 32, dtype=torch.uint8, device=dev), torch.empty(n // 32, dtype=torch.int8, device=dev)
     got = C.c_int64()
-    if stream is None:
-        stream = torch.cuda.current_stream(dev)
-    ptr = lambda t: C.c_void_p(t.data_ptr())  # noqa: E731
-    call("rq_q4k_of", ctx.handle, ptr(W), out, in_, ptr(wq), ptr(da), ptr(db), ptr(aq), ptr(bq), C.byref(got),
-         _stream_ptr(stream))
+    stream = _current_stream(W) if stream is None else _stream_ptr(stream)
+    call("rq_q4k_of", ctx.handle, W.data_ptr(), out, in_, wq.data_ptr(), da.data_ptr(), db.data_ptr(),
+         aq.data_ptr(), bq.data_ptr(), C.byref(got), stream)
     return {"wq": wq, "da": da, "db": db, "aq": aq, "bq": bq, "in": got.value, "out": out}
 
 
 def quantize_weight_q6k(ctx: Context, W, out: int, in_: int, stream=None):
     """quantize-weight-q6k on the device (rq_quantize_weight_q6k), in % 256 == 0:
     W f32 [out*in] CUDA tensor -> (wq u8 [out*in], sc i8 [out*in/16], ds f32 [out*in/256])."""
-    import torch
-
+    torch = _t()
     _need(W.is_cuda and W.is_contiguous() and W.dtype == torch.float32 and W.numel() == out * in_,
           "W must be a contiguous f32 CUDA tensor of out*in elements")
     dev = W.device
     wq = torch.empty(out * in_, dtype=torch.uint8, device=dev)
     sc = torch.empty(out * in_ // 16, dtype=torch.int8, device=dev)
     ds = torch.empty(out * in_ // 256, dtype=torch.float32, device=dev)
-    if stream is None:
-        stream = torch.cuda.current_stream(dev)
-    call("rq_quantize_weight_q6k", ctx.handle, C.c_void_p(W.data_ptr()), out, in_, C.c_void_p(wq.data_ptr()),
-         C.c_void_p(sc.data_ptr()), C.c_void_p(ds.data_ptr()), _stream_ptr(stream))
+    stream = _current_stream(W) if stream is None else _stream_ptr(stream)
+    call("rq_quantize_weight_q6k", ctx.handle, W.data_ptr(), out, in_, wq.data_ptr(),
+         sc.data_ptr(), ds.data_ptr(), stream)
     return wq, sc, ds
 
 
@@ -522,8 +518,7 @@ def dequant_q8_dense(codes, scales, in_: int, out: int, ctx: Context | None = No
     """raster.quant.train/dequant-q8-dense, decoded on the GPU: f32 W[out*in]."""
     w = QWeight.q8(codes, scales, out, in_, ctx)
     try:
-        import torch
-
+        torch = _t()
         return w.dequant().cpu().numpy().ravel()
     finally:
         w.destroy()
