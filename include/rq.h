@@ -169,7 +169,8 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    cost model's tile, 256 x 96 on the role-split kernel); f32 x: the
  *    exact-code f32 GEMM;
  *  - Q4_K / Q6_K weights (f32 x only, any m; bf16 x fails with RQ_ERR_DTYPE):
- *    x is quantized to q8_K in scratch and the K-quant matmul runs, the same
+ *    x is quantized to q8_K (in scratch, or inside the GEMV when m * in is at
+ *    most 12288) and the K-quant matmul runs, the same
  *    arithmetic as rq_quantize_act_q8k + rq_qmatmul_q8k and bit for bit their
  *    results (QMatrix apply of the built-in :q4_K / :q6_K formats,
  *    raster/quant/core.clj:55-75). m <= 4 is one GEMV pass over the

@@ -805,7 +805,9 @@ static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t 
 // A K-quant weight with f32 x in one call: x quantized to q8_K in scratch,
 // then the K-quant GEMV or GEMM -- rq_quantize_act_q8k + rq_qmatmul_q8k, with
 // the same arithmetic and so the same results (for the GEMM the quantizer
-// writes its operand order, in buffers of the same sizes) (QMatrix apply of the built-in :q4_K /
+// writes its operand order, in buffers of the same sizes; a short x of few rows
+// is quantized inside the GEMV, with the scratch asked for all the same, so that
+// what a call needs does not depend on the overlap of x and y) (QMatrix apply of the built-in :q4_K /
 // :q6_K formats, raster/quant/core.clj:55-75).
 static int run_kquant_matmul(Ctx* c, const Weight& w, const float* x, void* y, int y_dtype, int64_t m,
                              hipStream_t stream, FixedScratch* fixed) {
@@ -818,14 +820,16 @@ static int run_kquant_matmul(Ctx* c, const Weight& w, const float* x, void* y, i
   int8_t* xq = static_cast<int8_t*>(buf);
   float* xs = reinterpret_cast<float*>(static_cast<uint8_t*>(buf) + xq_b);
   int32_t* bs = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(buf) + xq_b + xs_b);
-  const bool gemm = kquant_gemm_takes(w, m);
-  hipError_t e = gemm ? launch_quantize_act_q8k_packed(x, m, w.in, sub, xq, xs, bs, stream)
-                      : launch_quantize_act_q8k(x, m, w.in, sub, xq, xs, bs, stream);
+  const bool gemm = kquant_gemm_takes(w, m), fused = !gemm && kquant_gemv_quantizes(w, x, y, y_dtype, m);
+  hipError_t e = fused  ? hipSuccess
+                 : gemm ? launch_quantize_act_q8k_packed(x, m, w.in, sub, xq, xs, bs, stream)
+                        : launch_quantize_act_q8k(x, m, w.in, sub, xq, xs, bs, stream);
   if (e != hipSuccess) return hip_fail(e, "quantizer launch");
   const EvSet ev = fixed ? EvSet{} : timing_set(c, stream);
   if (ev.n) (void)hipEventRecord(ev.e[0], stream);
-  e = gemm ? launch_kquant_gemm(w, xq, xs, bs, true, y, y_dtype, m, c->cu_count, stream)
-           : launch_kquant_gemv(w, xq, xs, bs, y, y_dtype, m, c->cu_count, stream);
+  e = fused  ? launch_kquant_gemv_f32(w, x, y, y_dtype, m, c->cu_count, stream)
+      : gemm ? launch_kquant_gemm(w, xq, xs, bs, true, y, y_dtype, m, c->cu_count, stream)
+             : launch_kquant_gemv(w, xq, xs, bs, y, y_dtype, m, c->cu_count, stream);
   if (ev.n && e == hipSuccess) (void)hipEventRecord(ev.e[1], stream);
   timing_done(c, ev, e == hipSuccess);
   if (e != hipSuccess) return hip_fail(e, "K-quant matmul launch");

@@ -25,7 +25,8 @@
 // and 6-bit codes are non-negative int8). The terms are added in f32 (Raster
 // adds in double). HBM-bound on the codes: a wave takes kKqRows rows at a time,
 // its lanes one sub-block each (16 code bytes, one load) strided by 64, the
-// activations of up to 4 rows staged in LDS once per workgroup.
+// activations of up to 4 rows staged in LDS once per workgroup; a short f32 x is
+// quantized there by the workgroup itself.
 #include <algorithm>
 #include <atomic>
 
@@ -36,6 +37,8 @@ namespace rq {
 namespace {
 
 constexpr int kKqThreads = 256;
+constexpr int kKqWaves = 16;        // most waves of a workgroup
+constexpr int kKqFusedMax = 12288;  // most elements of x quantized inside the GEMV (kquant_gemv_quantizes)
 // weight rows a wave takes at a time (14336 x 4096, m = 1, cold, rows 1 / 2 /
 // 4 / 8: Q4_K 12.1 / 10.3 / 11.3 / 12.7 us, Q6_K 15.7 / 12.5 / 13.8 / 14.4 us;
 // m = 4 likewise best at 2)
@@ -45,6 +48,39 @@ __device__ __forceinline__ float wave_sum64(float v) {
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
   return v;
+}
+
+// The largest of the wave's values, in every lane: quads and half rows by DPP,
+// then the rows by lane swaps.
+__device__ __forceinline__ float wave_max64(float v) {
+  v = max8(v);
+  v = fmaxf(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, false)));  // row_ror:8
+  const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(p[0]), __uint_as_float(p[1]));
+  const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+}
+
+// quantize-act-q8k of one super-block by one wave, four elements per lane: the
+// lane's codes as a word, d in every lane, and in the first lane of each SUB / 4
+// the sum of the sub-block's codes.
+template <int SUB>
+__device__ __forceinline__ uint32_t quantize_q8k(const f32x4& v, double& d, int& sum) {
+  const float a = wave_max64(fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+  d = (double)a / 127.0;
+  const double id = d == 0.0 ? 0.0 : 1.0 / d;
+  uint32_t word = 0u;
+  int s = 0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const int q = java_round_clamp127((double)v[i] * id);
+    word |= (uint32_t)(q & 0xFF) << (8 * i);
+    s += q;
+  }
+  s += dpp_xor1(s);
+  s += dpp_xor2(s);
+  sum = SUB == 32 ? s + dpp_half_mirror(s) : s;
+  return word;
 }
 
 }  // namespace
@@ -59,21 +95,9 @@ __global__ __launch_bounds__(kKqThreads) void quantize_act_q8k_kernel(const floa
   const int64_t sb = (int64_t)blockIdx.x * (kKqThreads / 64) + (threadIdx.x >> 6);
   const int64_t b = sb < nsb ? sb : nsb - 1;  // waves past the end reread the last one and store nothing
   const f32x4 v = *reinterpret_cast<const f32x4*>(x + b * 256 + lane * 4);
-  float a = fmaxf(fmaxf(fabsf(v[0]), fabsf(v[1])), fmaxf(fabsf(v[2]), fabsf(v[3])));
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) a = fmaxf(a, __shfl_xor(a, off, 64));
-  const double d = (double)a / 127.0;
-  const double id = d == 0.0 ? 0.0 : 1.0 / d;
-  uint32_t word = 0u;
-  int s = 0;
-#pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int q = java_round_clamp127((double)v[i] * id);
-    word |= (uint32_t)(q & 0xFF) << (8 * i);
-    s += q;
-  }
-#pragma unroll
-  for (int off = 1; off < SUB / 4; off <<= 1) s += __shfl_xor(s, off, 64);
+  double d;
+  int s;
+  const uint32_t word = quantize_q8k<SUB>(v, d, s);
   if (sb < nsb) {
     *reinterpret_cast<uint32_t*>(xq + b * 256 + lane * 4) = word;
     if (lane == 0) xs[b] = (float)d;
@@ -171,8 +195,10 @@ __device__ __forceinline__ u32x4 unpack_q6k(uint32_t p0, uint32_t p1, uint32_t p
 
 // ---- K-quant GEMV: y[t][o] for MT activation rows t. FMT RQ_Q4_K / RQ_Q6_K.
 // LDS: xq[MT][K] codes, bsums[MT][K/SUB], xs[MT][K/256].
-template <int FMT, int MT, int D>
-__global__ __launch_bounds__(kKqThreads) void kquant_gemv_kernel(
+// XF: x is given as f32 and quantized while it is staged (xq and bsums unused,
+// xs = x).
+template <int FMT, int MT, bool XF, int D>
+__global__ __launch_bounds__(64 * kKqWaves) void kquant_gemv_kernel(
     const uint8_t* __restrict__ wq, const void* __restrict__ sup, const void* __restrict__ subsc,
     const int8_t* __restrict__ xq, const float* __restrict__ xs, const int32_t* __restrict__ bsums,
     void* __restrict__ y, int M, int K, int N, int y_dtype) {
@@ -193,7 +219,8 @@ __global__ __launch_bounds__(kKqThreads) void kquant_gemv_kernel(
   // D = 1 measured best (14336 x 4096, m = 1: Q4_K 11.7 / 12.2 / 13.5 /
   // 15.5 us and Q6_K 16.9 / 17.4 / 18.9 / 19.0 us at D = 1 .. 4; before this
   // stream, loading each step only when it was computed: 15.0 and 16.3 us).
-  const int gw = (int)blockIdx.x * (kKqThreads / 64) + wave, nwaves = (int)gridDim.x * (kKqThreads / 64);
+  const int nthr = (int)blockDim.x;
+  const int gw = XF ? wave * (int)gridDim.x + (int)blockIdx.x : (int)blockIdx.x * (nthr / 64) + wave, nwaves = (int)gridDim.x * (nthr / 64);
   const int ngrp = (N + kKqRows - 1) / kKqRows;
   const int ng = gw < ngrp ? (ngrp - 1 - gw) / nwaves + 1 : 0;
   const int nit = (nsub + 63) / 64, nitp = (nit + D - 1) / D * D;
@@ -238,6 +265,23 @@ __global__ __launch_bounds__(kKqThreads) void kquant_gemv_kernel(
       ++gi;
     }
   };
+  // XF: the wave's super-blocks of x, wave, wave + waves, ... of the M rows; the
+  // first XJ go out before the weights, so that quantizing them waits for them
+  // only (loads complete in order)
+  constexpr int XJ = XF ? 2 : 1;
+  f32x4 xv[XJ];
+  const int nxb = M * nsb, xw = nthr / 64;
+  auto load_x = [&](int b0) {
+#pragma unroll
+    for (int j = 0; j < XJ; j++) {
+      const int b = min(b0 + j * xw, nxb - 1);
+      xv[j] = *reinterpret_cast<const f32x4*>(xs + (int64_t)b * 256 + lane * 4);
+    }
+  };
+  if (XF) {
+    load_x(wave);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   // the first weight loads go out before the activations are staged, so
   // their latency overlaps the staging (14336 x 4096, m = 1, cold: Q4_K
   // 11.65 -> 11.19 us; Q6_K unchanged at 16.9)
@@ -250,14 +294,37 @@ __global__ __launch_bounds__(kKqThreads) void kquant_gemv_kernel(
   }
 
   // stage the activations (rows past M as zeros)
-  for (int i = tid; i < MT * K / 16; i += kKqThreads) {
-    const int t = i / (K / 16);
-    u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (t < M) v = reinterpret_cast<const u32x4*>(xq + (int64_t)t * K)[i % (K / 16)];
-    reinterpret_cast<u32x4*>(lx)[i] = v;
+  if constexpr (XF) {
+    __builtin_amdgcn_sched_barrier(0);
+    for (int b0 = wave; b0 < nxb; b0 += XJ * xw) {
+      if (b0 != wave) load_x(b0);
+#pragma unroll
+      for (int j = 0; j < XJ; j++) {
+        const int b = b0 + j * xw;
+        if (b >= nxb) break;  // wave-uniform
+        double d;
+        int sum;
+        const uint32_t word = quantize_q8k<SUB>(xv[j], d, sum);
+        reinterpret_cast<uint32_t*>(lx)[b * 64 + lane] = word;
+        if (lane == 0) ls[b] = (float)d;
+        if (lane % (SUB / 4) == 0) lb[b * (256 / SUB) + lane / (SUB / 4)] = sum;
+      }
+    }
+    for (int b = nxb + wave; b < MT * nsb; b += xw) {
+      reinterpret_cast<uint32_t*>(lx)[b * 64 + lane] = 0u;
+      if (lane == 0) ls[b] = 0.0f;
+      if (lane % (SUB / 4) == 0) lb[b * (256 / SUB) + lane / (SUB / 4)] = 0;
+    }
+  } else {
+    for (int i = tid; i < MT * K / 16; i += nthr) {
+      const int t = i / (K / 16);
+      u32x4 v = u32x4{0u, 0u, 0u, 0u};
+      if (t < M) v = reinterpret_cast<const u32x4*>(xq + (int64_t)t * K)[i % (K / 16)];
+      reinterpret_cast<u32x4*>(lx)[i] = v;
+    }
+    for (int i = tid; i < MT * nsub; i += nthr) lb[i] = i / nsub < M ? bsums[(int64_t)i] : 0;
+    for (int i = tid; i < MT * nsb; i += nthr) ls[i] = i / nsb < M ? xs[(int64_t)i] : 0.0f;
   }
-  for (int i = tid; i < MT * nsub; i += kKqThreads) lb[i] = i / nsub < M ? bsums[(int64_t)i] : 0;
-  for (int i = tid; i < MT * nsb; i += kKqThreads) ls[i] = i / nsb < M ? xs[(int64_t)i] : 0.0f;
   __syncthreads();
   if (ng == 0) return;  // wave-uniform; no barrier follows
 
@@ -349,10 +416,10 @@ size_t kquant_gemv_lds(int format, int64_t k, int mt) {
   return (size_t)mt * (size_t)(k + 4 * (k / sub) + 4 * (k / 256));
 }
 
-template <int FMT, int MT, int D = 1>
+template <int FMT, int MT, bool XF, int D = 1>
 static hipError_t launch_kq_t(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
                               int y_dtype, int64_t m, int cu_count, hipStream_t stream) {
-  auto kernel = &kquant_gemv_kernel<FMT, MT, D>;
+  auto kernel = &kquant_gemv_kernel<FMT, MT, XF, D>;
   const size_t lds = kquant_gemv_lds(FMT, w.in, MT);
   if (lds > 65536) {
     static std::atomic<uint64_t> attr_set{0};
@@ -366,38 +433,84 @@ static hipError_t launch_kq_t(const Weight& w, const int8_t* xq, const float* xs
       attr_set.fetch_or(bit, std::memory_order_acq_rel);
     }
   }
-  // a wave per row group, all of them launched at once: at 14336 x 4096,
-  // m = 1, cold, Q4_K 10.9 us and Q6_K 17.4 us against 11.1-11.3 / 18.5 with
-  // at most 8 waves per CU (each then taking ~2 groups one after another)
-  const int64_t groups = (w.out + kKqRows - 1) / kKqRows;
-  const int64_t wg = (groups + 3) / 4;
-  (void)cu_count;
-  hipLaunchKernelGGL(kernel, dim3((unsigned)std::max<int64_t>(wg, 1)), dim3(kKqThreads), (unsigned)lds, stream, w.q,
+  // m = 1 with quantized activations of a short row: a wave per row group in
+  // workgroups of four, all launched at once (14336 x 4096, cold, Q4_K 12.3 and
+  // Q6_K 15.0 us with the quantizer, against 12.8 / 15.3 with one workgroup per
+  // CU). Otherwise at most one workgroup per CU, so that x is staged once per
+  // CU, with as many waves as spread the row groups evenly over whole turns:
+  // 28672 x 8192 m = 1 / 4 Q4_K 31.9 / 54.0 -> 30.5 / 40.7 us, Q6_K 43.2 / 79.7
+  // -> 39.7 / 54.2; 4096 x 14336 m = 4 Q4_K 21.9 -> 19.0. XF: the waves that
+  // quantizing x keeps busy, also where fewer have rows (1024 x 4096 m = 1 5.8
+  // us with the waves that have rows, 4.7 with all).
+  const int64_t groups = std::max<int64_t>((w.out + kKqRows - 1) / kKqRows, 1);
+  int64_t waves = kKqThreads / 64, wg = (groups + waves - 1) / waves;
+  if (XF || MT > 1 || w.in >= 8192) {
+    const int64_t turns = (groups + cu_count * kKqWaves - 1) / (cu_count * kKqWaves);
+    waves = std::max<int64_t>(waves, (groups + cu_count * turns - 1) / (cu_count * turns));
+    if (XF) {
+      waves = std::max<int64_t>(waves, std::min<int64_t>(kKqWaves, m * (w.in / 256)));
+      wg = std::min<int64_t>(cu_count, groups);
+    } else {
+      wg = std::min<int64_t>(cu_count, (groups + waves - 1) / waves);
+    }
+  }
+  hipLaunchKernelGGL(kernel, dim3((unsigned)wg), dim3((unsigned)(64 * waves)), (unsigned)lds, stream, w.q,
                      w.scales, w.sub_scales, xq, xs, bsums, y, (int)m, (int)w.in, (int)w.out, y_dtype);
   return hipGetLastError();
 }
 
-hipError_t launch_kquant_gemv(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
-                              int y_dtype, int64_t m, int cu_count, hipStream_t stream) {
+// XF: xs is the f32 x
+template <bool XF>
+static hipError_t launch_kquant_rows(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
+                                     int y_dtype, int64_t m, int cu_count, hipStream_t stream) {
   const int64_t nsub = w.in / (w.format == RQ_Q4_K ? 32 : 16), nsb = w.in / 256;
   const size_t ysz = y_dtype == RQ_F32 ? 4 : 2;
-  // four activation rows per launch
+  // four activation rows per launch; two rows have an instance of their own
+  // (14336 x 4096, Q4_K, with the quantizer: 17.6 us in the one for four, 14.5)
   for (int64_t t0 = 0; t0 < m; t0 += 4) {
     const int64_t mt = std::min<int64_t>(4, m - t0);
-    const int8_t* xq_t = xq + t0 * w.in;
-    const float* xs_t = xs + t0 * nsb;
-    const int32_t* bs_t = bsums + t0 * nsub;
+    const int8_t* xq_t = XF ? nullptr : xq + t0 * w.in;
+    const float* xs_t = xs + t0 * (XF ? w.in : nsb);
+    const int32_t* bs_t = XF ? nullptr : bsums + t0 * nsub;
     void* y_t = static_cast<uint8_t*>(y) + (size_t)(t0 * w.out) * ysz;
     hipError_t e;
     if (w.format == RQ_Q4_K)
-      e = mt == 1 ? launch_kq_t<RQ_Q4_K, 1>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream)
-                  : launch_kq_t<RQ_Q4_K, 4>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream);
+      e = mt == 1   ? launch_kq_t<RQ_Q4_K, 1, XF>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream)
+          : mt == 2 ? launch_kq_t<RQ_Q4_K, 2, XF>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream)
+                    : launch_kq_t<RQ_Q4_K, 4, XF>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream);
     else
-      e = mt == 1 ? launch_kq_t<RQ_Q6_K, 1>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream)
-                  : launch_kq_t<RQ_Q6_K, 4>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream);
+      e = mt == 1   ? launch_kq_t<RQ_Q6_K, 1, XF>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream)
+          : mt == 2 ? launch_kq_t<RQ_Q6_K, 2, XF>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream)
+                    : launch_kq_t<RQ_Q6_K, 4, XF>(w, xq_t, xs_t, bs_t, y_t, y_dtype, mt, cu_count, stream);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+hipError_t launch_kquant_gemv(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
+                              int y_dtype, int64_t m, int cu_count, hipStream_t stream) {
+  return launch_kquant_rows<false>(w, xq, xs, bsums, y, y_dtype, m, cu_count, stream);
+}
+
+// Every CU quantizes all of x, 0.08 us per 256 elements, against 1.5-2.5 us for
+// the quantizer's own launch. Cold, in a graph, own launch / fused: Q4_K
+// 14336 x 4096 m = 1 / 2 / 3 / 4 12.2 / 10.6, 14.7 / 13.2, 16.8 / 16.3,
+// 17.2 / 17.1 us; 4096 x 4096 m = 1 / 3 / 4 7.7 / 5.9, 10.0 / 10.0, 10.2 / 11.0;
+// 28672 x 8192 m = 1 / 2 31.2 / 28.6, 34.2 / 33.9; 2048 x 5632 m = 2 / 3 9.4 /
+// 8.4, 11.5 / 11.3; 4096 x 14336 m = 1 13.1 / 13.4; 32000 x 2048 m = 4 20.6 /
+// 19.4; Q6_K 14336 x 4096 m = 1 / 3 14.5 / 13.3, 19.5 / 18.9. The line is
+// between 3 x 4096 and 1 x 14336. Workgroups read x while others store y, so a
+// call whose y overlaps x keeps the quantizer's launch.
+bool kquant_gemv_quantizes(const Weight& w, const float* x, const void* y, int y_dtype, int64_t m) {
+  if (m > 4 || m * w.in > kKqFusedMax) return false;
+  const uintptr_t x0 = (uintptr_t)x, x1 = x0 + (size_t)m * (size_t)w.in * 4;
+  const uintptr_t y0 = (uintptr_t)y, y1 = y0 + (size_t)m * (size_t)w.out * (y_dtype == RQ_F32 ? 4 : 2);
+  return y1 <= x0 || x1 <= y0;
+}
+
+hipError_t launch_kquant_gemv_f32(const Weight& w, const float* x, void* y, int y_dtype, int64_t m, int cu_count,
+                                  hipStream_t stream) {
+  return launch_kquant_rows<true>(w, nullptr, x, nullptr, y, y_dtype, m, cu_count, stream);
 }
 
 // ---- dequantization, bitwise as dequant-q4k / dequant-q6k (the products are

@@ -200,6 +200,10 @@ hipError_t launch_quantize_act_i8(const float* x, int64_t m, int64_t in, int8_t*
 // K-quants (kquant.hip)
 hipError_t launch_quantize_act_q8k(const float* x, int64_t m, int64_t in, int sub, int8_t* xq, float* xs,
                                    int32_t* bsums, hipStream_t stream);
+// The GEMV with q8_K quantization of f32 x inside, and whether a call takes it.
+bool kquant_gemv_quantizes(const Weight& w, const float* x, const void* y, int y_dtype, int64_t m);
+hipError_t launch_kquant_gemv_f32(const Weight& w, const float* x, void* y, int y_dtype, int64_t m, int cu_count,
+                                  hipStream_t stream);
 size_t kquant_gemv_lds(int format, int64_t k, int mt);
 hipError_t launch_kquant_gemv(const Weight& w, const int8_t* xq, const float* xs, const int32_t* bsums, void* y,
                               int y_dtype, int64_t m, int cu_count, hipStream_t stream);
