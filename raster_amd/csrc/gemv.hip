@@ -59,10 +59,10 @@ struct SkinnyLds {
   int xsf;      // f32 xsf[mt + 1][xstr]: 2^(e-15), NaN for non-finite blocks; row mt zero
   int xs;       // i32 xs[mt + 1][xstr]: sum of X over the block (Q4 zero-point); row mt zero
   int zero;     // 16 zero bytes
-  int red;      // f32 red[waves][mg][64]
+  int red;      // f32 red[nred][waves][mg][64]
   int nss;      // f32 nss[waves][mt]: the waves' partial sums of squares (input RMSNorm)
   int bytes;
-  __host__ __device__ SkinnyLds(int mt, int k, int waves) {
+  __host__ __device__ SkinnyLds(int mt, int k, int waves, int nred) {
     kp = (k + 63) / 64 * 64;
     nbp = kp / 32;
     lstr = kp + 32;
@@ -72,7 +72,7 @@ struct SkinnyLds {
     xs = xsf + (mt + 1) * xstr * 4;
     zero = xs + (mt + 1) * xstr * 4;
     red = zero + 16;
-    nss = red + waves * (mt / 4) * 64 * 4;
+    nss = red + nred * waves * (mt / 4) * 64 * 4;
     bytes = nss + waves * mt * 4;
   }
 };
@@ -222,7 +222,7 @@ template <int FMT, typename ST, int XT, int MT, int WAVES, int NB, int RING, boo
 __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc,
                                                            const void* __restrict__ x, void* __restrict__ y, int M,
                                                            int K, int N, int npad, int y_dtype, int ksplit,
-                                                           float* __restrict__ part, DecodeOps ops) {
+                                                           int nred, float* __restrict__ part, DecodeOps ops) {
   constexpr int MG = MT / 4;                 // MFMAs per window (4 activation rows each)
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int nb = K / 32, nw = (K + 63) / 64;
@@ -232,7 +232,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(const uint8_t* __res
   const int s = (int)blockIdx.x % ksplit;
   const int sw = slice_windows(nw, ksplit, NB);
   const int s_beg = min(nw, s * sw), s_end = min(nw, s_beg + sw);
-  const SkinnyLds L(MT, 64 * sw, WAVES);
+  const SkinnyLds L(MT, 64 * sw, WAVES, nred);
   int8_t* lev = reinterpret_cast<int8_t*>(smem + L.lev);
   float* xsf = reinterpret_cast<float*>(smem + L.xsf);
   int* xs = reinterpret_cast<int*>(smem + L.xs);
@@ -515,21 +515,26 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(const uint8_t* __res
   // several it stores the slice's partial sums, which skinny_reduce_kernel
   // adds in slice order (workgroup 0 also leaves the rows' sums of squares
   // there for the input RMSNorm).
+  // The rounds take turns over the waves, and with two sets of partial sums
+  // (nred) over the sets: a set is written again two rounds later, past the
+  // barrier that the wave adding it up reaches only afterwards, so one barrier
+  // a round is enough.
   auto finish_group = [&](int t) {
-    const int g = gfirst + (t / nbg) * gcols;
+    const int rd = t / nbg, g = gfirst + rd * gcols;
+    float* rs = red + (nred == 2 ? (rd & 1) * WAVES * MG * 64 : 0);
 #pragma unroll
     for (int mg = 0; mg < MG; mg++) {
-      red[(wave * MG + mg) * 64 + lane] = acc[mg];
+      rs[(wave * MG + mg) * 64 + lane] = acc[mg];
       acc[mg] = 0.0f;
     }
     __syncthreads();
-    if (wave == 0) {
+    if (wave == rd % WAVES) {
       float v[MG], rinv[MG];
 #pragma unroll
       for (int mg = 0; mg < MG; mg++) {
         v[mg] = 0.0f;
 #pragma unroll
-        for (int wv = 0; wv < WAVES; wv++) v[mg] += red[(wv * MG + mg) * 64 + lane];
+        for (int wv = 0; wv < WAVES; wv++) v[mg] += rs[(wv * MG + mg) * 64 + lane];
         rinv[mg] = 1.0f;
         const int m = 4 * mg + g4;
         if (XT != kXtI8 && ops.norm_gain && m < M) {
@@ -552,7 +557,7 @@ __global__ __launch_bounds__(64 * WAVES) void skinny_kernel(const uint8_t* __res
         }
       }
     }
-    __syncthreads();
+    if (nred == 1) __syncthreads();
   };
   // a ring of RING batch slots: task t computes from slot t % RING while the
   // loads of tasks t + 1 .. t + RING - 1 are in flight. Task 0's batch went
@@ -631,11 +636,18 @@ DecodePlan plan_decode(int64_t m, int64_t k, int64_t npad, int cu_count) {
   p.waves = p.mt == 4 && (ngroups > cu_count || m > 2) && nw >= 16 * kBatch ? 16 : 8;
   const int per_cu_max = 1;
   int64_t ks = 1;
-  while (SkinnyLds(p.mt, 64 * slice_windows((int)nw, (int)ks, kBatch), p.waves).bytes > 163840) {
+  while (SkinnyLds(p.mt, 64 * slice_windows((int)nw, (int)ks, kBatch), p.waves, 1).bytes > 163840) {
     if (ks >= nw) return p;
     ks++;
   }
-  const int lds = SkinnyLds(p.mt, 64 * slice_windows((int)nw, (int)ks, kBatch), p.waves).bytes;
+  auto lds_bytes = [&](int nred) {
+    return SkinnyLds(p.mt, 64 * slice_windows((int)nw, (int)ks, kBatch), p.waves, nred).bytes;
+  };
+  // a second set of partial sums where workgroups take several groups and it
+  // fits (cold, one set / two: Q4_0 28672 x 8192 m = 2 32.6 / 31.5 us, with the
+  // input norm m = 1 32.6 / 30.4; 14336 x 4096 m = 4 14.0 / 13.7)
+  p.nred = ngroups * ks > cu_count && lds_bytes(2) <= 163840 ? 2 : 1;
+  const int lds = lds_bytes(p.nred);
   const int per_cu = std::max(1, std::min(163840 / lds, per_cu_max));
   const int64_t gcols = std::min<int64_t>(ngroups, std::max<int64_t>(1, (int64_t)per_cu * cu_count / ks));
   if (gcols * ks > INT32_MAX) return p;
@@ -666,7 +678,7 @@ static hipError_t launch_t(const MatmulArgs& a, const DecodePlan& p) {
   const bool split = p.ksplit > 1;
   hipExtLaunchKernelGGL(kernel, dim3((unsigned)p.grid), dim3(64 * WAVES), (unsigned)p.lds_bytes, a.stream,
                         a.ev_main[0], a.ev_main[1], 0, a.q, static_cast<const ST*>(a.scales_rb), a.x,
-                        a.y, (int)a.m, (int)a.k, (int)a.n, (int)a.npad, a.y_dtype, p.ksplit, a.part, a.ops);
+                        a.y, (int)a.m, (int)a.k, (int)a.n, (int)a.npad, a.y_dtype, p.ksplit, p.nred, a.part, a.ops);
   if (hipError_t e = hipGetLastError()) return e;
   if (split) {
     const int ngroups = (int)(a.npad / 16);

@@ -123,7 +123,7 @@ struct MatmulArgs {
 // decode kernel cannot take the shape (then the GEMM path runs).
 struct DecodePlan {
   bool ok;
-  int mt, waves, ksplit, grid, lds_bytes;
+  int mt, waves, ksplit, nred, grid, lds_bytes;  // nred: sets of partial sums in LDS, 1 or 2
   size_t part_bytes;  // scratch for the slices' partial sums (ksplit > 1)
 };
 DecodePlan plan_decode(int64_t m, int64_t k, int64_t npad, int cu_count);
