@@ -158,8 +158,11 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  * Kernel by call (plain calls; every rq_qmatmul_fused call takes the int8-level
  * decode kernel):
  *  - m = 1, Q4_0: the v_dot4_i32_i8 GEMV;
- *  - m <= 16, MFMA decode (bf16 MFMA on exact codes): Q4_0 at 5 <= m <= 16,
- *    Q8_0 at 9 <= m <= 16 when out * in <= 32 Mi (2^25) elements;
+ *  - m <= 16, MFMA decode (bf16 MFMA on exact codes; n = out rounded up to
+ *    16): Q4_0 at 5 <= m <= 16, and at 2 <= m <= 4 when in >= 5632 and
+ *    m * in > 2 n; Q8_0 with in >= 3072 and n * in <= 64 Mi (2^26) elements at
+ *    6 <= m <= 16 when 4 m * in >= 9 n and at m = 5 when m * in >= 6 n, with
+ *    in < 3072 and n * in <= 32 Mi at 9 <= m <= 16 when m * in >= 5 n;
  *  - every other m <= 16: the int8-level decode kernel (int8 MFMA on the raw
  *    codes, v_mfma_i32_16x16x64_i8);
  *  - m > 16: bf16 x: the bf16 MFMA GEMM (the weight-stream GEMM for Q4_0
@@ -190,9 +193,9 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    non-negative integers (c + 136 for Q4_0, c + 128 for Q8_0), the offset
  *    times the block's activation sum subtracted and the block scale applied
  *    in f32; f32 x split into two bf16 terms (|x - hi - lo| <= 2^-17 |x|).
- *    Finite input range: a block whose largest |x| exceeds about 7e34 (Q4_0)
- *    or 4e34 (Q8_0) overflows the offset sums and makes its row's outputs
- *    NaN; a non-finite activation makes its row's outputs non-finite.
+ *    A row with |x| >= 2^112 in a K-slice is taken there at 2^-13 x, so that
+ *    the sums of offset codes overflow for no finite x; a non-finite
+ *    activation makes its row's outputs non-finite.
  *  - bf16 x, m > 16: weights are dequantized to bf16 (exact f32 product
  *    scale*code, then one round-to-nearest-even) and multiplied with bf16 MFMA;
  *    on the eight-wave 16x16x32 tiles (m > 128 where the tile cost model
@@ -219,7 +222,9 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    m <= 8); the MFMA decode kernel when a slice of x would not fit two
  *    workgroups' LDS, and further until the grid covers about 85% of the CUs,
  *    rounded up to a power of two while each slice keeps 8 blocks (at most
- *    in / 32 slices); the weight-stream GEMM (bf16 x, 16 < m <= 64) on a
+ *    in / 32 slices; a call at m <= 8, or with Q8_0 and n * in above 32 Mi,
+ *    that cannot have them runs the int8-level kernel, except Q4_0 at m >= 5);
+ *    the weight-stream GEMM (bf16 x, 16 < m <= 64) on a
  *    thin grid (up to 8 slices);
  *  - Q4_K / Q6_K: the q8_K activations, m * (in + in/256*4 + in/sub*4)
  *    bytes (each part rounded up to 256), sub = 32 for Q4_K, 16 for Q6_K.

@@ -907,7 +907,7 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   a.part = nullptr;
   a.ops = dops;
   const bool plain = !dops.norm_gain && !dops.residual && !dops.swiglu && !dops.act_i8;
-  const MfPlan mf = plain && plan.ok ? plan_gemv_mf(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : MfPlan{};
+  MfPlan mf = plain && plan.ok ? plan_gemv_mf(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : MfPlan{};
   // the m = 1 GEMV also quantizes to int8 blocks itself (act_i8)
   const bool plain_g1 = !dops.norm_gain && !dops.residual && !dops.swiglu;
   const G1Plan g1 = plain_g1 && plan.ok ? plan_gemv1(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : G1Plan{};
@@ -919,11 +919,15 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   void* part = nullptr;
   if (g1.ok) {
     // the m = 1 GEMV uses no scratch
-  } else if (mf.ok) {
-    if (mf.ks > 1) {
-      if (int s = call_scratch(c, fixed, a.stream, (size_t)mf.ks * (size_t)m * (size_t)w.out * 4, 1, &part))
-        return s;
+  } else if (mf.ok && mf.ks > 1) {
+    if (int s = call_scratch(c, fixed, a.stream, (size_t)mf.ks * (size_t)m * (size_t)w.out * 4, 1, &part)) {
+      // without scratch (captured before it was grown, memory full): the
+      // int8-level kernel, which needs less of it or none
+      if (mf.always) return s;
+      mf.ok = false;
     }
+  }
+  if (g1.ok || mf.ok) {
   } else if (plan.ok && plan.ksplit > 1) {
     if (int s = call_scratch(c, fixed, a.stream, plan.part_bytes, 1, &part)) return s;
   } else if (!plan.ok && x_dtype == RQ_BF16 && wide.ok) {

@@ -1,5 +1,4 @@
-// gemv_mf.hip — decode matmul (m <= 16; planned for 4 < m <= 16 with Q4_0
-// weights, 8 < m <= 16 with Q8_0) of plain
+// gemv_mf.hip — decode matmul (2 <= m <= 16, where mf_takes says) of plain
 // rq_qmatmul calls with f32 or bf16 activations, on bf16 MFMA with exact
 // codes.
 //
@@ -119,7 +118,7 @@ __device__ __forceinline__ bf16x8 mf_q8_codes(const MfCodes<ST>& c) {
 }  // namespace
 
 // LDS bytes of a workgroup: x fragments (spl steps x P parts x m rows x 64 B),
-// the offset sums (spl x 16 floats), a 16-byte zero slot, and with KW > 1 two
+// the offset sums (spl x 16 floats), 16 bytes of wave flags, and with KW > 1 two
 // sets of the waves' partial outputs
 __host__ __device__ inline int mf_lds_bytes(int m, int spl, int parts, int kw, int gw) {
   return spl * parts * m * 64 + spl * 64 + 16 + (kw > 1 ? 2 * gw * kw * 1024 : 0);
@@ -138,7 +137,7 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
   const int s = (int)blockIdx.x % ks, col = (int)blockIdx.x / ks, gcols = (int)gridDim.x / ks;
   const int spl = (nkb + ks - 1) / ks;
   const int kb0 = min(nkb, s * spl), nst = min(nkb, kb0 + spl) - kb0;  // this slice: steps kb0 .. kb0+nst-1
-  const int xs_off = spl * P * M * 64, zero_off = xs_off + spl * 64, red_off = zero_off + 16;
+  const int xs_off = spl * P * M * 64, flag_off = xs_off + spl * 64, red_off = flag_off + 16;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int kw = wave % KW, gw = wave / KW;
@@ -151,6 +150,8 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
   constexpr int XI = 4;
   const int nitems = M * nst * 4, stride = 64 * WAVES;
   float xv[XI][8];
+  float amax = 0.0f;     // the lane's largest |x|
+  bool restage = false;  // rows flagged in LDS at 2^-13 x
   auto load_items = [&](int base) {
 #pragma unroll
     for (int i = 0; i < XI; i++) {
@@ -181,11 +182,13 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
       const int idx = min(idx0, nitems - 1);
       const int m = idx / (nst * 4), rem = idx - m * nst * 4, u = rem >> 2, qq = rem & 3;
       uint32_t hi[4], lo[4];
-      float sum = 0.0f;
+      float sum = 0.0f, xsc = 1.0f;
+      if (restage && smem[flag_off + m]) xsc = 0x1p-13f;
       if (XT == RQ_F32) {
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const float a = xv[i][2 * e], b = xv[i][2 * e + 1];
+          const float a = xv[i][2 * e] * xsc, b = xv[i][2 * e + 1] * xsc;
+          amax = fmaxf(amax, fmaxf(fabsf(a), fabsf(b)));
           hi[e] = pack2_bf16(a, b);
           const float ha = bf16_bits_to_f32(hi[e] & 0xFFFFu), hb = __uint_as_float(hi[e] & 0xFFFF0000u);
           lo[e] = pack2_bf16(a - ha, b - hb);
@@ -196,6 +199,9 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
 #pragma unroll
         for (int e = 0; e < 4; e++) {
           hi[e] = __float_as_uint(xv[i][e]);
+          const float a = bf16_bits_to_f32(hi[e] & 0xFFFFu), b = __uint_as_float(hi[e] & 0xFFFF0000u);
+          amax = fmaxf(amax, fmaxf(fabsf(a), fabsf(b)));
+          if (restage) hi[e] = pack2_bf16(a * xsc, b * xsc);
           sum += bf16_bits_to_f32(hi[e] & 0xFFFFu) + __uint_as_float(hi[e] & 0xFFFF0000u);
         }
       }
@@ -306,8 +312,44 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
     const int u = i / (16 - M), m = M + i % (16 - M);
     *reinterpret_cast<float*>(smem + xs_off + (u * 16 + m) * 4) = 0.0f;
   }
-  if (tid < 4) reinterpret_cast<uint32_t*>(smem + zero_off)[tid] = 0u;
+  // A row holding |x| >= 2^112 in the slice is staged again at 2^-13 x, so that
+  // sums of x (c + OFF), |c + OFF| <= 255, over a block cannot overflow where the
+  // block's dot product would not; its outputs take the factor back.
+  static_assert(16 % WAVES == 0, "flag bytes per wave");
+  uint8_t* flags = smem + flag_off;
+  const bool wbig = __any(amax >= 0x1p112f) != 0;
+  if (lane < 16 / WAVES) flags[wave * (16 / WAVES) + lane] = wbig ? 1 : 0;
   __syncthreads();
+  const u32x4 fl = *reinterpret_cast<const u32x4*>(flags);
+  f32x4 ysc = {1.0f, 1.0f, 1.0f, 1.0f};
+  if (__builtin_amdgcn_readfirstlane((int)(fl[0] | fl[1] | fl[2] | fl[3])) != 0) {
+    __syncthreads();  // the wave flags read; now a flag per row
+    if (tid < 4) reinterpret_cast<uint32_t*>(flags)[tid] = 0u;
+    __syncthreads();
+    for (int base = 0; base < nitems; base += stride * XI) {
+      load_items(base);
+#pragma unroll
+      for (int i = 0; i < XI; i++) {
+        if (base + stride * i >= nitems) break;
+        float t = 0.0f;
+#pragma unroll
+        for (int e = 0; e < (XT == RQ_F32 ? 8 : 4); e++) {
+          t = fmaxf(t, fabsf(xv[i][e]));
+          if (XT != RQ_F32) t = fmaxf(t, fabsf(__uint_as_float(__float_as_uint(xv[i][e]) << 16)));
+        }
+        if (t >= 0x1p112f) flags[min(base + tid + stride * i, nitems - 1) / (nst * 4)] = 1;
+      }
+    }
+    __syncthreads();
+    restage = true;
+    for (int base = 0; base < nitems; base += stride * XI) {
+      load_items(base);
+      convert_items(base);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; e++) ysc[e] = flags[4 * qd + e] ? 0x1p13f : 1.0f;
+  }
 
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
   auto store = [&](int j, const f32x4& v) {
@@ -318,12 +360,13 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
     for (int e = 0; e < 4; e++) {
       const int m = 4 * qd + e;
       if (m >= M) break;
+      const float ve = v[e] * ysc[e];
       if (ks > 1)
-        part[((int64_t)s * M + m) * N + o] = v[e];
+        part[((int64_t)s * M + m) * N + o] = ve;
       else if (y_dtype == RQ_F32)
-        static_cast<float*>(y)[(int64_t)m * N + o] = v[e];
+        static_cast<float*>(y)[(int64_t)m * N + o] = ve;
       else
-        static_cast<uint16_t*>(y)[(int64_t)m * N + o] = (uint16_t)f32_to_bf16_bits(v[e]);
+        static_cast<uint16_t*>(y)[(int64_t)m * N + o] = (uint16_t)f32_to_bf16_bits(ve);
     }
   };
   auto finish = [&](int j) {
@@ -480,12 +523,33 @@ hipError_t launch_gemv_mf_t(const MatmulArgs& a, int ks, int gcols) {
 
 namespace rq {
 
-// Plan: taken for 4 < m <= 16 with Q4_0 weights, 8 < m <= 16 with Q8_0. There
-// the int8 decode kernel spends most of its time forming its activation levels
-// and in its per-window epilogue (K = 4096, N = 14336 Q4, f32 x: m = 6 / 8 /
-// 16 21.4 / 23.6 / 38 us, this kernel 16.3 / 16.7 / 18 us); below it stays
-// ahead (m = 2 / 4: 12.3 / 14.9 us against 15.6 / 16.0 us). The waves of a workgroup take different groups
-// (splitting K between them measured slower at m = 16): Q4_0 16 waves with
+// Whether this kernel takes a call, or the int8-level kernel (gemv.hip). That one
+// forms the levels of all m rows in every workgroup, ~ m k, and has a long
+// epilogue per window; this one reads a slice of x a workgroup, but adds slices in
+// a second launch and streams Q8_0 by 8-byte loads. Cold, in a graph, f32 x,
+// int8-level kernel / this one, us:
+//  * Q4_0, m >= 5: always (14336 x 4096 m = 5 / 16 20.9 / 15.3, 40.2 / 16.5;
+//    the exceptions are short rows at m <= 8, 11264 x 2048 m = 8 12.5 / 14.5).
+//    m = 2 .. 4: long rows against few outputs, k >= 5632 and m k > 2 n (4096 x
+//    14336 m = 2 / 4 19.2 / 15.8, 26.4 / 16.2; 4096 x 11008 16.9 / 14.5, 20.7 /
+//    14.2; 2048 x 5632 9.5 / 9.2, 12.4 / 9.7; 8192 x 8192 m = 2 / 3 14.8 / 15.2,
+//    16.0 / 15.5; 28672 x 8192 m = 4 35.2 / 35.5; 4096 x 4096 m = 4 9.4 / 10.4).
+//  * Q8_0, rows of 3072 and more, weights to 64 Mi codes: m >= 6 with m k >= 9/4
+//    n, m = 5 with m k >= 6 n (14336 x 4096 m = 6 / 8 / 16 22.5 / 22.8, 24.3 /
+//    22.8, 37.4 / 28.7; 4096 x 14336 m = 5 / 16 28.0 / 22.8, 40.0 / 28.4; 4096 x
+//    4096 m = 5 / 6 / 8 12.4 / 12.8, 13.5 / 13.0, 16.2 / 13.1; 8192 x 8192 m = 12
+//    35.9 / 28.1; 8192 x 3072 m = 6 15.8 / 15.1; past the line 11008 x 8192 m =
+//    9 38.3 / 43.4, 28672 x 8192 m = 16 72.9 / 87.9). Shorter rows, weights to
+//    32 Mi: m >= 9 with m k >= 5 n (2048 x 2048 m = 9 11.1 / 9.9; 6144 x 2048 m
+//    = 12 / 16 14.9 / 17.3, 17.6 / 17.2; 11264 x 2048 m = 9 15.0 / 19.4).
+static bool mf_takes(int64_t m, int64_t k, int64_t npad, int format) {
+  if (format == RQ_Q4_0) return m >= 5 || (k >= 5632 && m * k > 2 * npad);
+  if (k >= 3072)
+    return npad * k <= (int64_t(64) << 20) && (m >= 6 ? 4 * m * k >= 9 * npad : m == 5 && m * k >= 6 * npad);
+  return m >= 9 && npad * k <= (int64_t(32) << 20) && m * k >= 5 * npad;
+}
+
+// Plan. The waves of a workgroup take different groups (splitting K between them measured slower at m = 16): Q4_0 16 waves with
 // an 8-step ring (two quads; at that shape 17.9 us against 18.8 for 8 waves
 // and 16 steps, and at K = 8192, N = 28672, bf16 x, 40.6 against 45.8),
 // Q8_0 8 waves with a 16-step ring (32 steps: 30 us with 8-byte Q4 loads);
@@ -495,12 +559,8 @@ namespace rq {
 // m = 6 the LDS alone would allow 2 (23.3 us against 16.3 at 4).
 MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format, int cu_count) {
   MfPlan p{};
-  const int64_t m_min = format == RQ_Q4_0 ? 5 : 9;
-  if (m < m_min || m > 16 || (x_dtype != RQ_F32 && x_dtype != RQ_BF16) || k % 32 != 0 || k < 32) return p;
-  // Q8_0 (8-byte loads, no quads) only for small weights: at 4096 x 4096
-  // m = 12 / 16 15.1 / 15.4 us against 26.9 for the int8-level kernel, at
-  // K = 8192, N = 28672 81 / 90 / 101 us against 62 / 66 / 70 (m = 9 / 12 / 16)
-  if (format == RQ_Q8_0 && npad * k > (int64_t(32) << 20)) return p;
+  if (m < 2 || m > 16 || (x_dtype != RQ_F32 && x_dtype != RQ_BF16) || k % 32 != 0 || k < 32) return p;
+  if (!mf_takes(m, k, npad, format)) return p;
   const int parts = x_dtype == RQ_F32 ? 2 : 1;
   const int64_t nkb = k / 32, ngroups = npad / 16;
   p.kw = 1;
@@ -525,6 +585,7 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
   ks = kf;
   p.ks = (int)ks;
   if ((int64_t)p.gcols * ks > INT32_MAX) return p;
+  p.always = format == RQ_Q4_0 ? m >= 5 : m >= 9 && npad * k <= (int64_t(32) << 20);
   p.ok = true;
   return p;
 }

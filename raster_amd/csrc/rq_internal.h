@@ -129,7 +129,7 @@ struct DecodePlan {
 DecodePlan plan_decode(int64_t m, int64_t k, int64_t npad, int cu_count);
 
 // Decode on bf16 MFMA with exact codes (gemv_mf.hip): plain calls, f32 / bf16
-// x, 4 < m <= 16 (Q4_0) or 8 < m <= 16 (Q8_0) (the kernel takes m <= 16).
+// x, 2 <= m <= 16, by m, k and n (mf_takes; the kernel takes m <= 16).
 // kw x gw waves per workgroup,
 // wd-step weight ring, ks K-slices, gcols workgroup columns per slice.
 // Dense f32 GEMM (dense.hip, rocBLAS): a library handle per context, created
@@ -146,6 +146,7 @@ hipError_t launch_bias_rows(const float* b, float* y, int64_t rows, int64_t cols
 
 struct MfPlan {
   bool ok;
+  bool always;  // no falling back to the int8-level kernel where its scratch cannot be had
   int kw, gw, wd, ks, gcols;
 };
 MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format, int cu_count);

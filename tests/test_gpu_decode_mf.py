@@ -186,3 +186,31 @@ def test_mf_matches_fused_path_closely(torch, ctx, orc):
     torch.cuda.synchronize()
     w.destroy()
     assert orc.normwise_relerr(a.cpu().numpy(), b.cpu().numpy().astype(np.float64)) < TOL_F32
+
+
+@pytest.mark.parametrize("fmt,m,out,in_", [("q4", 2, 2816, 5632), ("q4", 2, 2801, 5632), ("q4f", 3, 40, 5632),
+                                           ("q4", 4, 4096, 14336), ("q4", 4, 100, 5600), ("q8", 5, 2560, 3072), ("q8", 5, 2577, 3072),
+                                           ("q8", 6, 1500, 4096), ("q8", 8, 8190, 3072), ("q8", 9, 37, 2048),
+                                           ("q8", 9, 3700, 2048), ("q8", 16, 6400, 10496), ("q4", 4, 40, 17504)])
+@pytest.mark.parametrize("xdt", ["f32", "bf16"])
+def test_mf_lines_and_large_values(torch, ctx, orc, fmt, m, out, in_, xdt):
+    """Calls on both sides of the lines between this kernel and the int8-level
+    one, with one row of 2^112 .. 2^122: every finite result inside the looser
+    bound of the two, 2^-15 of the block's largest |x| per weight, and the small
+    row beside the large one inside its own."""
+    import raster_amd
+
+    x = wl.activations(m, in_, seed=7 * m).reshape(m, in_).copy()
+    x[m - 1] *= 2.0 ** 119 / np.abs(x[m - 1]).max()
+    x[0] *= 2.0 ** -60
+    if xdt == "bf16":
+        x = torch.from_numpy(x).bfloat16().float().numpy()
+    note(f"mf lines {fmt} m={m} {out}x{in_} {xdt}")
+    w, dense, s, off = make(raster_amd, ctx, orc, fmt, out, in_, seed=out)
+    y = run(torch, w, x, xdt, "f32")
+    w.destroy()
+    ref = x.astype(np.float64) @ dense.astype(np.float64).T
+    bmax = np.repeat(np.abs(x.astype(np.float64)).reshape(m, -1, 32).max(axis=2), 32, axis=1)
+    lvl = 2.0 ** -15 * (bmax @ np.abs(dense.astype(np.float64)).T) + 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ np.abs(dense.astype(np.float64)).T)
+    assert np.all(np.isfinite(y))
+    assert np.all(np.abs(y - ref) <= np.maximum(mf_bound(x, dense, s, off), lvl))
