@@ -14,7 +14,7 @@ raster/compiler/backend/cpu/quant.clj:85-90,206-212) and run on the device:
   q4_K : rq_q4k_of (quantize-weight-q4k on the device; rows of `cols` not a
          multiple of 256 are zero-padded as raster.quant.pack/q4k-of does),
          a resident Q4_K weight, then per call rq_qmatmul with f32 x, which
-         quantizes x to q8_K and runs the K-quant GEMV in one call
+         quantizes x to q8_K and runs the K-quant GEMV or GEMM in one call
          (quantize-act-q8k + qmatmul-q4k-composable!, bitwise the same as
          rq_quantize_act_q8k + rq_qmatmul_q8k);
   q6_K : the same with rq_quantize_weight_q6k and the Q6_K kernel;

@@ -1,5 +1,5 @@
-"""GPU parity of the MFMA decode kernel (plain rq_qmatmul, 8 < m <= 16, f32 or
-bf16 activations) against the C oracle.
+"""GPU parity of the MFMA decode kernel (plain rq_qmatmul, 2 <= m <= 16 by
+the lines of mf_takes, f32 or bf16 activations) against the C oracle.
 
 The kernel splits each f32 activation into bf16 hi + lo (|x - hi - lo| <=
 2^-17 |x|), feeds the codes to the MFMA exactly with an offset (Q4 nibble n as
