@@ -223,7 +223,8 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    workgroups' LDS, and further until the grid covers about 85% of the CUs,
  *    rounded up to a power of two while each slice keeps 8 blocks (at most
  *    in / 32 slices; a call at m <= 8, or with Q8_0 and n * in above 32 Mi,
- *    that cannot have them runs the int8-level kernel, except Q4_0 at m >= 5);
+ *    that cannot have them or needs more than RQ_NOALLOC_SCRATCH_MAX runs the
+ *    int8-level kernel, except Q4_0 at m >= 5);
  *    the weight-stream GEMM (bf16 x, 16 < m <= 64) on a
  *    thin grid (up to 8 slices);
  *  - Q4_K / Q6_K: the q8_K activations, m * (in + in/256*4 + in/sub*4)
@@ -231,7 +232,7 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  * Under HIP graph capture nothing can be allocated: run the same (or a
  * larger) shape once on the capturing stream before capturing, otherwise the
  * call fails with RQ_ERR_SHAPE and a message saying so (except f32 x with
- * m > 16, as above). A buffer that grows is
+ * m > 16 and the MFMA decode calls that fall back, as above). A buffer that grows is
  * replaced but not freed until rq_ctx_destroy, so a graph captured before a
  * larger call still replays on its own (still allocated) buffers; graphs and
  * eager calls on one stream share a buffer only while it has not grown, and

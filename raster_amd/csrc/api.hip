@@ -908,6 +908,10 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   a.ops = dops;
   const bool plain = !dops.norm_gain && !dops.residual && !dops.swiglu && !dops.act_i8;
   MfPlan mf = plain && plan.ok ? plan_gemv_mf(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : MfPlan{};
+  const size_t mf_bytes = mf.ok && mf.ks > 1 ? (size_t)mf.ks * (size_t)m * (size_t)w.out * 4 : 0;
+  // a call that rq_qmatmul_noalloc could not give its scratch takes the
+  // int8-level kernel in rq_qmatmul too: the two give the same bits
+  if (!mf.always && mf_bytes > kNoAllocScratchBytes) mf.ok = false;
   // the m = 1 GEMV also quantizes to int8 blocks itself (act_i8)
   const bool plain_g1 = !dops.norm_gain && !dops.residual && !dops.swiglu;
   const G1Plan g1 = plain_g1 && plan.ok ? plan_gemv1(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : G1Plan{};
@@ -920,7 +924,7 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   if (g1.ok) {
     // the m = 1 GEMV uses no scratch
   } else if (mf.ok && mf.ks > 1) {
-    if (int s = call_scratch(c, fixed, a.stream, (size_t)mf.ks * (size_t)m * (size_t)w.out * 4, 1, &part)) {
+    if (int s = call_scratch(c, fixed, a.stream, mf_bytes, 1, &part)) {
       // without scratch (captured before it was grown, memory full): the
       // int8-level kernel, which needs less of it or none
       if (mf.always) return s;

@@ -214,3 +214,39 @@ def test_mf_lines_and_large_values(torch, ctx, orc, fmt, m, out, in_, xdt):
     lvl = 2.0 ** -15 * (bmax @ np.abs(dense.astype(np.float64)).T) + 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ np.abs(dense.astype(np.float64)).T)
     assert np.all(np.isfinite(y))
     assert np.all(np.abs(y - ref) <= np.maximum(mf_bound(x, dense, s, off), lvl))
+
+
+@pytest.mark.parametrize("fmt,m,out,in_", [("q4", 4, 2048, 5632), ("q8", 6, 1024, 4096)])
+def test_mf_without_scratch(torch, orc, fmt, m, out, in_):
+    """A first call under graph capture cannot have the K-slices' scratch and
+    runs the int8-level kernel: every replay inside that kernel's bound, and the
+    same bits each time."""
+    import raster_amd
+
+    note(f"mf captured first {fmt} m={m} {out}x{in_}")
+    with raster_amd.Context(0) as c:
+        w, dense, s, off = make(raster_amd, c, orc, fmt, out, in_, seed=out)
+        x = wl.activations(m, in_, seed=m).reshape(m, in_).copy()
+        xt = torch.from_numpy(x).cuda()
+        y = torch.empty((m, out), device="cuda")
+        st = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=st):
+            w.matmul(xt, y=y)
+        ref = x.astype(np.float64) @ dense.astype(np.float64).T
+        bmax = np.repeat(np.abs(x.astype(np.float64)).reshape(m, -1, 32).max(axis=2), 32, axis=1)
+        lvl = 2.0 ** -15 * (bmax @ np.abs(dense.astype(np.float64)).T)
+        lvl += 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ np.abs(dense.astype(np.float64)).T)
+        first = None
+        for i in range(3):
+            y.fill_(float("nan"))
+            g.replay()
+            torch.cuda.synchronize()
+            got = y.cpu().numpy()
+            assert np.all(np.abs(got - ref) <= lvl)
+            first = got if first is None else first
+            assert np.array_equal(got, first)
+            w.matmul(xt * (i + 2))
+        torch.cuda.synchronize()
+        w.destroy()
