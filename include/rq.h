@@ -160,9 +160,9 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *  - m = 1, Q4_0: the v_dot4_i32_i8 GEMV;
  *  - m <= 16, MFMA decode (bf16 MFMA on exact codes; n = out rounded up to
  *    16): Q4_0 at 5 <= m <= 16, and at 2 <= m <= 4 when in >= 5632 and
- *    m * in > 2 n; Q8_0 with in >= 3072 and n * in <= 64 Mi (2^26) elements at
- *    6 <= m <= 16 when 4 m * in >= 9 n and at m = 5 when m * in >= 6 n, with
- *    in < 3072 and n * in <= 32 Mi at 9 <= m <= 16 when m * in >= 5 n;
+ *    m * in > 2 n; Q8_0 at 9 <= m <= 16 when n * in <= 32 Mi (2^25) elements,
+ *    and with in >= 3072 and n * in <= 64 Mi at 6 <= m <= 16 when 4 m * in >= 9 n
+ *    and at m = 5 when m * in >= 6 n;
  *  - every other m <= 16: the int8-level decode kernel (int8 MFMA on the raw
  *    codes, v_mfma_i32_16x16x64_i8);
  *  - m > 16: bf16 x: the bf16 MFMA GEMM (the weight-stream GEMM for Q4_0

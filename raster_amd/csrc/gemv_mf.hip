@@ -534,19 +534,22 @@ namespace rq {
 //    14336 m = 2 / 4 19.2 / 15.8, 26.4 / 16.2; 4096 x 11008 16.9 / 14.5, 20.7 /
 //    14.2; 2048 x 5632 9.5 / 9.2, 12.4 / 9.7; 8192 x 8192 m = 2 / 3 14.8 / 15.2,
 //    16.0 / 15.5; 28672 x 8192 m = 4 35.2 / 35.5; 4096 x 4096 m = 4 9.4 / 10.4).
+//  * Q8_0, weights to 32 Mi codes, m >= 9: always. This kernel carries x to 2^-17
+//    per element, that one to 2^-15 of its block's largest (2-norm error 2.5e-6
+//    against 3.2e-5), and the calls where that one is the faster are close (2048 x
+//    2048 m = 9 11.1 / 9.9; 4096 x 4096 m = 12 / 16 26.9 / 15.1; 6144 x 2048 m =
+//    12 / 16 14.9 / 17.3, 17.6 / 17.2; 11264 x 2048 m = 9 15.0 / 19.4).
 //  * Q8_0, rows of 3072 and more, weights to 64 Mi codes: m >= 6 with m k >= 9/4
 //    n, m = 5 with m k >= 6 n (14336 x 4096 m = 6 / 8 / 16 22.5 / 22.8, 24.3 /
 //    22.8, 37.4 / 28.7; 4096 x 14336 m = 5 / 16 28.0 / 22.8, 40.0 / 28.4; 4096 x
 //    4096 m = 5 / 6 / 8 12.4 / 12.8, 13.5 / 13.0, 16.2 / 13.1; 8192 x 8192 m = 12
 //    35.9 / 28.1; 8192 x 3072 m = 6 15.8 / 15.1; past the line 11008 x 8192 m =
-//    9 38.3 / 43.4, 28672 x 8192 m = 16 72.9 / 87.9). Shorter rows, weights to
-//    32 Mi: m >= 9 with m k >= 5 n (2048 x 2048 m = 9 11.1 / 9.9; 6144 x 2048 m
-//    = 12 / 16 14.9 / 17.3, 17.6 / 17.2; 11264 x 2048 m = 9 15.0 / 19.4).
+//    9 38.3 / 43.4, 28672 x 8192 m = 16 72.9 / 87.9).
 static bool mf_takes(int64_t m, int64_t k, int64_t npad, int format) {
   if (format == RQ_Q4_0) return m >= 5 || (k >= 5632 && m * k > 2 * npad);
-  if (k >= 3072)
-    return npad * k <= (int64_t(64) << 20) && (m >= 6 ? 4 * m * k >= 9 * npad : m == 5 && m * k >= 6 * npad);
-  return m >= 9 && npad * k <= (int64_t(32) << 20) && m * k >= 5 * npad;
+  if (m >= 9 && npad * k <= (int64_t(32) << 20)) return true;
+  return k >= 3072 && npad * k <= (int64_t(64) << 20) &&
+         (m >= 6 ? 4 * m * k >= 9 * npad : m == 5 && m * k >= 6 * npad);
 }
 
 // Plan. The waves of a workgroup take different groups (splitting K between them measured slower at m = 16): Q4_0 16 waves with
