@@ -45,10 +45,24 @@ __device__ __forceinline__ void split8(const f32x4& v0, const f32x4& v1, u32x4& 
   }
 }
 
-// bytes of the packed activations: bf16 hi + lo, or (int8) bf16 codes and f32 block scales
+// Blocks past the last one, which fill up a step, add zeros: rereading the last
+// block and scaling its sum by 0 would make NaN where y is infinite. f32
+// activations, whose sums can overflow, read as zero there, out of a resource of
+// no bytes; the int8 sums cannot, so the codes are the last block's again, with
+// scales from the zeros that the packed scales end with.
+struct ActBlock {
+  __amdgpu_buffer_rsrc_t r;
+  int off;  // of the block
+};
+__device__ __forceinline__ ActBlock act_block(const void* x, uint32_t x_bytes, int kb, int nkb, uint32_t block_bytes) {
+  return {buffer_rsrc(x, kb < nkb ? x_bytes : 0u), (int)(kb < nkb ? (uint32_t)kb * block_bytes : 0u)};
+}
+
+// bytes of the packed activations: bf16 hi + lo, or (int8) bf16 codes and f32 block
+// scales, of one block more
 int64_t packed_bytes(int x_dtype, int64_t m, int64_t k) {
   const int64_t m32 = (m + 31) / 32 * 32;
-  return x_dtype == kXtI8 ? m32 * k * 2 + m32 * (k / 32) * 4 : m32 * k * 4;
+  return x_dtype == kXtI8 ? m32 * k * 2 + m32 * (k / 32 + 1) * 4 : m32 * k * 4;
 }
 
 }  // namespace
@@ -78,7 +92,8 @@ __global__ __launch_bounds__(256) void pack_x32_split_kernel(const float* __rest
 }
 
 // int8 codes xq[M][K] and their block scales xs[M][K/32] -> the same fragments
-// (codes as bf16, exact) and, after them, the scales as [M/32][K/32][32].
+// (codes as bf16, exact) and, after them, the scales as [M/32][K/32 + 1][32], the
+// last block's zero.
 __global__ __launch_bounds__(256) void pack_x32_i8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xs,
                                                           uint16_t* __restrict__ xf, int M, int K) {
   const int nkb = K / 32, nq = (nkb + 1) / 2;
@@ -91,9 +106,9 @@ __global__ __launch_bounds__(256) void pack_x32_i8_kernel(const int8_t* __restri
   const u32x2 p = q8_dword_bf16(v[0], 1.0f), q = q8_dword_bf16(v[1], 1.0f);
   const int64_t at = (int64_t)tile * nkb + kb;
   reinterpret_cast<u32x4*>(xf)[(at * 2 + (cc & 1)) * 64 + row + 32 * (cc >> 1)] = u32x4{p[0], p[1], q[0], q[1]};
-  if (cc == 0)
-    reinterpret_cast<float*>(xf + (int64_t)((M + 31) / 32) * nkb * 1024)[at * 32 + row] =
-        m < M ? xs[(int64_t)m * nkb + kb] : 0.0f;
+  float* sf = reinterpret_cast<float*>(xf + (int64_t)((M + 31) / 32) * nkb * 1024) + (at + tile) * 32 + row;
+  if (cc == 0) sf[0] = m < M ? xs[(int64_t)m * nkb + kb] : 0.0f;
+  if (cc == 1 && kb == nkb - 1) sf[32] = 0.0f;
 }
 
 // Workgroup: WM x KG waves; tile 32 MF WM rows x 32 NF columns, a wave 32 MF x
@@ -216,33 +231,33 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
   };
 
   // ---- this wave's activation fragments: rows m0 + 32 f + lane % 32
-  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
   const int r32_last = (M + 31) / 32 - 1;
   const uint32_t xs_base = (uint32_t)(r32_last + 1) * (uint32_t)nkb * 2048u;  // I8: the scales' region
   uint32_t xo[MF], so[MF];
 #pragma unroll
   for (int f = 0; f < MF; f++) {
-    const uint32_t r32 = (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb;
-    xo[f] = PK ? r32 * (1024u * AF) + 16u * (uint32_t)lane
+    const uint32_t t32 = (uint32_t)min(m0 / 32 + f, r32_last);
+    xo[f] = PK ? t32 * (uint32_t)nkb * (1024u * AF) + 16u * (uint32_t)lane
                : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
-    so[f] = xs_base + r32 * 128u + 16u * (uint32_t)g;
+    so[f] = xs_base + t32 * (uint32_t)(nkb + 1) * 128u + 16u * (uint32_t)g;
   }
   u32x4 a[2][MF][AF];     // PK: hi j 0, 1, f32: lo j 0, 1; else the 16 f32
   f32x4 xs[2][I8 ? MF : 1][4];  // I8: the scales of rows 8 q + 4 g + 0..3
   auto aload = [&](int slot, int kb) {
-    kb = min(kb, nkb - 1);
+    const ActBlock b = I8 ? act_block(x, x_bytes, min(kb, nkb - 1), nkb, 2048u)
+                          : act_block(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
 #pragma unroll
     for (int f = 0; f < MF; f++) {
 #pragma unroll
       for (int i = 0; i < AF; i++)
         a[slot][f][i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
-                                                         (int)((uint32_t)kb * (PK ? 1024u * AF : 128u)), 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)(xo[f] + (PK ? 1024u : 16u) * i), b.off, 0));
       if (I8)
 #pragma unroll
         for (int i = 0; i < 4; i++)
           xs[slot][f][i] = __builtin_bit_cast(
-              f32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(so[f] + 32u * i), (int)((uint32_t)kb * 128u), 0));
+              f32x4,
+              __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)(so[f] + 32u * i), (int)((uint32_t)min(kb, nkb) * 128u), 0));
     }
   };
 
@@ -471,7 +486,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
   // ---- consumer
   const int l32 = lane & 31, g = lane >> 5;
   const int m0 = tm * BM + wave * 32 * MF;
-  const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
   const int r32_last = (M + 31) / 32 - 1;
   f32x16 zero, acc[MF][NF];
 #pragma unroll
@@ -489,19 +503,21 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     // rounding, as a multiply; 32 cycles a tile where 16 multiplies on the VALU
     // cost about 70 beside the FMAs that wait for them), issued ahead of the next
     // pair's MFMAs, beside which the pair before is scaled
-    const uint32_t r32 = (uint32_t)min(m0 / 32, r32_last) * (uint32_t)nkb;
-    const uint32_t xo = r32 * 2048u + 16u * (uint32_t)lane;
-    const uint32_t so = ((uint32_t)(r32_last + 1) * (uint32_t)nkb * 512u + r32 * 32u + (uint32_t)l32) * 4u;
+    const uint32_t t32 = (uint32_t)min(m0 / 32, r32_last);
+    const uint32_t xo = t32 * (uint32_t)nkb * 2048u + 16u * (uint32_t)lane;
+    const uint32_t so = ((uint32_t)(r32_last + 1) * (uint32_t)nkb * 512u + t32 * (uint32_t)(nkb + 1) * 32u + (uint32_t)l32) * 4u;
     constexpr int NP = NF / 2, TP = NB * NP;  // pairs per block and step
+    const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
     u32x4 a[RA][2];
     float xs[RA];
     auto aload = [&](int slot, int kb) {
-      kb = min(kb, nkb - 1);
+      const int ka = min(kb, nkb - 1);
 #pragma unroll
       for (int i = 0; i < 2; i++)
         a[slot][i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo + 1024u * i), (int)((uint32_t)kb * 2048u), 0));
-      xs[slot] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)so, (int)((uint32_t)kb * 128u), 0));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo + 1024u * i), (int)((uint32_t)ka * 2048u), 0));
+      xs[slot] =
+          __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)so, (int)((uint32_t)min(kb, nkb) * 128u), 0));
     };
     f32x16 p[2][2];
 #pragma unroll
@@ -566,14 +582,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
                  : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
     u32x4 a[RA][MF][4];
     auto aload = [&](int slot, int kb) {
-      kb = min(kb, nkb - 1);
+      const ActBlock b = act_block(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
 #pragma unroll
       for (int f = 0; f < MF; f++)
 #pragma unroll
         for (int i = 0; i < 4; i++)
           a[slot][f][i] = __builtin_bit_cast(
-              u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo[f] + (PK ? 1024u : 16u) * i),
-                                                           (int)((uint32_t)kb * (PK ? 4096u : 128u)), 0));
+              u32x4, __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)(xo[f] + (PK ? 1024u : 16u) * i), b.off, 0));
     };
     f32x16 p[PR];
 #pragma unroll

@@ -116,3 +116,29 @@ def test_gemm_f32_special_rows(torch, ctx, m, out, in_):
     w.destroy()
     keep = [i for i in range(m) if i not in (1, 7, m - 1)]
     assert not bool(torch.isfinite(y[[1, m - 1]]).any()) and bool((y[7] == 0).all()) and torch.equal(y[keep], y0[keep])
+
+
+@pytest.mark.parametrize("m,out,in_", [(20, 64, 96), (64, 4099, 160), (200, 3000, 288), (129, 11008, 160),
+                                       (130, 20003, 224)])
+def test_gemm_f32_overflowing_tail(torch, m, out, in_):
+    """A last block whose sum passes the largest float gives inf for finite x, also
+    where the blocks do not fill the kernels' steps; with and without scratch."""
+    import raster_amd
+
+    print(f"[gpu] f32 GEMM overflowing tail m={m} {out}x{in_}", flush=True)
+    with raster_amd.Context(0) as c:
+        w = raster_amd.QWeight.q8(np.full(out * in_, 127, np.int8), np.full(out * in_ // 32, 0.01, np.float32), out, in_,
+                                  c)
+        x = torch.ones((m, in_), device="cuda")
+        x[3:, in_ - 32:] = 2.0 ** 126
+        y = torch.empty((m, out), device="cuda")
+        s = torch.cuda.Stream()
+        torch.cuda.synchronize()
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            w.matmul(x, y=y)
+        g.replay()
+        for got in (y, w.matmul(x)):
+            torch.cuda.synchronize()
+            assert bool(torch.isfinite(got[:3]).all()) and bool((got[3:] == float("inf")).all())
+        w.destroy()

@@ -37,3 +37,19 @@ def test_gemm_i8(torch, ctx, m, out, in_, fmt, ydt):  # noqa: F811
     bound = (in_ / 32 + 8) * 2.0 ** -23 * mag + (2.0 ** -8 * ref.abs() if ydt == "bf16" else 0.0)
     # the dequantized weight is scale * code rounded to f32: one more rounding of the operands
     assert bool(((y - ref).abs() <= bound + 2.0 ** -23 * (x.abs().double() @ W.abs().T)).all())
+
+
+@pytest.mark.parametrize("m,out,in_", [(18, 40, 96), (129, 4099, 160), (200, 30001, 288)])
+def test_gemm_i8_infinite_tail_scale(torch, ctx, m, out, in_):  # noqa: F811
+    """An infinite activation scale of the last block makes its row's outputs
+    infinite, also where the blocks do not fill the kernel's steps."""
+    import raster_amd
+
+    print(f"[gpu] int8 GEMM infinite tail m={m} {out}x{in_}", flush=True)
+    w = raster_amd.QWeight.q8(np.full(out * in_, 127, np.int8), np.full(out * in_ // 32, 0.01, np.float32), out, in_,
+                              ctx)
+    xq, xs, xsum = raster_amd.quantize_act_i8(ctx, torch.ones((m, in_), device="cuda"), in_)
+    xs[3:, -1] = float("inf")
+    y = w.matmul_i8(xq, xs, xsum)
+    w.destroy()
+    assert bool(torch.isfinite(y[:3]).all()) and bool((y[3:] == float("inf")).all())
