@@ -45,18 +45,56 @@ __device__ __forceinline__ void split8(const f32x4& v0, const f32x4& v1, u32x4& 
   }
 }
 
+// Reads from one array, at a lane's offset plus a uniform one: 32-bit offsets into a
+// buffer resource, or (WIDE) 64-bit addresses.
+template <bool WIDE>
+struct Src {
+  using Off = uint32_t;
+  __amdgpu_buffer_rsrc_t r;
+  __device__ __forceinline__ Src(const void* p, int64_t bytes) : r(buffer_rsrc(p, (uint32_t)bytes)) {}
+  __device__ __forceinline__ u32x4 b128(Off v, Off s) const {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)v, (int)s, 0));
+  }
+  __device__ __forceinline__ u32x2 b64(Off v, Off s) const {
+    return __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(r, (int)v, (int)s, 0));
+  }
+  __device__ __forceinline__ uint32_t b32(Off v, Off s) const {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, (int)v, (int)s, 0);
+  }
+  __device__ __forceinline__ uint32_t b16(Off v, Off s) const {
+    return __builtin_amdgcn_raw_buffer_load_b16(r, (int)v, (int)s, 0);
+  }
+};
+template <>
+struct Src<true> {
+  using Off = uint64_t;
+  const uint8_t* p;
+  bool any;
+  __device__ __forceinline__ Src(const void* q, int64_t bytes) : p(static_cast<const uint8_t*>(q)), any(bytes != 0) {}
+  template <typename T>
+  __device__ __forceinline__ T at(Off v, Off s) const {
+    return any ? *reinterpret_cast<const T*>(p + v + s) : T{};
+  }
+  __device__ __forceinline__ u32x4 b128(Off v, Off s) const { return at<u32x4>(v, s); }
+  __device__ __forceinline__ u32x2 b64(Off v, Off s) const { return at<u32x2>(v, s); }
+  __device__ __forceinline__ uint32_t b32(Off v, Off s) const { return at<uint32_t>(v, s); }
+  __device__ __forceinline__ uint32_t b16(Off v, Off s) const { return at<uint16_t>(v, s); }
+};
+
 // Blocks past the last one, which fill up a step, add zeros: rereading the last
 // block and scaling its sum by 0 would make NaN where y is infinite. f32
 // activations, whose sums can overflow, read as zero there, out of a resource of
 // no bytes; the int8 sums cannot, so the codes are the last block's again, with
 // scales from the zeros that the packed scales end with.
+template <bool WIDE, bool I8>
 struct ActBlock {
-  __amdgpu_buffer_rsrc_t r;
-  int off;  // of the block
+  using Off = typename Src<WIDE>::Off;
+  Src<WIDE> x;
+  Off off;  // of the block
+  __device__ __forceinline__ ActBlock(const void* p, uint32_t x_bytes, int kb, int nkb, uint32_t block_bytes)
+      : x(p, I8 || kb < nkb ? x_bytes : 0u),
+        off(I8 ? (Off)min(kb, nkb - 1) * block_bytes : kb < nkb ? (Off)kb * block_bytes : 0u) {}
 };
-__device__ __forceinline__ ActBlock act_block(const void* x, uint32_t x_bytes, int kb, int nkb, uint32_t block_bytes) {
-  return {buffer_rsrc(x, kb < nkb ? x_bytes : 0u), (int)(kb < nkb ? (uint32_t)kb * block_bytes : 0u)};
-}
 
 // bytes of the packed activations: bf16 hi + lo, or (int8) bf16 codes and f32 block
 // scales, of one block more
@@ -118,8 +156,9 @@ __global__ __launch_bounds__(256) void pack_x32_i8_kernel(const int8_t* __restri
 // double-buffered LDS ring while the current ones compute; one barrier per KG
 // steps. Activation fragments go straight into registers, a block ahead: from
 // the packed copy, or (PK false: calls that have no scratch) from x itself,
-// split in registers, with the same result.
-template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int WM, int KG>
+// split in registers, with the same result. WIDE: rows so long that a tile's
+// weights or activations pass 4 GiB.
+template <int FMT, typename ST, int XT, bool PK, bool WIDE, int MF, int NF, int WM, int KG>
 __global__ __attribute__((amdgpu_flat_work_group_size(64 * WM * KG, 64 * WM * KG), amdgpu_waves_per_eu(1))) void
 gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x,
                 void* __restrict__ y, int M, int K, int N, int npad, int y_dtype, int tiles_m, uint32_t x_bytes) {
@@ -157,12 +196,11 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
   // reread it and get zero scales)
   constexpr uint32_t CB = FMT == RQ_Q8_0 ? 512u : 256u, RB = FMT == RQ_Q8_0 ? 32u : 16u;
   constexpr uint32_t HB = RB / 2;
-  // the tile's own groups: 32-bit offsets whatever the weight's size
+  // the tile's own groups: offsets that do not grow with the weight's rows
+  using Off = typename Src<WIDE>::Off;
   const int g0 = n0 / 16, g_last = min(G, npad / 16 - g0) - 1;
-  const __amdgpu_buffer_rsrc_t qr =
-      buffer_rsrc(q + (int64_t)g0 * nkb * CB, (uint32_t)(g_last + 1) * (uint32_t)nkb * CB);
-  const __amdgpu_buffer_rsrc_t sr =
-      buffer_rsrc(sc + (int64_t)g0 * nkb * 16, (uint32_t)(g_last + 1) * (uint32_t)nkb * 16 * (uint32_t)sizeof(ST));
+  const Src<WIDE> qs(q + (int64_t)g0 * nkb * CB, (int64_t)(g_last + 1) * nkb * CB);
+  const Src<WIDE> ss(sc + (int64_t)g0 * nkb * 16, (int64_t)(g_last + 1) * nkb * 16 * (int)sizeof(ST));
   const int tr = tid & 15, th = (tid >> 4) & 1;
   u32x4 raw[NT];
   uint32_t rs[NS];
@@ -170,13 +208,13 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
 #pragma unroll
     for (int i = 0; i < NT; i++) {
       const int u = (tid + T * i) >> 5, b = u % NB, k = u / NB % KG;
-      const uint32_t grp = (uint32_t)min(u / NB / KG, g_last);
-      const uint32_t kb = (uint32_t)min((turn * KG + k) * NB + b, nkb - 1);
-      const uint32_t off = (grp * (uint32_t)nkb + kb) * CB + (uint32_t)tr * RB + (uint32_t)th * HB;
+      const Off grp = (Off)min(u / NB / KG, g_last);
+      const Off kb = (Off)min((turn * KG + k) * NB + b, nkb - 1);
+      const Off off = (grp * (Off)nkb + kb) * CB + (Off)tr * RB + (Off)th * HB;
       if (FMT == RQ_Q8_0) {
-        raw[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(qr, (int)off, 0, 0));
+        raw[i] = qs.b128(off, 0);
       } else {
-        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(qr, (int)off, 0, 0));
+        const u32x2 v = qs.b64(off, 0);
         raw[i] = u32x4{v[0], v[1], 0u, 0u};
       }
     }
@@ -184,13 +222,10 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
     for (int i = 0; i < NS; i++) {
       // scale t = tid + T i: row t % 16 of block t / 16 % NB, kg, group as above
       const int t = tid + T * i, b = (t >> 4) % NB, k = (t >> 4) / NB % KG;
-      const uint32_t grp = (uint32_t)min((t >> 4) / NB / KG, g_last);
+      const Off grp = (Off)min((t >> 4) / NB / KG, g_last);
       const int kb = (turn * KG + k) * NB + b;
-      const uint32_t off = ((grp * (uint32_t)nkb + (uint32_t)min(kb, nkb - 1)) * 16 + (uint32_t)(t & 15)) * sizeof(ST);
-      if (sizeof(ST) == 4)
-        rs[i] = __builtin_amdgcn_raw_buffer_load_b32(sr, (int)off, 0, 0);
-      else
-        rs[i] = __builtin_amdgcn_raw_buffer_load_b16(sr, (int)off, 0, 0);
+      const Off off = ((grp * (Off)nkb + (Off)min(kb, nkb - 1)) * 16 + (Off)(t & 15)) * sizeof(ST);
+      rs[i] = sizeof(ST) == 4 ? ss.b32(off, 0) : ss.b16(off, 0);
       if (kb >= nkb) rs[i] = 0u;
     }
   };
@@ -232,32 +267,27 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
 
   // ---- this wave's activation fragments: rows m0 + 32 f + lane % 32
   const int r32_last = (M + 31) / 32 - 1;
-  const uint32_t xs_base = (uint32_t)(r32_last + 1) * (uint32_t)nkb * 2048u;  // I8: the scales' region
-  uint32_t xo[MF], so[MF];
+  const Off xs_base = (Off)(r32_last + 1) * (Off)nkb * 2048u;  // I8: the scales' region
+  Off xo[MF], so[MF];
 #pragma unroll
   for (int f = 0; f < MF; f++) {
-    const uint32_t t32 = (uint32_t)min(m0 / 32 + f, r32_last);
-    xo[f] = PK ? t32 * (uint32_t)nkb * (1024u * AF) + 16u * (uint32_t)lane
-               : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
-    so[f] = xs_base + t32 * (uint32_t)(nkb + 1) * 128u + 16u * (uint32_t)g;
+    const Off t32 = (Off)min(m0 / 32 + f, r32_last);
+    xo[f] = PK ? t32 * (Off)nkb * (1024u * AF) + 16u * (Off)lane
+               : (Off)min(m0 + 32 * f + l32, M - 1) * (Off)nkb * 128u + 64u * (Off)g;
+    so[f] = xs_base + t32 * (Off)(nkb + 1) * 128u + 16u * (Off)g;
   }
   u32x4 a[2][MF][AF];     // PK: hi j 0, 1, f32: lo j 0, 1; else the 16 f32
   f32x4 xs[2][I8 ? MF : 1][4];  // I8: the scales of rows 8 q + 4 g + 0..3
   auto aload = [&](int slot, int kb) {
-    const ActBlock b = I8 ? act_block(x, x_bytes, min(kb, nkb - 1), nkb, 2048u)
-                          : act_block(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
+    const ActBlock<WIDE, I8> b(x, x_bytes, kb, nkb, PK ? 1024u * AF : 128u);
 #pragma unroll
     for (int f = 0; f < MF; f++) {
 #pragma unroll
-      for (int i = 0; i < AF; i++)
-        a[slot][f][i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)(xo[f] + (PK ? 1024u : 16u) * i), b.off, 0));
+      for (int i = 0; i < AF; i++) a[slot][f][i] = b.x.b128(xo[f] + (PK ? 1024u : 16u) * i, b.off);
       if (I8)
 #pragma unroll
         for (int i = 0; i < 4; i++)
-          xs[slot][f][i] = __builtin_bit_cast(
-              f32x4,
-              __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)(so[f] + 32u * i), (int)((uint32_t)min(kb, nkb) * 128u), 0));
+          xs[slot][f][i] = __builtin_bit_cast(f32x4, b.x.b128(so[f] + 32u * i, (Off)min(kb, nkb) * 128u));
     }
   };
 
@@ -582,13 +612,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
                  : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
     u32x4 a[RA][MF][4];
     auto aload = [&](int slot, int kb) {
-      const ActBlock b = act_block(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
+      const ActBlock<false, false> b(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
 #pragma unroll
       for (int f = 0; f < MF; f++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-          a[slot][f][i] = __builtin_bit_cast(
-              u32x4, __builtin_amdgcn_raw_buffer_load_b128(b.r, (int)(xo[f] + (PK ? 1024u : 16u) * i), b.off, 0));
+        for (int i = 0; i < 4; i++) a[slot][f][i] = b.x.b128(xo[f] + (PK ? 1024u : 16u) * i, b.off);
     };
     f32x16 p[PR];
 #pragma unroll
@@ -704,14 +732,14 @@ static hipError_t launch_rs_t(const MatmulArgs& a, const void* x, void* y, int64
   return hipGetLastError();
 }
 
-template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int WM, int KG>
+template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int WM, int KG, bool WIDE = false>
 static hipError_t launch_t(const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
                            hipEvent_t done) {
   constexpr int BM = 32 * MF * WM, BN = 32 * NF;
   const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
   if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
   const int64_t bytes = std::min<int64_t>(PK ? packed_bytes(XT, m, a.k) : m * a.k * 4, UINT32_MAX);
-  hipExtLaunchKernelGGL((gemm_blk_kernel<FMT, ST, XT, PK, MF, NF, WM, KG>), dim3((unsigned)(tiles_m * tiles_n)),
+  hipExtLaunchKernelGGL((gemm_blk_kernel<FMT, ST, XT, PK, WIDE, MF, NF, WM, KG>), dim3((unsigned)(tiles_m * tiles_n)),
                         dim3(64 * WM * KG), 0, a.stream, begin, done, 0, a.q, static_cast<const ST*>(a.scales), x, y,
                         (int)m, (int)a.k, (int)a.n, (int)a.npad, a.y_dtype, (int)tiles_m, (uint32_t)bytes);
   return hipGetLastError();
@@ -779,6 +807,14 @@ hipError_t launch_tile(int tile, const MatmulArgs& a, const void* x, void* y, in
   }
 }
 
+// Rows longer than this run the first tile with 64-bit addresses (WIDE): up to it the
+// weights of the widest tile (192 columns, 16 B of Q8_0 codes per row and 16
+// elements) and the least rows of packed int8 activations (32) stay within 32-bit
+// offsets
+constexpr int64_t kMaxK32 = (int64_t)1 << 24;
+static_assert(192 * kMaxK32 <= UINT32_MAX && 32 * (2 * kMaxK32 + (kMaxK32 / 32 + 1) * 4) <= UINT32_MAX,
+              "32-bit offsets");
+
 // Rows per launch: the packed copy within rq_qmatmul_noalloc's scratch, x within
 // the 32-bit buffer offsets
 int64_t chunk_rows(int64_t k, bool packed) {
@@ -801,8 +837,10 @@ size_t gemm_f32_pack_bytes(int64_t m, int64_t k) {
 template <int FMT, typename ST>
 static hipError_t launch_x(const MatmulArgs& a, int cu_count) {
   const bool pk = a.scratch != nullptr;
-  // of the whole call, whatever its chunks; a tile's weights within 32-bit offsets
-  const int tile = a.k > (int64_t)1 << 24 ? 0 : pick_tile(kF32Tiles, 5, a.m, a.k, a.n, cu_count);
+  if (a.k > kMaxK32)
+    return launch_t<FMT, ST, RQ_F32, false, 1, 1, 1, 4, true>(a, a.x, a.y, a.m, a.ev_main[0], a.ev_main[1]);
+  // of the whole call, whatever its chunks
+  const int tile = pick_tile(kF32Tiles, 5, a.m, a.k, a.n, cu_count);
   const int64_t chunk = chunk_rows(a.k, pk);
   for (int64_t m0 = 0; m0 < a.m; m0 += chunk) {
     const int64_t m = std::min(chunk, a.m - m0);
@@ -826,7 +864,7 @@ static hipError_t launch_x(const MatmulArgs& a, int cu_count) {
 template <int FMT, typename ST>
 static hipError_t launch_i8(const MatmulArgs& a, int cu_count) {
   const int64_t chunk = i8_chunk_rows(a.k), nb = a.k / 32;
-  const int tile = a.k > (int64_t)1 << 24 ? 0 : pick_tile(kI8Tiles, 3, a.m, a.k, a.n, cu_count);
+  const int tile = a.k > kMaxK32 ? -1 : pick_tile(kI8Tiles, 3, a.m, a.k, a.n, cu_count);
   for (int64_t m0 = 0; m0 < a.m; m0 += chunk) {
     const int64_t m = std::min(chunk, a.m - m0);
     void* y = static_cast<uint8_t*>(a.y) + m0 * a.n * (a.y_dtype == RQ_F32 ? 4 : 2);
@@ -837,7 +875,8 @@ static hipError_t launch_i8(const MatmulArgs& a, int cu_count) {
     if (hipError_t e = hipGetLastError()) return e;
     const hipEvent_t done = m0 + chunk >= a.m ? a.ev_main[1] : nullptr;
     const hipError_t e =
-        tile == 0   ? launch_t<FMT, ST, kXtI8, true, 1, 1, 1, 4>(a, a.scratch, y, m, nullptr, done)
+        tile < 0    ? launch_t<FMT, ST, kXtI8, true, 1, 1, 1, 4, true>(a, a.scratch, y, m, nullptr, done)
+        : tile == 0 ? launch_t<FMT, ST, kXtI8, true, 1, 1, 1, 4>(a, a.scratch, y, m, nullptr, done)
         : tile == 1 ? launch_rs_t<FMT, ST, kXtI8, true, 1, 2, 4>(a, a.scratch, y, m, nullptr, done)
                     : launch_rs_t<FMT, ST, kXtI8, true, 1, 4, 4>(a, a.scratch, y, m, nullptr, done);
     if (e != hipSuccess) return e;

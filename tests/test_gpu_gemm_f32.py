@@ -142,3 +142,29 @@ def test_gemm_f32_overflowing_tail(torch, m, out, in_):
             torch.cuda.synchronize()
             assert bool(torch.isfinite(got[:3]).all()) and bool((got[3:] == float("inf")).all())
         w.destroy()
+
+
+@pytest.mark.parametrize("fmt,out,in_", [("q4h", 40, 2 ** 24 + 96), ("q4f", 3, 2 ** 24 + 32), ("q8", 1, 2 ** 28)])
+def test_gemm_f32_long_rows(torch, ctx, fmt, out, in_):
+    """Rows whose weights or activations pass 32-bit offsets (16 padded rows of 2^28
+    codes are 4 GiB): x and codes of -1, 0 and 1, so that y is an exact integer."""
+    import raster_amd
+
+    m = 17
+    print(f"[gpu] f32 GEMM long rows {fmt} {out}x{in_}", flush=True)
+    rng = np.random.default_rng(in_)
+    scales = np.ones(out * in_ // 32, np.float16 if fmt == "q4h" else np.float32)
+    if fmt == "q8":
+        w = raster_amd.QWeight.q8(rng.integers(-1, 2, out * in_, dtype=np.int8), scales, out, in_, ctx)
+    else:
+        nib = rng.integers(7, 10, out * in_ // 2, dtype=np.uint8)
+        w = raster_amd.QWeight.q4(nib | (rng.integers(7, 10, out * in_ // 2, dtype=np.uint8) << 4), scales, out, in_,
+                                  ctx)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randint(-1, 2, (m, in_), generator=g, device="cuda", dtype=torch.int8).float()
+    y = w.matmul(x)
+    W = w.dequant()
+    w.destroy()
+    for o in range(out):
+        for t in (0, 7, 16):
+            assert float(y[t, o]) == float((x[t] * W[o]).sum(dtype=torch.float64)), (t, o)

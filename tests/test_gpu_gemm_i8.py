@@ -53,3 +53,32 @@ def test_gemm_i8_infinite_tail_scale(torch, ctx, m, out, in_):  # noqa: F811
     y = w.matmul_i8(xq, xs, xsum)
     w.destroy()
     assert bool(torch.isfinite(y[:3]).all()) and bool((y[3:] == float("inf")).all())
+
+
+@pytest.mark.parametrize("fmt,out,in_", [("q4f", 35, 2 ** 24 + 96), ("q8", 1, 2 ** 26)])
+def test_gemm_i8_long_rows(torch, ctx, fmt, out, in_):  # noqa: F811
+    """Rows whose packed activations pass 32-bit offsets (2^26: 4 GiB of codes, then
+    their scales): codes of -1, 0 and 1 and scales of 1 and 2, y an exact integer."""
+    import raster_amd
+
+    m = 17
+    print(f"[gpu] int8 GEMM long rows {fmt} {out}x{in_}", flush=True)
+    rng = np.random.default_rng(in_)
+    scales = np.ones(out * in_ // 32, np.float32)
+    if fmt == "q8":
+        w = raster_amd.QWeight.q8(rng.integers(-1, 2, out * in_, dtype=np.int8), scales, out, in_, ctx)
+    else:
+        nib = rng.integers(7, 10, out * in_ // 2, dtype=np.uint8)
+        w = raster_amd.QWeight.q4(nib | (rng.integers(7, 10, out * in_ // 2, dtype=np.uint8) << 4), scales, out, in_,
+                                  ctx)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    xq = torch.randint(-1, 2, (m, in_), generator=g, device="cuda", dtype=torch.int8)
+    xs = torch.randint(1, 3, (m, in_ // 32), generator=g, device="cuda").float()
+    xsum = xq.view(m, -1, 32).sum(2, dtype=torch.int32)
+    y = w.matmul_i8(xq, xs, xsum)
+    W = w.dequant()
+    w.destroy()
+    for t in (0, 7, 16):
+        x = (xq[t].view(-1, 32).float() * xs[t].view(-1, 1)).view(-1)
+        for o in range(out):
+            assert float(y[t, o]) == float((x * W[o]).sum(dtype=torch.float64)), (t, o)
