@@ -222,17 +222,17 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    m <= 8); the MFMA decode kernel when a slice of x would not fit two
  *    workgroups' LDS, and further until the grid covers about 85% of the CUs,
  *    rounded up to a power of two while each slice keeps 8 blocks (at most
- *    in / 32 slices; a call at m <= 8, or with Q8_0 and n * in above 32 Mi,
- *    that cannot have them or needs more than RQ_NOALLOC_SCRATCH_MAX runs the
- *    int8-level kernel, except Q4_0 at m >= 5);
- *    the weight-stream GEMM (bf16 x, 16 < m <= 64) on a
- *    thin grid (up to 8 slices);
+ *    in / 32 slices; Q4_0 at m <= 4, and Q8_0 at m <= 8 or with n * in above
+ *    32 Mi, grow it under capture too, and where they cannot have it (device
+ *    memory full, rq_qmatmul_noalloc past RQ_NOALLOC_SCRATCH_MAX) take the
+ *    slices one after another, slower, with the same results); the
+ *    weight-stream GEMM (bf16 x, 16 < m <= 64) on a thin grid (up to 8 slices);
  *  - Q4_K / Q6_K: the q8_K activations, m * (in + in/256*4 + in/sub*4)
  *    bytes (each part rounded up to 256), sub = 32 for Q4_K, 16 for Q6_K.
- * Under HIP graph capture nothing can be allocated: run the same (or a
+ * Under HIP graph capture nothing else can be allocated: run the same (or a
  * larger) shape once on the capturing stream before capturing, otherwise the
  * call fails with RQ_ERR_SHAPE and a message saying so (except f32 x with
- * m > 16 and the MFMA decode calls that fall back, as above). A buffer that grows is
+ * m > 16, as above). A buffer that grows is
  * replaced but not freed until rq_ctx_destroy, so a graph captured before a
  * larger call still replays on its own (still allocated) buffers; graphs and
  * eager calls on one stream share a buffer only while it has not grown, and
@@ -249,12 +249,13 @@ int rq_qmatmul(rq_ctx ctx, rq_weight w, const void* x, int x_dtype, void* y, int
  * graph capture, tight serving loops, harnesses that forbid hipMalloc). Same
  * arguments, kernels and results as rq_qmatmul, bit for bit; no kernel-timing
  * events are recorded. Where rq_qmatmul would use per-stream scratch (the
- * packed activations of the bf16 GEMM, K-slice partial sums, a K-quant
+ * packed activations of the bf16 and f32 GEMMs, K-slice partial sums, a K-quant
  * weight's q8_K activations) this call uses a
  * fixed device array of RQ_NOALLOC_SCRATCH_MAX bytes that each GPU holds from
  * the first context created on it until the process ends; a call that needs
  * more fails with RQ_ERR_SHAPE and a message saying so (for example bf16 x
- * with m * in above 16 Mi elements). Every call on one GPU shares that GPU's
+ * with m * in above 16 Mi elements; the calls that rq_qmatmul's notes let do
+ * without scratch run without it). Every call on one GPU shares that GPU's
  * array, whatever its context or stream: calls that may overlap on one GPU
  * (different streams, or different host threads) race and must be ordered
  * by the caller. Nothing in the array needs to start at zero: each call

@@ -232,12 +232,23 @@ static int stream_pack(Ctx* c, hipStream_t stream, size_t bytes, void** out) {
   return RQ_OK;
 }
 
-// The K-split partial sums for `stream`: `part_bytes` (grow-only).
-static int stream_split(Ctx* c, hipStream_t stream, size_t part_bytes, float** part) {
+// This thread may allocate while a stream is being captured.
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  bool on = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
+  ~RelaxedCapture() {
+    if (on) (void)hipThreadExchangeStreamCaptureMode(&mode);
+  }
+};
+
+// The K-split partial sums for `stream`: `part_bytes` (grow-only), grown under
+// capture only where the call asks for it.
+static int stream_split(Ctx* c, hipStream_t stream, size_t part_bytes, float** part, bool captured = false) {
   std::lock_guard<std::mutex> lk(g_mu);
   auto& e = c->scratch[stream];
   if (e.red_bytes < part_bytes) {
-    if (capturing(stream)) return fail(RQ_ERR_SHAPE, kCaptureScratch);
+    if (!captured && capturing(stream)) return fail(RQ_ERR_SHAPE, kCaptureScratch);
+    const RelaxedCapture relaxed;
     if (int s = regrow(c, part_bytes, &e.red, &e.red_bytes)) return s;
   }
   *part = static_cast<float*>(e.red);
@@ -784,7 +795,8 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
 
 // A scratch region of `bytes` for one call: from the fixed scratch when the
 // call allocates nothing, else the stream's grow-only buffer (`which` 0: the
-// packed activations, 1: the K-slices' partial sums).
+// packed activations, 1: the K-slices' partial sums, 2: those, also grown while the
+// stream is being captured).
 static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t bytes, int which, void** out) {
   if (fixed) {
     const size_t at = align256(fixed->used);
@@ -797,7 +809,7 @@ static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t 
   }
   if (which == 0) return stream_pack(c, stream, bytes, out);
   float* p = nullptr;
-  const int s = stream_split(c, stream, bytes, &p);
+  const int s = stream_split(c, stream, bytes, &p, which == 2);
   *out = p;
   return s;
 }
@@ -905,11 +917,7 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   a.part = nullptr;
   a.ops = dops;
   const bool plain = !dops.norm_gain && !dops.residual && !dops.swiglu && !dops.act_i8;
-  MfPlan mf = plain && plan.ok ? plan_gemv_mf(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : MfPlan{};
-  const size_t mf_bytes = mf.ok && mf.ks > 1 ? (size_t)mf.ks * (size_t)m * (size_t)w.out * 4 : 0;
-  // a call that rq_qmatmul_noalloc could not give its scratch takes the
-  // int8-level kernel in rq_qmatmul too: the two give the same bits
-  if (!mf.always && mf_bytes > kNoAllocScratchBytes) mf.ok = false;
+  const MfPlan mf = plain && plan.ok ? plan_gemv_mf(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : MfPlan{};
   // the m = 1 GEMV also quantizes to int8 blocks itself (act_i8)
   const bool plain_g1 = !dops.norm_gain && !dops.residual && !dops.swiglu;
   const G1Plan g1 = plain_g1 && plan.ok ? plan_gemv1(m, w.in, w.npad, x_dtype, w.format, c->cu_count) : G1Plan{};
@@ -922,14 +930,12 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   if (g1.ok) {
     // the m = 1 GEMV uses no scratch
   } else if (mf.ok && mf.ks > 1) {
-    if (int s = call_scratch(c, fixed, a.stream, mf_bytes, 1, &part)) {
-      // without scratch (captured before it was grown, memory full): the
-      // int8-level kernel, which needs less of it or none
-      if (mf.always) return s;
-      mf.ok = false;
-    }
-  }
-  if (g1.ok || mf.ok) {
+    // calls that must not fail for want of scratch: grown under capture too, and without
+    // it (memory full, past the fixed scratch) the slices one after another, same bits
+    if (int s = call_scratch(c, fixed, a.stream, (size_t)mf.ks * (size_t)m * (size_t)w.out * 4, mf.scratch ? 1 : 2, &part))
+      if (mf.scratch) return s;
+  } else if (mf.ok) {
+    // one slice: no partial sums
   } else if (plan.ok && plan.ksplit > 1) {
     if (int s = call_scratch(c, fixed, a.stream, plan.part_bytes, 1, &part)) return s;
   } else if (!plan.ok && x_dtype == RQ_BF16 && wide.ok) {
@@ -960,7 +966,7 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
   a.part = static_cast<float*>(part);
   // no timing events for calls that allocate nothing (creating one allocates);
   // calls whose partial sums a second kernel adds time both kernels
-  const bool two = (mf.ok && mf.ks > 1) || (!mf.ok && !g1.ok && plan.ok && plan.ksplit > 1) || a.slices > 1;
+  const bool two = (mf.ok && part) || (!mf.ok && !g1.ok && plan.ok && plan.ksplit > 1) || a.slices > 1;
   const EvSet ev = fixed ? EvSet{} : timing_set(c, a.stream, two);
   a.ev_main[0] = ev.e[0];
   a.ev_main[1] = ev.e[1];

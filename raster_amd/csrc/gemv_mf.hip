@@ -32,7 +32,8 @@
 //   chunks are broadcast the same way.
 //   The KW waves of a column split the slice's steps and add their partial
 //   sums through LDS in wave order; with ks > 1 the slices' partial sums go
-//   to `part` and gemm_sm_reduce_kernel adds them in slice order.
+//   to `part` and gemm_sm_reduce_kernel adds them in slice order (or, without
+//   scratch, one workgroup takes the slices in that order: gemv_mf_seq_kernel).
 //   Deterministic either way.
 #include <algorithm>
 #include <atomic>
@@ -124,17 +125,17 @@ __host__ __device__ inline int mf_lds_bytes(int m, int spl, int parts, int kw, i
   return spl * parts * m * 64 + spl * 64 + 16 + (kw > 1 ? 2 * gw * kw * 1024 : 0);
 }
 
-template <int FMT, typename ST, int XT, int KW, int GW, int WD>
-__global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __restrict__ q,
-                                                               const ST* __restrict__ sc,
-                                                               const void* __restrict__ x, void* __restrict__ y,
-                                                               float* __restrict__ part, int M, int K, int N,
-                                                               int npad, int y_dtype, int ks) {
+// K-slice s of the workgroup's column col of gcols. SEQ: the workgroup takes every
+// slice itself (one unit per wave) and adds this one to sum.
+template <int FMT, typename ST, int XT, int KW, int GW, int WD, bool SEQ>
+__device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST* __restrict__ sc,
+                                         const void* __restrict__ x, void* __restrict__ y, float* __restrict__ part,
+                                         int M, int K, int N, int npad, int y_dtype, int ks, int s, int col, int gcols,
+                                         f32x4& sum) {
   constexpr int WAVES = KW * GW, P = XT == RQ_F32 ? 2 : 1;
   constexpr float OFF = FMT == RQ_Q8_0 ? 128.0f : 136.0f;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int nkb = K / 32, ngroups = npad / 16;
-  const int s = (int)blockIdx.x % ks, col = (int)blockIdx.x / ks, gcols = (int)gridDim.x / ks;
   const int spl = (nkb + ks - 1) / ks;
   const int kb0 = min(nkb, s * spl), nst = min(nkb, kb0 + spl) - kb0;  // this slice: steps kb0 .. kb0+nst-1
   const int xs_off = spl * P * M * 64, flag_off = xs_off + spl * 64, red_off = flag_off + 16;
@@ -239,7 +240,6 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
   const int spw = (nst + KW - 1) / KW;
   const int spp = (spw + WD - 1) / WD * WD;
   const int nunits = (ngroups + gcols * GW - 1) / (gcols * GW);
-  const int T = nunits * spp;
   static_assert(WD % 4 == 0, "the Q4_0 ring holds whole quads");
   MfCodes<ST> wc[FMT == RQ_Q4_0 ? 1 : WD];
   MfQuad<ST> wq[FMT == RQ_Q4_0 ? WD / 4 : 1];
@@ -353,6 +353,16 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
 
   f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
   auto store = [&](int j, const f32x4& v) {
+    if constexpr (SEQ) {
+      // as gemm_sm_reduce_kernel adds the slices
+#pragma clang fp contract(off)
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const float ve = v[e] * ysc[e];
+        sum[e] = s == 0 ? ve : sum[e] + ve;
+      }
+      return;
+    }
     const int g = col * GW + gw + j * gcols * GW;
     const int o = 16 * g + r;
     if (g >= ngroups || o >= N) return;
@@ -485,17 +495,62 @@ __global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __
   }
 }
 
+template <int FMT, typename ST, int XT, int KW, int GW, int WD>
+__global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __restrict__ q,
+                                                               const ST* __restrict__ sc,
+                                                               const void* __restrict__ x, void* __restrict__ y,
+                                                               float* __restrict__ part, int M, int K, int N,
+                                                               int npad, int y_dtype, int ks) {
+  f32x4 none;
+  mf_slice<FMT, ST, XT, KW, GW, WD, false>(q, sc, x, y, part, M, K, N, npad, y_dtype, ks, (int)blockIdx.x % ks,
+                                           (int)blockIdx.x / ks, (int)gridDim.x / ks, none);
+}
+
+// For a call without scratch for the slices' sums: a workgroup takes the slices of
+// its column one after another and adds them as the reduction does, so the bits are
+// the same. It has fewer waves in flight (us, against slices side by side: Q8_0
+// 4096 x 4096 m = 8 41.6 / 11.0, 14336 x 4096 m = 8 36.1 / 22.5, Q4_0 4096 x 14336
+// m = 4 72 / 15.4; 1, 2 and 16 waves per workgroup there 103, 82, 125).
+constexpr int kSeqWaves = 4;
+template <int FMT, typename ST, int XT, int WD>
+__global__ __launch_bounds__(64 * kSeqWaves) void gemv_mf_seq_kernel(const uint8_t* __restrict__ q,
+                                                                     const ST* __restrict__ sc,
+                                                                     const void* __restrict__ x, void* __restrict__ y,
+                                                                     int M, int K, int N, int npad, int y_dtype,
+                                                                     int ks) {
+  f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < ks; s++) {
+    if (s > 0) __syncthreads();  // the slice before has been read
+    mf_slice<FMT, ST, XT, 1, kSeqWaves, WD, true>(q, sc, x, y, nullptr, M, K, N, npad, y_dtype, ks, s,
+                                                  (int)blockIdx.x, (int)gridDim.x, sum);
+  }
+  const int lane = threadIdx.x & 63, o = 16 * ((int)blockIdx.x * kSeqWaves + (int)(threadIdx.x >> 6)) + (lane & 15);
+  if (o >= N) return;
+#pragma unroll
+  for (int e = 0; e < 4; e++) {
+    const int m = 4 * (lane >> 4) + e;
+    if (m >= M) break;
+    if (y_dtype == RQ_F32)
+      static_cast<float*>(y)[(int64_t)m * N + o] = sum[e];
+    else
+      static_cast<uint16_t*>(y)[(int64_t)m * N + o] = (uint16_t)f32_to_bf16_bits(sum[e]);
+  }
+}
+
 hipError_t launch_split_reduce(const float* part, void* y, int64_t n, int ks, int y_dtype, hipStream_t stream,
                                hipEvent_t start, hipEvent_t stop);
 
-// One configuration: ks K-slices, gcols workgroup columns per slice.
+// One configuration: ks K-slices, gcols workgroup columns per slice; without a.part
+// the slices one after another.
 template <int FMT, typename ST, int XT, int KW, int GW, int WD>
 hipError_t launch_gemv_mf_t(const MatmulArgs& a, int ks, int gcols) {
   constexpr int P = XT == RQ_F32 ? 2 : 1;
   auto kernel = &gemv_mf_kernel<FMT, ST, XT, KW, GW, WD>;
+  auto seq_kernel = &gemv_mf_seq_kernel<FMT, ST, XT, WD>;
+  const bool seq = ks > 1 && !a.part;
   const int nkb = (int)(a.k / 32);
   if (ks < 1 || ks > nkb || gcols < 1 || a.m < 1 || a.m > 16) return hipErrorInvalidValue;
-  if (ks > 1 && !a.part) return hipErrorInvalidValue;
+  if (seq && KW != 1) return hipErrorInvalidValue;
   const int spl = (nkb + ks - 1) / ks;
   if ((int64_t)(ks - 1) * spl >= nkb) return hipErrorInvalidValue;  // every slice holds steps
   const int lds = mf_lds_bytes((int)a.m, spl, P, KW, GW);
@@ -506,10 +561,16 @@ hipError_t launch_gemv_mf_t(const MatmulArgs& a, int ks, int gcols) {
   if (hipError_t e = hipGetDevice(&dev)) return e;
   const uint64_t bit = uint64_t(1) << (dev & 63);
   if (!(attr_set.load(std::memory_order_acquire) & bit)) {
-    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, 163840);
-    if (e != hipSuccess) return e;
+    for (const void* f : {reinterpret_cast<const void*>(kernel), reinterpret_cast<const void*>(seq_kernel)})
+      if (hipError_t e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 163840)) return e;
     attr_set.fetch_or(bit, std::memory_order_acq_rel);
+  }
+  if (seq) {
+    const int64_t wg = (a.npad / 16 + kSeqWaves - 1) / kSeqWaves;  // a group per wave
+    hipExtLaunchKernelGGL(seq_kernel, dim3((unsigned)wg), dim3(64 * kSeqWaves), (unsigned)lds, a.stream, a.ev_main[0],
+                          a.ev_main[1], 0, a.q, static_cast<const ST*>(a.scales), a.x, a.y, (int)a.m, (int)a.k,
+                          (int)a.n, (int)a.npad, a.y_dtype, ks);
+    return hipGetLastError();
   }
   hipExtLaunchKernelGGL(kernel, dim3((unsigned)(gcols * ks)), dim3(64 * KW * GW), (unsigned)lds, a.stream,
                         a.ev_main[0], a.ev_main[1], 0, a.q, static_cast<const ST*>(a.scales),
@@ -588,7 +649,7 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
   ks = kf;
   p.ks = (int)ks;
   if ((int64_t)p.gcols * ks > INT32_MAX) return p;
-  p.always = format == RQ_Q4_0 ? m >= 5 : m >= 9 && npad * k <= (int64_t(32) << 20);
+  p.scratch = format == RQ_Q4_0 ? m >= 5 : m >= 9 && npad * k <= (int64_t(32) << 20);
   p.ok = true;
   return p;
 }

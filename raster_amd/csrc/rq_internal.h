@@ -146,7 +146,9 @@ hipError_t launch_bias_rows(const float* b, float* y, int64_t rows, int64_t cols
 
 struct MfPlan {
   bool ok;
-  bool always;  // no falling back to the int8-level kernel where its scratch cannot be had
+  // a call whose slices' scratch cannot be had fails; else (calls that an int8-level
+  // kernel without scratch could serve) it runs without, slower
+  bool scratch;
   int kw, gw, wd, ks, gcols;
 };
 MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format, int cu_count);

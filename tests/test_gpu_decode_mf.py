@@ -232,37 +232,36 @@ def test_mf_lines_and_large_values(torch, ctx, orc, fmt, m, out, in_, kernel, xd
         assert np.all(np.abs(y - ref) <= lvl)
 
 
-@pytest.mark.parametrize("fmt,m,out,in_", [("q4", 4, 2048, 5632), ("q8", 6, 1024, 4096)])
-def test_mf_without_scratch(torch, orc, fmt, m, out, in_):
-    """A first call under graph capture cannot have the K-slices' scratch and
-    runs the int8-level kernel: every replay inside that kernel's bound, and the
-    same bits each time."""
+@pytest.mark.parametrize("fmt,m,out,in_,xdt,ydt", [("q4", 4, 2048, 5632, "f32", "f32"), ("q4f", 2, 300, 8224, "f32", "bf16"),
+                                                   ("q4", 3, 2801, 5632, "bf16", "f32"), ("q8", 6, 1024, 4096, "f32", "f32"),
+                                                   ("q8", 5, 37, 14336, "bf16", "bf16"), ("q8", 16, 6200, 8192, "f32", "bf16"),
+                                                   ("q8", 8, 1500, 3104, "f32", "f32")])
+def test_mf_captured_first(torch, orc, fmt, m, out, in_, xdt, ydt):
+    """A first call under graph capture grows the K-slices' scratch there: the bits of
+    the eager call on every replay (a row of 2^112 and more among them)."""
     import raster_amd
 
-    note(f"mf captured first {fmt} m={m} {out}x{in_}")
+    note(f"mf captured first {fmt} m={m} {out}x{in_} {xdt} {ydt}")
     with raster_amd.Context(0) as c:
         w, dense, s, off = make(raster_amd, c, orc, fmt, out, in_, seed=out)
-        x = wl.activations(m, in_, seed=m).reshape(m, in_).copy()
-        xt = torch.from_numpy(x).cuda()
-        y = torch.empty((m, out), device="cuda")
+        x = wl.activations(m, in_, seed=m, dtype=xdt).reshape(m, in_).copy()
+        x[m - 1, in_ // 2:] *= 2.0 ** 117
+        xt = torch.from_numpy(x).cuda().to(torch.bfloat16 if xdt == "bf16" else torch.float32)
+        y = torch.empty((m, out), device="cuda", dtype=torch.bfloat16 if ydt == "bf16" else torch.float32)
         st = torch.cuda.Stream()
         torch.cuda.synchronize()
         g = torch.cuda.CUDAGraph()
         with torch.cuda.graph(g, stream=st):
             w.matmul(xt, y=y)
-        ref = x.astype(np.float64) @ dense.astype(np.float64).T
-        bmax = np.repeat(np.abs(x.astype(np.float64)).reshape(m, -1, 32).max(axis=2), 32, axis=1)
-        lvl = 2.0 ** -15 * (bmax @ np.abs(dense.astype(np.float64)).T)
-        lvl += 2.0 ** -20 * (np.abs(x.astype(np.float64)) @ np.abs(dense.astype(np.float64)).T)
-        first = None
+        eager = w.matmul(xt, out_dtype=y.dtype)
+        if ydt == "f32":
+            ref = x.astype(np.float64) @ dense.astype(np.float64).T
+            assert np.all(np.abs(eager.cpu().numpy() - ref) <= mf_bound(x, dense, s, off))
         for i in range(3):
             y.fill_(float("nan"))
             g.replay()
             torch.cuda.synchronize()
-            got = y.cpu().numpy()
-            assert np.all(np.abs(got - ref) <= lvl)
-            first = got if first is None else first
-            assert np.array_equal(got, first)
+            assert torch.equal(y, eager)
             w.matmul(xt * (i + 2))
         torch.cuda.synchronize()
         w.destroy()

@@ -163,3 +163,24 @@ def test_noalloc_sweep(torch, ctx, i, m, in_, out, fmt, xdt, ydt):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     finally:
         w.destroy()
+
+
+def test_noalloc_slices_past_the_fixed_scratch(torch, ctx):
+    """A decode call whose K-slices' partial sums pass the fixed scratch (32 slices of 4 x
+    65552 f32: 32.008 MiB): one workgroup takes a column's slices one after another,
+    bit for bit what rq_qmatmul adds from its own, larger scratch."""
+    import raster_amd
+
+    out, in_, m = 65552, 72736, 4
+    rng = np.random.default_rng(1)
+    packed = np.resize(rng.integers(0, 256, 10007 * 1009, dtype=np.uint8), out * in_ // 2)
+    scales = np.resize(rng.uniform(0.002, 0.02, 100003).astype(np.float16), out * in_ // 32)
+    w = raster_amd.QWeight.q4(packed, scales, out, in_, ctx)
+    del packed, scales
+    try:
+        for xdt, ydt, rows in (("f32", "f32", m), ("f32", "bf16", m)):
+            note(f"noalloc q4 {out}x{in_} m={rows} x={xdt} y={ydt}")
+            a, b = both(torch, ctx, w, rows, xdt, ydt, seed=rows)
+            assert np.all(np.isfinite(a)) and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    finally:
+        w.destroy()
