@@ -621,6 +621,12 @@ static bool mf_takes(int64_t m, int64_t k, int64_t npad, int format) {
 // enough workgroups for ~85% of the CUs (slices of at least 8 steps): at
 // K = 4096, m = 16 both give 4 (18 us, against 20 at ks = 2 and 22 at 8); at
 // m = 6 the LDS alone would allow 2 (23.3 us against 16.3 at 4).
+// Q8_0: the most slices that stay within the rounds of the CUs that the LDS's number
+// takes. Measured, f32 x, us at this number (and at the rule above's, which left a
+// second round part empty): 5632 x 2048 m = 9 / 16 5 slices 9.8 / 10.6 (8: 15.6 /
+// 16.3), 11264 x 2048 m = 9 2 14.1 (4: 16.9), 10240 x 3072 m = 8 3 14.3 (4: 22.3),
+// 11008 x 4096 m = 8 2 21.4 (4: 24.3), 10000 x 5120 m = 8 3 21.3 (4: 30.0), in two
+// rounds 8192 x 8192 m = 16 8 27.8 (the LDS's 7: 32.8); 4096 x 4096 8 10.5 by both.
 MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format, int cu_count) {
   MfPlan p{};
   if (m < 2 || m > 16 || (x_dtype != RQ_F32 && x_dtype != RQ_BF16) || k % 32 != 0 || k < 32) return p;
@@ -636,6 +642,16 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
     if (++ks > nkb) return p;
   }
   p.gcols = (int)((ngroups + p.gw - 1) / p.gw);
+  if (format == RQ_Q8_0) {
+    const int64_t cu = std::max(cu_count, 1), rounds = (p.gcols * ks + cu - 1) / cu;
+    int64_t n = std::max(ks, std::min(rounds * cu / p.gcols, nkb / 8));
+    while (n > ks && (n - 1) * ((nkb + n - 1) / n) >= nkb) --n;  // no empty slice
+    p.ks = (int)n;
+    if (p.gcols * n > INT32_MAX) return p;
+    p.scratch = m >= 9 && npad * k <= (int64_t(32) << 20);
+    p.ok = true;
+    return p;
+  }
   const int64_t fill = std::min<int64_t>(((int64_t)cu_count * 85 / 100 + p.gcols - 1) / p.gcols,
                                          std::max<int64_t>(1, nkb / 8));
   int64_t kf = std::max(ks, fill);
@@ -649,7 +665,7 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
   ks = kf;
   p.ks = (int)ks;
   if ((int64_t)p.gcols * ks > INT32_MAX) return p;
-  p.scratch = format == RQ_Q4_0 ? m >= 5 : m >= 9 && npad * k <= (int64_t(32) << 20);
+  p.scratch = m >= 5;
   p.ok = true;
   return p;
 }
