@@ -47,8 +47,11 @@ struct Ctx {
   std::unordered_set<void*> buffers;
   // Per-stream scratch, grow-only, freed with the context: packed
   // activations, and the K-split partial sums. Calls on one stream run in
-  // order, so a stream's buffers are never used by two kernels at once.
+  // order, so a stream's buffers are never used by two kernels at once; a call
+  // holds `enqueue` from taking a buffer to its last launch, so that two host
+  // threads' calls on one stream do not put their kernels between each other's.
   struct StreamScratch {
+    std::mutex enqueue;
     void* pack = nullptr;
     size_t pack_bytes = 0;
     void* red = nullptr;  // K-split partial sums
@@ -218,6 +221,18 @@ static int regrow(Ctx* c, size_t bytes, void** buf, size_t* have) {
   *buf = p;
   *have = want;
   return RQ_OK;
+}
+
+// Makes the call the only one to enqueue on `stream` with its scratch (taken before
+// g_mu, never under it).
+static void own_scratch(Ctx* c, hipStream_t stream, std::unique_lock<std::mutex>* own) {
+  if (own->owns_lock()) return;
+  std::mutex* m;
+  {
+    std::lock_guard<std::mutex> lk(g_mu);
+    m = &c->scratch[stream].enqueue;
+  }
+  *own = std::unique_lock<std::mutex>(*m);
 }
 
 // The bf16 GEMM's packed-activation buffer for `stream`, at least `bytes`.
@@ -796,8 +811,9 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
 // A scratch region of `bytes` for one call: from the fixed scratch when the
 // call allocates nothing, else the stream's grow-only buffer (`which` 0: the
 // packed activations, 1: the K-slices' partial sums, 2: those, also grown while the
-// stream is being captured).
-static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t bytes, int which, void** out) {
+// stream is being captured), which the call then owns.
+static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t bytes, int which, void** out,
+                        std::unique_lock<std::mutex>* own) {
   if (fixed) {
     const size_t at = align256(fixed->used);
     if (bytes > fixed->cap || at > fixed->cap - bytes)
@@ -807,6 +823,7 @@ static int call_scratch(Ctx* c, FixedScratch* fixed, hipStream_t stream, size_t 
     fixed->used = at + bytes;
     return RQ_OK;
   }
+  own_scratch(c, stream, own);
   if (which == 0) return stream_pack(c, stream, bytes, out);
   float* p = nullptr;
   const int s = stream_split(c, stream, bytes, &p, which == 2);
@@ -828,7 +845,8 @@ static int run_kquant_matmul(Ctx* c, const Weight& w, const float* x, void* y, i
   const size_t bs_b = (size_t)m * (size_t)(w.in / sub) * 4;
   if (int s = set_device(c)) return s;  // before the scratch: growing it allocates on this device
   void* buf = nullptr;
-  if (int s = call_scratch(c, fixed, stream, xq_b + xs_b + bs_b, 0, &buf)) return s;
+  std::unique_lock<std::mutex> own;
+  if (int s = call_scratch(c, fixed, stream, xq_b + xs_b + bs_b, 0, &buf, &own)) return s;
   int8_t* xq = static_cast<int8_t*>(buf);
   float* xs = reinterpret_cast<float*>(static_cast<uint8_t*>(buf) + xq_b);
   int32_t* bs = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(buf) + xq_b + xs_b);
@@ -927,41 +945,43 @@ static int run_matmul(Ctx* c, const Weight& w, const DecodePlan& plan, const voi
                             ? plan_gemm_wide(m, w.in, w.npad, c->cu_count)
                             : WidePlan{};
   void* part = nullptr;
+  std::unique_lock<std::mutex> own;
   if (g1.ok) {
     // the m = 1 GEMV uses no scratch
   } else if (mf.ok && mf.ks > 1) {
     // calls that must not fail for want of scratch: grown under capture too, and without
     // it (memory full, past the fixed scratch) the slices one after another, same bits
-    if (int s = call_scratch(c, fixed, a.stream, (size_t)mf.ks * (size_t)m * (size_t)w.out * 4, mf.scratch ? 1 : 2, &part))
+    if (int s = call_scratch(c, fixed, a.stream, (size_t)mf.ks * (size_t)m * (size_t)w.out * 4, mf.scratch ? 1 : 2, &part,
+                             &own))
       if (mf.scratch) return s;
   } else if (mf.ok) {
     // one slice: no partial sums
   } else if (plan.ok && plan.ksplit > 1) {
-    if (int s = call_scratch(c, fixed, a.stream, plan.part_bytes, 1, &part)) return s;
+    if (int s = call_scratch(c, fixed, a.stream, plan.part_bytes, 1, &part, &own)) return s;
   } else if (!plan.ok && x_dtype == RQ_BF16 && wide.ok) {
     // the 32x32x16 operand copy of x: ceil(m/32)*32 rows
-    if (int s = call_scratch(c, fixed, a.stream, pack_x32_bytes(m, w.in), 0, &a.scratch)) return s;
+    if (int s = call_scratch(c, fixed, a.stream, pack_x32_bytes(m, w.in), 0, &a.scratch, &own)) return s;
   } else if (!plan.ok && x_dtype == RQ_BF16 && gemm_sm_takes(w.format, m, w.in)) {
     // the weight-stream GEMM reads x as it is; K-slices' partial sums
     a.slices = gemm_sm_slices(w.format, m, w.in, w.npad, c->cu_count);
     if (a.slices > 1) {
-      if (int s = call_scratch(c, fixed, a.stream, (size_t)a.slices * (size_t)m * (size_t)w.out * 4, 1, &part))
+      if (int s = call_scratch(c, fixed, a.stream, (size_t)a.slices * (size_t)m * (size_t)w.out * 4, 1, &part, &own))
         return s;
     }
   } else if (!plan.ok && x_dtype == RQ_BF16) {
     // fragment-major copy of the activations: ceil(m/16)*16 rows (16x16x32
     // operands), or ceil(m/32)*32 rows for the 32x32x16 K-pair kernel
     const size_t bytes = std::max((size_t)((m + 15) / 16 * 16) * (size_t)w.in * 2, pack_x32_bytes(m, w.in));
-    if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch)) return s;
+    if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch, &own)) return s;
   } else if (!plan.ok && x_dtype == kXtI8) {
     // the int8 activations as bf16 fragments, with their scales
     const size_t bytes = gemm_i8_pack_bytes(m, w.in);
-    if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch)) return s;
+    if (int s = call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch, &own)) return s;
   } else if (!plan.ok) {
     // bf16 hi + lo copy of the f32 activations; a call that cannot have the
     // scratch (captured before it was grown, memory full) reads x itself
     const size_t bytes = gemm_f32_pack_bytes(m, w.in);
-    if (bytes == 0 || call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch) != RQ_OK) a.scratch = nullptr;
+    if (bytes == 0 || call_scratch(c, fixed, a.stream, bytes, 0, &a.scratch, &own) != RQ_OK) a.scratch = nullptr;
   }
   a.part = static_cast<float*>(part);
   // no timing events for calls that allocate nothing (creating one allocates);
@@ -1131,8 +1151,11 @@ int rq_decode_attention(rq_ctx h, const float* q, const float* k, const float* v
   if (int s = set_device(c)) return s;
   const AttnSplit sp = plan_decode_attention(pos, n_q, n_kv, head_dim, c->cu_count);
   void* scratch_buf = nullptr;
-  if (sp.nsplit > 1)
+  std::unique_lock<std::mutex> own;
+  if (sp.nsplit > 1) {
+    own_scratch(c, (hipStream_t)stream, &own);
     if (int s = stream_attn(c, (hipStream_t)stream, sp.scratch_bytes, &scratch_buf)) return s;
+  }
   hipError_t e = launch_decode_attention(q, k, v, kcache, vcache, pos, n_q, n_kv, head_dim, theta, scale, out, sp,
                                          scratch_buf, (hipStream_t)stream);
   if (e != hipSuccess) return hip_fail(e, "attention launch");
@@ -1195,6 +1218,8 @@ int rq_qmatmul_dx(rq_ctx h, rq_weight wh, const float* dy, float* dx, int64_t m,
   const int slices = mf ? dx_mf_slices(m, w.in, w.npad, c->cu_count) : dx_fm_slices(m, w.in, w.npad, c->cu_count);
   float* part = nullptr;
   void* pack = nullptr;
+  std::unique_lock<std::mutex> own;
+  if (slices > 1 || mf) own_scratch(c, st, &own);
   if (slices > 1) {
     if (int s = stream_split(c, st, (size_t)slices * (size_t)m * (size_t)w.in * 4, &part)) return s;
   }

@@ -16,7 +16,10 @@ graph, replays are idempotent and each op reads its own buffers
     still replays correctly (a grown buffer is retired, not freed);
   * two streams, and two host threads with a stream each, running split and
     GEMM calls of different shapes at once on one context: each result equals
-    its single-stream result bit for bit.
+    its single-stream result bit for bit;
+  * two host threads on one stream: calls of several kernels (packing + GEMM,
+    slices + reduction, ranges + merge) do not put their launches between each
+    other's, so every result equals the single-threaded one bit for bit.
 """
 import threading
 
@@ -270,4 +273,74 @@ def test_two_host_threads_at_once(torch, ctx):
         assert not errors, errors
     finally:
         for w, _, _ in cases:
+            w.destroy()
+
+
+def test_two_host_threads_on_one_stream(torch, ctx, orc):
+    import raster_amd
+
+    note("two host threads on one stream")
+    nq, nkv, hd, pos = 16, 4, 128, 3000
+    kvd = nkv * hd
+    w8, w4, wk = q8(raster_amd, ctx, 512, 2048, 61), q4(raster_amd, ctx, 256, 5632, 62), q4k(raster_amd, ctx, orc, 256, 1024, 63)
+    try:
+        s = torch.cuda.Stream()
+
+        def calls(seed):
+            g = torch.Generator(device="cuda").manual_seed(seed)
+            rnd = lambda *shape: torch.randn(shape, generator=g, device="cuda")  # noqa: E731
+            x1, x2, x3, x4, x5 = rnd(40, 2048), rnd(4, 5632), rnd(20, 1024), rnd(64, 512), rnd(12, 2048)
+            q, k, v = rnd(nq * hd), rnd(kvd), rnd(kvd)
+            kc, vc = rnd(pos + 1, kvd), rnd(pos + 1, kvd)
+            xq = raster_amd.quantize_act_i8(ctx, x1, 2048)
+            shapes = ((40, 512), (4, 256), (20, 256), (64, 2048), (12, 512), (40, 512), (nq * hd,))
+
+            def run(o):
+                w8.matmul(x1, y=o[0], stream=s)
+                w4.matmul(x2, y=o[1], stream=s)
+                wk.matmul(x3, y=o[2], stream=s)
+                w8.matmul_dx(x4, dx=o[3], stream=s)
+                w8.matmul(x5, y=o[4], stream=s)
+                w8.matmul_i8(*xq, y=o[5], stream=s)
+                raster_amd.decode_attention(ctx, q, k, v, kc, vc, pos, nq, nkv, hd, 1e4, hd ** -0.5, out=o[6], stream=s)
+
+            return run, shapes
+
+        reps, work = 60, []
+        for seed in (1, 2):
+            run, shapes = calls(seed)
+            work.append((run, [[torch.empty(sh, device="cuda") for sh in shapes] for _ in range(reps)]))
+        torch.cuda.synchronize()
+        refs = []
+        for run, outs in work:
+            run(outs[0])
+            torch.cuda.synchronize()
+            refs.append([t.clone() for t in outs[0]])
+            for o in outs:
+                for t in o:
+                    t.fill_(float("nan"))
+        torch.cuda.synchronize()
+        gate, errors = threading.Barrier(2), []
+
+        def worker(run, outs):
+            try:
+                gate.wait(timeout=30)
+                for o in outs:
+                    run(o)
+            except Exception as e:  # reported by the main thread
+                errors.append(repr(e))
+
+        threads = [threading.Thread(target=worker, args=a) for a in work]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join(timeout=90)
+        assert not any(t.is_alive() for t in threads) and not errors, errors
+        torch.cuda.synchronize()
+        for (_, outs), ref in zip(work, refs):
+            for r, o in enumerate(outs):
+                for i, (t, want) in enumerate(zip(o, ref)):
+                    assert torch.equal(t, want), (r, i)
+    finally:
+        for w in (w8, w4, wk):
             w.destroy()
