@@ -5,15 +5,15 @@
 //   rope-pos               raster/dl/attention.clj:197-214 (NeoX half split)
 //   kv-append!             raster/dl/attention.clj:413-416
 //   gqa-decode-attention   raster/dl/attention.clj:248-287
-// One workgroup per query head. It rotates its query and its KV head's new
-// key (angles pos * theta^(-2i/head_dim) in double, as the reference), takes
-// the scores of positions 0..pos (the new key from LDS, the older ones from
-// the cache), their softmax, and the weighted sum of values. The first query
-// head of each KV head writes the rotated key and the value into the caches
-// at row pos; no workgroup reads row pos from memory, so none waits for
-// another.
+// One workgroup per query head, or per KV head and range of rows. It rotates its
+// queries and its KV head's new key (angles pos * theta^(-2i/head_dim) in double,
+// as the reference), takes the scores of positions 0..pos (the new key from LDS,
+// the older ones from the cache), their softmax, and the weighted sum of values.
+// The first query head of each KV head writes the rotated key and the value into
+// the caches at row pos; no workgroup reads row pos from memory, so none waits
+// for another.
 //
-// Two kernels:
+// Three kernels (plan_decode_attention chooses), and two that merge ranges:
 //   chunk kernel (head_dim a multiple of 4, at most 512): the cached rows
 //     0..pos-1 stream through registers in chunks of rows, K and V of a chunk
 //     loaded together as 16-byte vectors and the next chunk's loads in flight
@@ -26,7 +26,11 @@
 //     rows are split into nsplit contiguous ranges, one workgroup per (head,
 //     range): each writes its range's softmax state (running maximum, sum of
 //     exponentials, weighted values) to a scratch record, and a second
-//     kernel merges each head's records in range order.
+//     kernel merges each head's records in range order (more than kWideMerge of
+//     them side by side, a partial sum per thread group).
+//   grouped-query kernel (1, 2, 4 or 8 query heads per KV head, long caches): the
+//     same ranges, a workgroup per (KV head, range) that loads each cached row
+//     once for all its query heads.
 //   generic kernel (any even head_dim): a wave per position for the scores,
 //     a thread per dimension for the values; the scores sit in LDS, so the
 //     cache length is bounded by it.
@@ -732,19 +736,34 @@ AttnSplit plan_decode_attention(int64_t pos, int64_t n_q, int64_t n_kv, int64_t 
   // is n_q head_dim pos = 4 Mi (8 heads: 6 Mi), where the two cross; below it the
   // launches bound and a workgroup per query head has more of them in flight.
   // Measured (us a call in a graph, heads / KV heads / hd, rows; this kernel
-  // against the one it replaces there):
+  // against a workgroup per query head):
   //   32/8/128   734 11.1 / 9.4   1024 9.7 / 10.6   4096 12.5 / 20.3  16383 27.5 / 41.9
   //   64/8/128   734 14.7 / 15.6  1024 12.8 / 18.0  4096 16.5 / 28.8  16383 33.4 / 64.0
-  //   16/2/128  2048 12.9 / 11.0  4096 13.4 / 25.0  16383 21.8 / 56.3
+  //   16/2/128  2048 13.1 / 11.4  3072 13.2 / 12.8  6144 15.7 / 20    16383 21.5 / 56
+  //   8/2/64    2048  9.8 / 8.8   6144  9.9 / 10.3  8/1/128  2048 12.8 / 8.6  4096 13.0 / 11.1
   //   16/16/128 1024  8.0 / 8.0   2048 10.0 / 11.4  4096 16.7 / 19.2  16383 44.9 / 48.3
   //   32/16/64  1024  8.8 / 7.7   2048  9.0 / 10.7  4096 10.7 / 18.0  16383 25.7 / 47.2
   // (two workgroups per CU: 64/8/128 4096 22.7, 16383 42.0.)
-  const int64_t g = n_q / n_kv;
+  // From 86 query heads (256 CUs) a workgroup per query head takes one range, with
+  // twice the waves, and the line is higher: 5 Mi, and with nothing to share (G = 1)
+  // 32 Mi, a cache past the last-level one, or 12 Mi where two ranges of every head
+  // are one round of the CUs:
+  //   128/32/128 4 Mi  9.6 / 8.7    5 Mi 10.0 / 12.5   96/96/128   8 Mi 18.6 / 17.7  24 Mi 39.6 / 36.9
+  //   144/72/128 4 Mi 10.3 / 8.6    5 Mi 10.8 / 12.6   160/160/128 8 Mi 17.9 / 16.3  24 Mi 37.0 / 34.9
+  //   96/24/256  5 Mi 14.4 / 13.0   6 Mi 12.2 / 13.0   128/128/128 8 Mi 16.6 / 15.6  24 Mi 35.0 / 36.5
+  const int64_t cu = std::max(cu_count, 1), g = n_q / n_kv;
+  int64_t line = g == 8 ? 6 : 4;
+  if (n_q <= cu && (cu + n_q - 1) / n_q < 4) {
+    if (g == 1 && n_q < cu) line = cu % n_q == 0 ? 12 : 32;
+    if (g == 2 || g == 4) line = g == 4 && head_dim > 128 ? 6 : 5;
+  }
   const bool gqa = (g == 1 || g == 2 || g == 4 || g == 8) && g * head_dim <= 1024 &&
-                   n_q * head_dim * pos >= (int64_t)(g == 8 ? 6 : 4) << 20;
+                   n_q * head_dim * pos >= line << 20;
   if (gqa) p.group = (int)g;
-  const int64_t want = ((int64_t)std::max(cu_count, 1) + (gqa ? n_kv : n_q) - 1) / (gqa ? n_kv : n_q);
-  const int64_t ns = std::min<int64_t>({want, pos / kMinSplitRows, (int64_t)kMaxSplits});
+  const int64_t want = (cu + (gqa ? n_kv : n_q) - 1) / (gqa ? n_kv : n_q);
+  // (the grouped kernel's ranges rounded up: one of 67 rows takes two of its chunks)
+  const int64_t ns = std::min<int64_t>(
+      {want, (pos + (gqa ? kMinSplitRows - 1 : 0)) / kMinSplitRows, (int64_t)kMaxSplits});
   if (gqa && ns < 2) return p;
   if (!gqa && ns < 4) {
     // one range per head: beyond two chunks of 2 rows per lane, 8 rows per

@@ -38,10 +38,13 @@ def rope(torch, t, hd, pos):
 
 # heads, KV heads, head_dim, cached rows: 1, 2, 4 and 8 heads per KV head at each
 # lanes-per-row width, partial vectors, ranges and chunks that do not divide,
-# either side of the planner's line, one to 64 ranges
+# either side of the planner's line, 16 to 64 ranges; then many heads: one range
+# (two cases), 2, 2, 4, 8 and 10 of them, and two cases below their line
 CASES = [(32, 8, 128, 4096), (32, 8, 128, 1021), (64, 8, 128, 1999), (16, 2, 64, 9001), (16, 16, 128, 2050),
          (24, 12, 128, 1500), (32, 8, 64, 2049), (12, 12, 64, 5463), (8, 4, 256, 2100), (16, 4, 256, 1100),
-         (8, 8, 512, 1100), (16, 2, 100, 5300), (16, 4, 36, 8000), (64, 8, 128, 767), (32, 8, 128, 300)]
+         (8, 8, 512, 1100), (16, 2, 100, 5300), (16, 4, 36, 8000), (64, 8, 128, 767), (32, 8, 128, 300),
+         (256, 256, 128, 130), (256, 256, 128, 200), (512, 128, 64, 140), (128, 128, 128, 800), (256, 32, 128, 200),
+         (64, 32, 128, 777), (96, 24, 128, 600), (96, 96, 128, 600), (144, 72, 128, 230)]
 
 
 @pytest.mark.parametrize("nq,nkv,hd,pos", CASES)
@@ -66,7 +69,34 @@ def test_long_cache(torch, ctx, nq, nkv, hd, pos):
     assert torch.equal(vc[pos], v) and float((kc[pos].double() - kr[pos]).abs().max()) < 1e-6
 
 
-def test_infinite_and_nan_scores(torch, ctx):
+@pytest.mark.parametrize("nq,nkv,pos", [(32, 8, 2000), (256, 256, 200)])
+def test_infinite_scores(torch, ctx, nq, nkv, pos):
+    """A key of +inf: a head whose score is +inf is NaN (inf - inf, as in the
+    reference's softmax), one whose score is -inf leaves the row out."""
+    import raster_amd
+
+    hd, row = 128, pos // 2
+    print(f"[gpu] attention infinite key {nq}/{nkv} pos={pos}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    q, k, v = (torch.randn(n * hd, generator=g, device="cuda") for n in (nq, nkv, nkv))
+    kc, vc = (torch.randn((pos + 1, nkv * hd), generator=g, device="cuda") for _ in range(2))
+    kc[row, 5::hd] = float("inf")
+    out = raster_amd.decode_attention(ctx, q, k, v, kc, vc, pos, nq, nkv, hd, 1e4, hd ** -0.5).view(nq, hd)
+    qr, keep = rope(torch, q.double().view(nq, hd), hd, pos), torch.arange(pos + 1, device="cuda") != row
+    neg = 0
+    for h in range(nq):
+        if float(qr[h, 5]) > 0:
+            assert bool(torch.isnan(out[h]).all())
+            continue
+        j = h // (nq // nkv)
+        p = torch.softmax(kc[keep, j * hd:(j + 1) * hd].double() @ qr[h] * hd ** -0.5, 0)
+        ref = p @ vc[keep, j * hd:(j + 1) * hd].double()
+        assert float((out[h].double() - ref).abs().max()) <= 1e-5 * float(ref.abs().max())
+        neg += 1
+    assert 0 < neg < nq
+
+
+def test_nan_scores(torch, ctx):
     """A NaN key makes its head's outputs NaN; the other heads are as before."""
     import raster_amd
 
