@@ -10,8 +10,10 @@ timed with HIP events on the stream the kernels run on. Before the W warm-up
 steps the step runs untimed for RAMP_S seconds so that the timed steps see the
 GPU at its working clocks.
 
-Beside it, on the same JSON line (default suite "all"; "headline" keeps C2,
-the C1 GEMV and the CPU baseline):
+Beside it (default suite "all"; "headline" keeps C2, the C1 GEMV and the CPU
+baseline), the two rooflines and the CPU baseline on the same JSON line, the others
+and the baseline's legs as a JSON record each on stderr ("[bench] record {...}"):
+on the result line they made it longer than a reader of a log's tail gets whole.
   gemv          C1: the M=1 Q8 decode GEMV (K=N=4096, f32 in/out).
   configs       every other workload configuration, one line per shape:
                 C3 (Q4, M = 1 / 4 / 16, K=4096 N=14336, f32) and C5 (Q4 and Q8,
@@ -100,6 +102,22 @@ SPIN_CYCLES = 20_000_000  # GPU spin ahead of event-timed calls (~8 ms at 2.4 GH
 
 def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
+
+
+RECORDS = ("gemv", "configs", "decoder", "read_ceiling", "int8", "dx", "kquant", "dense")
+
+
+def report(result: dict) -> str:
+    """The result line: everything but RECORDS and the CPU baseline's legs, which
+    go to stderr."""
+    line = {k: v for k, v in result.items() if k not in RECORDS}
+    records = {k: result[k] for k in RECORDS if k in result}
+    if line.get("cpu_baseline"):
+        line["cpu_baseline"] = {k: v for k, v in line["cpu_baseline"].items() if k != "legs"}
+        records["cpu_baseline_legs"] = result["cpu_baseline"].get("legs")
+    for k, v in records.items():
+        log("record " + json.dumps({k: v}))
+    return json.dumps(line)
 
 
 def act_bytes(xdt):
@@ -1117,7 +1135,7 @@ def main():
     else:
         result["cpu_baseline"] = None
     ctx.close()
-    print(json.dumps(result), flush=True)
+    print(report(result), flush=True)
 
 
 if __name__ == "__main__":
