@@ -103,7 +103,7 @@ def test_graph_of_mixed_calls_replays_bit_for_bit(torch, ctx, orc):
     wa = q8(raster_amd, ctx, 11008, 4096, seed=1)      # prefill GEMM (role-split kernel)
     wb = q4(raster_amd, ctx, 4096, 4096, seed=2)       # int8 chain: quantize_act_i8 -> int8 GEMM
     wc = q4k(raster_amd, ctx, orc, 2048, 2048, seed=3)  # K-quant, f32 x quantized in the call
-    wd = q8(raster_amd, ctx, 4160, 8192, seed=4)       # no-alloc: int8-level decode with K-split
+    wd = q8(raster_amd, ctx, 8208, 8192, seed=4)       # no-alloc: int8-level decode with K-split
     we = q4(raster_amd, ctx, 8192, 8192, seed=5)       # no-alloc: small-m GEMM with K-slices
     s = torch.cuda.Stream()
     try:
@@ -118,7 +118,7 @@ def test_graph_of_mixed_calls_replays_bit_for_bit(torch, ctx, orc):
               torch.empty((64, 128), dtype=torch.int32, device="cuda"))
         yb = torch.empty((64, 4096), dtype=torch.float32, device="cuda")
         yc = torch.empty((4, 2048), dtype=torch.float32, device="cuda")
-        yd = torch.empty((12, 4160), dtype=torch.float32, device="cuda")
+        yd = torch.empty((12, 8208), dtype=torch.float32, device="cuda")
         ye = torch.empty((64, 8192), dtype=torch.bfloat16, device="cuda")
         outs = [ya, yb, yc, yd, ye]
 
@@ -198,7 +198,7 @@ def concurrent_cases(raster_amd, ctx, torch):
     """(weight, x, y dtype) of calls with scratch: K-split decode, MFMA decode
     with slices, small-m GEMM with slices, prefill GEMM."""
     return [
-        (q8(raster_amd, ctx, 4160, 8192, seed=41), act(torch, 12, 8192, 51, "f32"), torch.float32),
+        (q8(raster_amd, ctx, 8208, 8192, seed=41), act(torch, 12, 8192, 51, "f32"), torch.float32),
         (q4(raster_amd, ctx, 14336, 4096, seed=42), act(torch, 16, 4096, 52, "f32"), torch.float32),
         (q8(raster_amd, ctx, 28672, 8192, seed=43), act(torch, 32, 8192, 53, "bf16"), torch.bfloat16),
         (q8(raster_amd, ctx, 11008, 4096, seed=44), act(torch, 512, 4096, 54, "bf16"), torch.bfloat16),

@@ -1,7 +1,7 @@
 """rq_qmatmul_noalloc, the rq_qmatmul variant that allocates nothing, against
 rq_qmatmul itself through the C ABI: bit-identical outputs on every kernel
 route that uses scratch (K-slice partial sums of the decode kernels, the packed
-activations of the bf16 GEMMs, both for the small-m GEMM, a K-quant weight's
+activations of the bf16 and f32 GEMMs, both for the small-m GEMM, a K-quant weight's
 q8_K activations) and on routes that
 use none, two calls in a row with the second one smaller, and a call that needs
 more than the fixed scratch is refused with RQ_ERR_SHAPE. The seeded shapes
@@ -81,12 +81,15 @@ CASES = [
     ("q4", 14336, 4096, [1, 1], "f32", "f32"),           # v_dot4 GEMV, no scratch
     ("q8", 48, 8192, [16, 9], "f32", "f32"),             # MFMA decode with K-slices
     ("q4", 14336, 4096, [16, 6], "f32", "f32"),          # MFMA decode, Q4_0, K-slices
-    ("q8", 4160, 8192, [12, 3], "f32", "f32"),           # int8-level decode with K-split (above 32 Mi)
+    ("q8", 4160, 8192, [12, 3], "f32", "f32"),           # MFMA decode above 32 Mi, then int8-level decode, no scratch
+    ("q8", 8208, 8192, [12, 9], "f32", "bf16"),          # int8-level decode with K-split (above 64 Mi)
+    ("q8", 48, 20480, [2, 1], "f32", "f32"),             # int8-level decode with K-split (a long row)
+    ("q4", 2048, 5632, [4, 2], "f32", "f32"),            # MFMA decode of few rows, K-slices
     ("q4", 8192, 8192, [64, 32], "bf16", "bf16"),        # small-m GEMM: packed x + K-slices
     ("q8", 28672, 8192, [32, 17], "bf16", "bf16"),       # small-m GEMM, Q8_0: packed x + K-slices
     ("q8", 11008, 4096, [512, 128], "bf16", "bf16"),     # prefill GEMM: packed x (role-split kernel, then 128-row tiles)
     ("q8", 11008, 4096, [1024, 512], "bf16", "bf16"),    # 256 x 192 one-wave GEMM, then the role-split kernel
-    ("q8", 1000, 1024, [300, 17], "f32", "f32"),         # exact-f32 GEMM, no scratch
+    ("q8", 1000, 1024, [300, 17], "f32", "f32"),         # f32 GEMM: packed hi + lo activations
     ("q4k", 4096, 4096, [8, 1], "f32", "f32"),           # K-quant: q8_K activations in scratch
     ("q6k", 1024, 2048, [40, 3], "f32", "bf16"),         # K-quant, m above the decode range
 ]
