@@ -392,23 +392,21 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
     }
 }
 
-// Role-split form for the larger tiles: eight waves, waves 0..3 (consumers) 32 MF
+// Role-split form for the larger tiles: eight waves, waves 0..3 (consumers) 32
 // rows x 32 NF columns each, waves 4..7 (producers) load the codes RW - 1 steps
 // ahead and convert step s + 2 into LDS buffer (s + 2) % 3 while the consumers
 // run step s. A wave's loads complete in issue order, so a wave that loads both
 // would wait for its codes (HBM) whenever it waits for activations (L2).
-template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int RA>
+template <int FMT, typename ST, int XT, bool PK, int NF, int RA>
 __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_per_eu(2, 2))) void gemm_blk_rs_kernel(
     const uint8_t* __restrict__ q, const ST* __restrict__ sc, const void* __restrict__ x, void* __restrict__ y, int M,
     int K, int N, int npad, int y_dtype, int tiles_m, uint32_t x_bytes) {
   constexpr int NB = kGbBlocks, RW = 3;
-  constexpr int BM = 128 * MF, BN = 32 * NF, G = BN / 16;
+  constexpr int BM = 128, BN = 32 * NF, G = BN / 16;
   constexpr int NT = G * NB * 32 / 256;
   constexpr int NS = (BN * NB + 255) / 256;
-  constexpr int TPS = NB * NF * MF, PR = TPS % 3 == 0 ? 3 : 4;  // tiles per step, block sums in flight
-  static_assert(XT == kXtI8 ? NB % RA == 0 && NF % 2 == 0 && MF == 1
-                            : NB % RA == 0 && NB * NF % 3 == 0 && NB * NF % 4 == 0 && TPS % PR == 0,
-                "rings turn whole in a step");
+  constexpr int TPS = NB * NF;  // tiles per step
+  static_assert(NB % RA == 0 && (XT == kXtI8 ? NF % 2 == 0 : TPS % 3 == 0 && TPS % 4 == 0), "rings turn whole in a step");
   struct Lds {
     u32x4 w[3][NB][2][NF][64];
     float s[3][NB][BN];
@@ -515,15 +513,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
 
   // ---- consumer
   const int l32 = lane & 31, g = lane >> 5;
-  const int m0 = tm * BM + wave * 32 * MF;
+  const int m0 = tm * BM + wave * 32;
   const int r32_last = (M + 31) / 32 - 1;
-  f32x16 zero, acc[MF][NF];
+  f32x16 zero, acc[NF];
 #pragma unroll
   for (int e = 0; e < 16; e++) zero[e] = 0.0f;
 #pragma unroll
-  for (int f = 0; f < MF; f++)
-#pragma unroll
-    for (int c = 0; c < NF; c++) acc[f][c] = zero;
+  for (int c = 0; c < NF; c++) acc[c] = zero;
   if constexpr (XT == kXtI8) {
     f32x32 zero2;
 #pragma unroll
@@ -586,7 +582,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
         for (int t = 0; t < 2; t++)
 #pragma unroll
           for (int e = 0; e < 16; e++)
-            acc[0][2 * q1 + t][e] = fmaf(sc2[cur ^ 1][16 * t + e], p[cur ^ 1][t][e], acc[0][2 * q1 + t][e]);
+            acc[2 * q1 + t][e] = fmaf(sc2[cur ^ 1][16 * t + e], p[cur ^ 1][t][e], acc[2 * q1 + t][e]);
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 12, 0);
 #pragma unroll
@@ -603,27 +599,22 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     for (int t = 0; t < 2; t++)
 #pragma unroll
       for (int e = 0; e < 16; e++)
-        acc[0][NF - 2 + t][e] = fmaf(sc2[1][16 * t + e], p[1][t][e], acc[0][NF - 2 + t][e]);
+        acc[NF - 2 + t][e] = fmaf(sc2[1][16 * t + e], p[1][t][e], acc[NF - 2 + t][e]);
   } else {
-    uint32_t xo[MF];
-#pragma unroll
-    for (int f = 0; f < MF; f++)
-      xo[f] = PK ? (uint32_t)min(m0 / 32 + f, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
-                 : (uint32_t)min(m0 + 32 * f + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
-    u32x4 a[RA][MF][4];
+    const uint32_t xo = PK ? (uint32_t)min(m0 / 32, r32_last) * (uint32_t)nkb * 4096u + 16u * (uint32_t)lane
+                           : (uint32_t)min(m0 + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
+    u32x4 a[RA][4];
     auto aload = [&](int slot, int kb) {
       const ActBlock<false, false> b(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
 #pragma unroll
-      for (int f = 0; f < MF; f++)
-#pragma unroll
-        for (int i = 0; i < 4; i++) a[slot][f][i] = b.x.b128(xo[f] + (PK ? 1024u : 16u) * i, b.off);
+      for (int i = 0; i < 4; i++) a[slot][i] = b.x.b128(xo + (PK ? 1024u : 16u) * i, b.off);
     };
-    f32x16 p[PR];
+    f32x16 p[3];  // the block sums in flight
 #pragma unroll
-    for (int i = 0; i < PR; i++) p[i] = zero;
+    for (int i = 0; i < 3; i++) p[i] = zero;
     bf16x8 w[3][2];
     float ws[4] = {0.0f, 0.0f, 0.0f, 0.0f};  // scales of the column fragments j - 2 .. j + 1
-    bf16x8 h[MF][2], l[MF][2], lp[2];  // the block's hi and lo fragments; the last tile's lo of the block before
+    bf16x8 h[2], l[2], lp[2];  // the block's hi and lo fragments; the last tile's lo of the block before
     const bf16x8 none = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
     w[2][0] = w[2][1] = lp[0] = lp[1] = none;
     auto wread = [&](int j, int buf, int b, int c) {
@@ -638,45 +629,41 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     int buf = 0;
     for (int s = 0; s < steps; s++) {
       const int nbuf = buf == 2 ? 0 : buf + 1;
-      // tile i of the step: column fragment j = i / MF, row fragment i % MF. Its
-      // four MFMAs (hi, hi, lo, lo of the two 16-k halves) are spread over two
-      // turns, so that two chains alternate, and the block sums are scaled in
-      // the turn after, beside the MFMAs of the next two tiles
+      // tile j of the step: a block's column fragment. Its four MFMAs (hi, hi, lo, lo
+      // of the two 16-k halves) are spread over two turns, so that two chains
+      // alternate, and the block sums are scaled in the turn after, beside the MFMAs
+      // of the next two tiles
 #pragma unroll
-      for (int i = 0; i < TPS; i++) {
-        const int j = i / MF, f = i % MF, b = j / NF, c = j % NF;
-        const int q1 = (i + TPS - 1) % TPS, j1 = q1 / MF, f1 = q1 % MF;  // the tile before
-        const int q2 = (i + TPS - 2) % TPS, j2 = q2 / MF, f2 = q2 % MF;  // and the one before it
-        if (c == 0 && f == 0) {
+      for (int j = 0; j < TPS; j++) {
+        const int b = j / NF, c = j % NF;
+        const int j1 = (j + TPS - 1) % TPS, j2 = (j + TPS - 2) % TPS;  // the tile before, and the one before it
+        if (c == 0) {
 #pragma unroll
-          for (int ff = 0; ff < MF; ff++)
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-              const u32x4* r = a[b % RA][ff];
-              u32x4 hv, lv;
-              if (PK) {
-                hv = r[e];
-                lv = r[2 + e];
-              } else {
-                split8(__builtin_bit_cast(f32x4, r[2 * e]), __builtin_bit_cast(f32x4, r[2 * e + 1]), hv, lv);
-              }
-              h[ff][e] = __builtin_bit_cast(bf16x8, hv);
-              l[ff][e] = __builtin_bit_cast(bf16x8, lv);
+          for (int e = 0; e < 2; e++) {
+            const u32x4* r = a[b % RA];
+            u32x4 hv, lv;
+            if (PK) {
+              hv = r[e];
+              lv = r[2 + e];
+            } else {
+              split8(__builtin_bit_cast(f32x4, r[2 * e]), __builtin_bit_cast(f32x4, r[2 * e + 1]), hv, lv);
             }
+            h[e] = __builtin_bit_cast(bf16x8, hv);
+            l[e] = __builtin_bit_cast(bf16x8, lv);
+          }
         }
-        if (f == 0) wread(j + 1, j + 1 < NB * NF ? buf : nbuf, (j + 1) / NF % NB, (j + 1) % NF);
-        const bool head = c == 0 && f == 0;  // the tile before is of the block before
-        p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][0], w[j % 3][0], zero, 0, 0, 0);
-        p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[0] : l[f1][0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
-        p[i % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[f][1], w[j % 3][1], p[i % PR], 0, 0, 0);
-        p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[1] : l[f1][1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+        wread(j + 1, j + 1 < TPS ? buf : nbuf, (j + 1) / NF % NB, (j + 1) % NF);
+        const bool head = c == 0;  // the tile before is of the block before
+        p[j % 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[0], w[j % 3][0], zero, 0, 0, 0);
+        p[j1 % 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[0] : l[0], w[j1 % 3][0], p[j1 % 3], 0, 0, 0);
+        p[j % 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(h[1], w[j % 3][1], p[j % 3], 0, 0, 0);
+        p[j1 % 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(head ? lp[1] : l[1], w[j1 % 3][1], p[j1 % 3], 0, 0, 0);
 #pragma unroll
-        for (int e = 0; e < 16; e++)
-          acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
-        if (c == 0 && f == 0) aload((b + RA - 1) % RA, s * NB + b + RA - 1);
-        if (c == NF - 1 && f == MF - 1) {
-          lp[0] = l[f][0];
-          lp[1] = l[f][1];
+        for (int e = 0; e < 16; e++) acc[j2 % NF][e] = fmaf(ws[j2 % 4], p[j2 % 3][e], acc[j2 % NF][e]);
+        if (c == 0) aload((b + RA - 1) % RA, s * NB + b + RA - 1);
+        if (c == NF - 1) {
+          lp[0] = l[0];
+          lp[1] = l[1];
         }
         if (PK) {
 #pragma unroll
@@ -691,42 +678,40 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
       buf = nbuf;
     }
     {
-      constexpr int q1 = TPS - 1, j1 = q1 / MF, f1 = q1 % MF, q2 = TPS - 2, j2 = q2 / MF, f2 = q2 % MF;
-      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[0], w[j1 % 3][0], p[q1 % PR], 0, 0, 0);
-      p[q1 % PR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[1], w[j1 % 3][1], p[q1 % PR], 0, 0, 0);
+      constexpr int j1 = TPS - 1, j2 = TPS - 2;
+      p[j1 % 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[0], w[j1 % 3][0], p[j1 % 3], 0, 0, 0);
+      p[j1 % 3] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lp[1], w[j1 % 3][1], p[j1 % 3], 0, 0, 0);
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[f2][j2 % NF][e] = fmaf(ws[j2 % 4], p[q2 % PR][e], acc[f2][j2 % NF][e]);
+      for (int e = 0; e < 16; e++) acc[j2 % NF][e] = fmaf(ws[j2 % 4], p[j2 % 3][e], acc[j2 % NF][e]);
 #pragma unroll
-      for (int e = 0; e < 16; e++) acc[f1][j1 % NF][e] = fmaf(ws[j1 % 4], p[q1 % PR][e], acc[f1][j1 % NF][e]);
+      for (int e = 0; e < 16; e++) acc[j1 % NF][e] = fmaf(ws[j1 % 4], p[j1 % 3][e], acc[j1 % NF][e]);
     }
   }
 
 #pragma unroll
-  for (int f = 0; f < MF; f++)
+  for (int c = 0; c < NF; c++) {
+    const int n = n0 + 32 * c + l32;
+    if (n >= N) continue;
 #pragma unroll
-    for (int c = 0; c < NF; c++) {
-      const int n = n0 + 32 * c + l32;
-      if (n >= N) continue;
-#pragma unroll
-      for (int e = 0; e < 16; e++) {
-        const int m = m0 + 32 * f + 8 * (e >> 2) + 4 * g + (e & 3);
-        if (m >= M) continue;
-        if (y_dtype == RQ_F32)
-          static_cast<float*>(y)[(int64_t)m * N + n] = acc[f][c][e];
-        else
-          static_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)f32_to_bf16_bits(acc[f][c][e]);
-      }
+    for (int e = 0; e < 16; e++) {
+      const int m = m0 + 8 * (e >> 2) + 4 * g + (e & 3);
+      if (m >= M) continue;
+      if (y_dtype == RQ_F32)
+        static_cast<float*>(y)[(int64_t)m * N + n] = acc[c][e];
+      else
+        static_cast<uint16_t*>(y)[(int64_t)m * N + n] = (uint16_t)f32_to_bf16_bits(acc[c][e]);
     }
+  }
 }
 
-template <int FMT, typename ST, int XT, bool PK, int MF, int NF, int RA>
+template <int FMT, typename ST, int XT, bool PK, int NF, int RA>
 static hipError_t launch_rs_t(const MatmulArgs& a, const void* x, void* y, int64_t m, hipEvent_t begin,
                            hipEvent_t done) {
-  constexpr int BM = 128 * MF, BN = 32 * NF;
+  constexpr int BM = 128, BN = 32 * NF;
   const int64_t tiles_m = (m + BM - 1) / BM, tiles_n = (a.n + BN - 1) / BN;
   if (tiles_m * tiles_n > INT32_MAX) return hipErrorInvalidValue;
   const int64_t bytes = std::min<int64_t>(PK ? packed_bytes(XT, m, a.k) : m * a.k * 4, UINT32_MAX);
-  hipExtLaunchKernelGGL((gemm_blk_rs_kernel<FMT, ST, XT, PK, MF, NF, RA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0,
+  hipExtLaunchKernelGGL((gemm_blk_rs_kernel<FMT, ST, XT, PK, NF, RA>), dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0,
                         a.stream, begin, done, 0, a.q, static_cast<const ST*>(a.scales), x, y, (int)m, (int)a.k,
                         (int)a.n, (int)a.npad, a.y_dtype, (int)tiles_m, (uint32_t)bytes);
   return hipGetLastError();
@@ -802,8 +787,8 @@ hipError_t launch_tile(int tile, const MatmulArgs& a, const void* x, void* y, in
     case 0: return launch_t<FMT, ST, XT, PK, 1, 1, 1, 4>(a, x, y, m, begin, done);
     case 1: return launch_t<FMT, ST, XT, PK, 2, 1, 1, 4>(a, x, y, m, begin, done);
     case 2: return launch_t<FMT, ST, XT, PK, 1, 2, 4, 1>(a, x, y, m, begin, done);
-    case 3: return launch_rs_t<FMT, ST, XT, PK, 1, 3, 4>(a, x, y, m, begin, done);
-    default: return launch_rs_t<FMT, ST, XT, PK, 1, 6, 2>(a, x, y, m, begin, done);
+    case 3: return launch_rs_t<FMT, ST, XT, PK, 3, 4>(a, x, y, m, begin, done);
+    default: return launch_rs_t<FMT, ST, XT, PK, 6, 2>(a, x, y, m, begin, done);
   }
 }
 
@@ -877,8 +862,8 @@ static hipError_t launch_i8(const MatmulArgs& a, int cu_count) {
     const hipError_t e =
         tile < 0    ? launch_t<FMT, ST, kXtI8, true, 1, 1, 1, 4, true>(a, a.scratch, y, m, nullptr, done)
         : tile == 0 ? launch_t<FMT, ST, kXtI8, true, 1, 1, 1, 4>(a, a.scratch, y, m, nullptr, done)
-        : tile == 1 ? launch_rs_t<FMT, ST, kXtI8, true, 1, 2, 4>(a, a.scratch, y, m, nullptr, done)
-                    : launch_rs_t<FMT, ST, kXtI8, true, 1, 4, 4>(a, a.scratch, y, m, nullptr, done);
+        : tile == 1 ? launch_rs_t<FMT, ST, kXtI8, true, 2, 4>(a, a.scratch, y, m, nullptr, done)
+                    : launch_rs_t<FMT, ST, kXtI8, true, 4, 4>(a, a.scratch, y, m, nullptr, done);
     if (e != hipSuccess) return e;
   }
   return hipSuccess;

@@ -15,7 +15,7 @@
 //   -OFF * sum (hi + lo) (formed when the activations are staged, fed as the
 //   MFMA's C operand), which leaves the block's dot product for the block
 //   scale to multiply in f32. No rounding of scale * code is involved.
-// * A workgroup has GW x KW waves and one K-slice (grid.x = columns x ks). It
+// * A workgroup has GW waves and one K-slice (grid.x = columns x ks). It
 //   stages its slice of x (all m rows, hi and lo) in LDS once; then each wave
 //   streams the weight chunks of its 16-row groups through a WD-step register
 //   ring: A = the activation fragment from LDS (lane (r, q): row r, k = 8q ..
@@ -30,11 +30,9 @@
 //   (low nibbles) and 4q+16 .. 4q+19 (high nibbles). The activation
 //   fragments in LDS are laid out in that k order; the scales of the four
 //   chunks are broadcast the same way.
-//   The KW waves of a column split the slice's steps and add their partial
-//   sums through LDS in wave order; with ks > 1 the slices' partial sums go
-//   to `part` and gemm_sm_reduce_kernel adds them in slice order (or, without
-//   scratch, one workgroup takes the slices in that order: gemv_mf_seq_kernel).
-//   Deterministic either way.
+//   With ks > 1 the slices' partial sums go to `part` and gemm_sm_reduce_kernel
+//   adds them in slice order (or, without scratch, one workgroup takes the
+//   slices in that order: gemv_mf_seq_kernel). Deterministic either way.
 #include <algorithm>
 #include <atomic>
 
@@ -119,29 +117,27 @@ __device__ __forceinline__ bf16x8 mf_q8_codes(const MfCodes<ST>& c) {
 }  // namespace
 
 // LDS bytes of a workgroup: x fragments (spl steps x P parts x m rows x 64 B),
-// the offset sums (spl x 16 floats), 16 bytes of wave flags, and with KW > 1 two
-// sets of the waves' partial outputs
-__host__ __device__ inline int mf_lds_bytes(int m, int spl, int parts, int kw, int gw) {
-  return spl * parts * m * 64 + spl * 64 + 16 + (kw > 1 ? 2 * gw * kw * 1024 : 0);
+// the offset sums (spl x 16 floats), 16 bytes of wave flags
+__host__ __device__ inline int mf_lds_bytes(int m, int spl, int parts) {
+  return spl * parts * m * 64 + spl * 64 + 16;
 }
 
 // K-slice s of the workgroup's column col of gcols. SEQ: the workgroup takes every
 // slice itself (one unit per wave) and adds this one to sum.
-template <int FMT, typename ST, int XT, int KW, int GW, int WD, bool SEQ>
+template <int FMT, typename ST, int XT, int GW, int WD, bool SEQ>
 __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST* __restrict__ sc,
                                          const void* __restrict__ x, void* __restrict__ y, float* __restrict__ part,
                                          int M, int K, int N, int npad, int y_dtype, int ks, int s, int col, int gcols,
                                          f32x4& sum) {
-  constexpr int WAVES = KW * GW, P = XT == RQ_F32 ? 2 : 1;
+  constexpr int P = XT == RQ_F32 ? 2 : 1;
   constexpr float OFF = FMT == RQ_Q8_0 ? 128.0f : 136.0f;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int nkb = K / 32, ngroups = npad / 16;
   const int spl = (nkb + ks - 1) / ks;
   const int kb0 = min(nkb, s * spl), nst = min(nkb, kb0 + spl) - kb0;  // this slice: steps kb0 .. kb0+nst-1
-  const int xs_off = spl * P * M * 64, flag_off = xs_off + spl * 64, red_off = flag_off + 16;
+  const int xs_off = spl * P * M * 64, flag_off = xs_off + spl * 64;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int kw = wave % KW, gw = wave / KW;
   const int r = lane & 15, qd = lane >> 4;
 
   // ---- activations of the slice into LDS. Item = 8 consecutive x of one
@@ -149,7 +145,7 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
   // lanes, which add their sums by shuffles. The first round's loads go out
   // before the weight ring's, so converting them waits for them only.
   constexpr int XI = 4;
-  const int nitems = M * nst * 4, stride = 64 * WAVES;
+  const int nitems = M * nst * 4, stride = 64 * GW;
   float xv[XI][8];
   float amax = 0.0f;     // the lane's largest |x|
   bool restage = false;  // rows flagged in LDS at 2^-13 x
@@ -229,30 +225,28 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
     }
   };
 
-  // ---- this wave's work: units j = 0 .. nunits-1 (group col GW + gw + j
-  // gcols GW of the slice), each its share of the slice's steps (spw steps
-  // from kw spw), padded to spp, a whole number of ring turns, so that the
+  // ---- this wave's work: units j = 0 .. nunits-1 (group col GW + wave + j
+  // gcols GW of the slice), the slice's steps padded to spp, a whole number of
+  // ring turns, so that the
   // unrolled ring loop holds steps only (a unit ends between turns; its
   // store code exists once: each wave runs the loop only a few times, and
   // a large unrolled body would be fetched from a cold instruction cache).
   // Flat step t = j spp + u; padding steps load their unit's last step
   // again and compute nothing.
-  const int spw = (nst + KW - 1) / KW;
-  const int spp = (spw + WD - 1) / WD * WD;
+  const int spp = (nst + WD - 1) / WD * WD;
   const int nunits = (ngroups + gcols * GW - 1) / (gcols * GW);
   static_assert(WD % 4 == 0, "the Q4_0 ring holds whole quads");
   MfCodes<ST> wc[FMT == RQ_Q4_0 ? 1 : WD];
   MfQuad<ST> wq[FMT == RQ_Q4_0 ? WD / 4 : 1];
   // Q4_0: quad slot of steps u .. u+3 (u a multiple of 4); lane (r, qd)
-  // loads step u + qd, clamped to the wave's share (steps past it compute
-  // nothing)
+  // loads step u + qd, clamped to the slice (steps past it compute nothing)
   auto load_q = [&](int slot, int j, int u) {
     if (j >= nunits) {  // past the end: the last quad again
       j = nunits - 1;
       u = spp - 4;
     }
-    const int g = min(col * GW + gw + j * gcols * GW, ngroups - 1);
-    const int kb = kb0 + min(kw * spw + min(u + qd, spw - 1), nst - 1);
+    const int g = min(col * GW + wave + j * gcols * GW, ngroups - 1);
+    const int kb = kb0 + min(u + qd, nst - 1);
     const int64_t chunk = (int64_t)g * nkb + kb;
     wq[slot].v = *reinterpret_cast<const u32x4*>(q + chunk * 256 + r * 16);
     wq[slot].s = sc[chunk * 16 + r];
@@ -263,8 +257,8 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
       j = nunits - 1;
       u = spp - 1;
     }
-    const int g = min(col * GW + gw + j * gcols * GW, ngroups - 1);
-    const int kb = kb0 + min(kw * spw + min(u, spw - 1), nst - 1);
+    const int g = min(col * GW + wave + j * gcols * GW, ngroups - 1);
+    const int kb = kb0 + min(u, nst - 1);
     const int64_t chunk = (int64_t)g * nkb + kb;
     wc[slot].v = *reinterpret_cast<const u32x2*>(q + chunk * 512 + r * 32 + 8 * qd);
     wc[slot].s = sc[chunk * 16 + r];
@@ -315,10 +309,10 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
   // A row holding |x| >= 2^112 in the slice is staged again at 2^-13 x, so that
   // sums of x (c + OFF), |c + OFF| <= 255, over a block cannot overflow where the
   // block's dot product would not; its outputs take the factor back.
-  static_assert(16 % WAVES == 0, "flag bytes per wave");
+  static_assert(16 % GW == 0, "flag bytes per wave");
   uint8_t* flags = smem + flag_off;
   const bool wbig = __any(amax >= 0x1p112f) != 0;
-  if (lane < 16 / WAVES) flags[wave * (16 / WAVES) + lane] = wbig ? 1 : 0;
+  if (lane < 16 / GW) flags[wave * (16 / GW) + lane] = wbig ? 1 : 0;
   __syncthreads();
   const u32x4 fl = *reinterpret_cast<const u32x4*>(flags);
   f32x4 ysc = {1.0f, 1.0f, 1.0f, 1.0f};
@@ -363,7 +357,7 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
       }
       return;
     }
-    const int g = col * GW + gw + j * gcols * GW;
+    const int g = col * GW + wave + j * gcols * GW;
     const int o = 16 * g + r;
     if (g >= ngroups || o >= N) return;
 #pragma unroll
@@ -380,20 +374,7 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
     }
   };
   auto finish = [&](int j) {
-    if (KW > 1) {
-      f32x4* red = reinterpret_cast<f32x4*>(smem + red_off);
-      const int base = (j & 1) * GW * KW * 64 + gw * KW * 64;
-      red[base + kw * 64 + lane] = acc;
-      __syncthreads();
-      if (kw == 0) {
-        f32x4 t = red[base + lane];
-#pragma unroll
-        for (int k = 1; k < KW; k++) t += red[base + k * 64 + lane];
-        store(j, t);
-      }
-    } else {
-      store(j, acc);
-    }
+    store(j, acc);
     acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   };
 
@@ -440,7 +421,7 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
           // the quad's four steps side by side: their LDS reads, then the
           // four MFMA chains, then the four block epilogues, so that neither
           // the LDS latency nor the MFMA latency is paid once per step. A
-          // step past the share reads the slice's last step again and has
+          // step past the slice reads the slice's last step again and has
           // factor 0 (a finite block dot, or a row already non-finite).
           bf16x8 ah[4], al[4];
           f32x4 xo[4];
@@ -448,8 +429,8 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
 #pragma unroll
           for (int jj = 0; jj < 4; jj++) {
             const int u = u0 + 4 * t + jj;
-            const bool live = u < spw && kw * spw + u < nst;  // workgroup-uniform
-            const int su = min(kw * spw + u, nst - 1);
+            const bool live = u < nst;  // workgroup-uniform
+            const int su = min(u, nst - 1);
             const int ab = su * P * M * 64;
             ah[jj] = *reinterpret_cast<const bf16x8*>(smem + ab + aoff);
             if (P == 2) al[jj] = *reinterpret_cast<const bf16x8*>(smem + ab + M * 64 + aoff);
@@ -486,8 +467,7 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
         // flight, and its waits then drain the ring once per turn
         load_w(i, lj, lu);
         advance(lj, lu);
-        const int su = kw * spw + u;
-        if (u < spw && su < nst) step(su, bw, sv);
+        if (u < nst) step(u, bw, sv);
       }
     }
     finish(j);
@@ -495,14 +475,14 @@ __device__ __forceinline__ void mf_slice(const uint8_t* __restrict__ q, const ST
   }
 }
 
-template <int FMT, typename ST, int XT, int KW, int GW, int WD>
-__global__ __launch_bounds__(64 * KW * GW) void gemv_mf_kernel(const uint8_t* __restrict__ q,
+template <int FMT, typename ST, int XT, int GW, int WD>
+__global__ __launch_bounds__(64 * GW) void gemv_mf_kernel(const uint8_t* __restrict__ q,
                                                                const ST* __restrict__ sc,
                                                                const void* __restrict__ x, void* __restrict__ y,
                                                                float* __restrict__ part, int M, int K, int N,
                                                                int npad, int y_dtype, int ks) {
   f32x4 none;
-  mf_slice<FMT, ST, XT, KW, GW, WD, false>(q, sc, x, y, part, M, K, N, npad, y_dtype, ks, (int)blockIdx.x % ks,
+  mf_slice<FMT, ST, XT, GW, WD, false>(q, sc, x, y, part, M, K, N, npad, y_dtype, ks, (int)blockIdx.x % ks,
                                            (int)blockIdx.x / ks, (int)gridDim.x / ks, none);
 }
 
@@ -521,7 +501,7 @@ __global__ __launch_bounds__(64 * kSeqWaves) void gemv_mf_seq_kernel(const uint8
   f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
   for (int s = 0; s < ks; s++) {
     if (s > 0) __syncthreads();  // the slice before has been read
-    mf_slice<FMT, ST, XT, 1, kSeqWaves, WD, true>(q, sc, x, y, nullptr, M, K, N, npad, y_dtype, ks, s,
+    mf_slice<FMT, ST, XT, kSeqWaves, WD, true>(q, sc, x, y, nullptr, M, K, N, npad, y_dtype, ks, s,
                                                   (int)blockIdx.x, (int)gridDim.x, sum);
   }
   const int lane = threadIdx.x & 63, o = 16 * ((int)blockIdx.x * kSeqWaves + (int)(threadIdx.x >> 6)) + (lane & 15);
@@ -542,18 +522,17 @@ hipError_t launch_split_reduce(const float* part, void* y, int64_t n, int ks, in
 
 // One configuration: ks K-slices, gcols workgroup columns per slice; without a.part
 // the slices one after another.
-template <int FMT, typename ST, int XT, int KW, int GW, int WD>
+template <int FMT, typename ST, int XT, int GW, int WD>
 hipError_t launch_gemv_mf_t(const MatmulArgs& a, int ks, int gcols) {
   constexpr int P = XT == RQ_F32 ? 2 : 1;
-  auto kernel = &gemv_mf_kernel<FMT, ST, XT, KW, GW, WD>;
+  auto kernel = &gemv_mf_kernel<FMT, ST, XT, GW, WD>;
   auto seq_kernel = &gemv_mf_seq_kernel<FMT, ST, XT, WD>;
   const bool seq = ks > 1 && !a.part;
   const int nkb = (int)(a.k / 32);
   if (ks < 1 || ks > nkb || gcols < 1 || a.m < 1 || a.m > 16) return hipErrorInvalidValue;
-  if (seq && KW != 1) return hipErrorInvalidValue;
   const int spl = (nkb + ks - 1) / ks;
   if ((int64_t)(ks - 1) * spl >= nkb) return hipErrorInvalidValue;  // every slice holds steps
-  const int lds = mf_lds_bytes((int)a.m, spl, P, KW, GW);
+  const int lds = mf_lds_bytes((int)a.m, spl, P);
   if (lds > 163840) return hipErrorInvalidValue;
   // dynamic LDS above 64 KB is allowed once per kernel and device
   static std::atomic<uint64_t> attr_set{0};
@@ -572,7 +551,7 @@ hipError_t launch_gemv_mf_t(const MatmulArgs& a, int ks, int gcols) {
                           (int)a.n, (int)a.npad, a.y_dtype, ks);
     return hipGetLastError();
   }
-  hipExtLaunchKernelGGL(kernel, dim3((unsigned)(gcols * ks)), dim3(64 * KW * GW), (unsigned)lds, a.stream,
+  hipExtLaunchKernelGGL(kernel, dim3((unsigned)(gcols * ks)), dim3(64 * GW), (unsigned)lds, a.stream,
                         a.ev_main[0], a.ev_main[1], 0, a.q, static_cast<const ST*>(a.scales),
                         a.x, a.y, a.part, (int)a.m, (int)a.k, (int)a.n, (int)a.npad, a.y_dtype, ks);
   if (hipError_t e = hipGetLastError()) return e;
@@ -633,11 +612,10 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
   if (!mf_takes(m, k, npad, format)) return p;
   const int parts = x_dtype == RQ_F32 ? 2 : 1;
   const int64_t nkb = k / 32, ngroups = npad / 16;
-  p.kw = 1;
   p.gw = format == RQ_Q4_0 ? 16 : 8;
   p.wd = format == RQ_Q4_0 ? 8 : 16;
   int64_t ks = 1;
-  while (mf_lds_bytes((int)m, (int)((nkb + ks - 1) / ks), parts, p.kw, p.gw) > 81920 ||
+  while (mf_lds_bytes((int)m, (int)((nkb + ks - 1) / ks), parts) > 81920 ||
          (ks - 1) * ((nkb + ks - 1) / ks) >= nkb) {
     if (++ks > nkb) return p;
   }
@@ -673,9 +651,9 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
 template <int FMT, typename ST, int XT>
 static hipError_t launch_mf_x(const MatmulArgs& a, const MfPlan& p) {
   if constexpr (FMT == RQ_Q4_0) {
-    if (p.kw == 1 && p.gw == 16 && p.wd == 8) return launch_gemv_mf_t<FMT, ST, XT, 1, 16, 8>(a, p.ks, p.gcols);
+    if (p.gw == 16 && p.wd == 8) return launch_gemv_mf_t<FMT, ST, XT, 16, 8>(a, p.ks, p.gcols);
   } else {
-    if (p.kw == 1 && p.gw == 8 && p.wd == 16) return launch_gemv_mf_t<FMT, ST, XT, 1, 8, 16>(a, p.ks, p.gcols);
+    if (p.gw == 8 && p.wd == 16) return launch_gemv_mf_t<FMT, ST, XT, 8, 16>(a, p.ks, p.gcols);
   }
   return hipErrorInvalidValue;
 }

@@ -130,7 +130,7 @@ DecodePlan plan_decode(int64_t m, int64_t k, int64_t npad, int cu_count);
 
 // Decode on bf16 MFMA with exact codes (gemv_mf.hip): plain calls, f32 / bf16
 // x, 2 <= m <= 16, by m, k and n (mf_takes; the kernel takes m <= 16).
-// kw x gw waves per workgroup,
+// gw waves per workgroup,
 // wd-step weight ring, ks K-slices, gcols workgroup columns per slice.
 // Dense f32 GEMM (dense.hip, rocBLAS): a library handle per context, created
 // on first use. Statuses are rocBLAS's (0 = success).
@@ -149,7 +149,7 @@ struct MfPlan {
   // a call whose slices' scratch cannot be had fails; else (calls that an int8-level
   // kernel without scratch could serve) it runs without, slower
   bool scratch;
-  int kw, gw, wd, ks, gcols;
+  int gw, wd, ks, gcols;
 };
 MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format, int cu_count);
 hipError_t launch_gemv_mf(const MatmulArgs& a, const MfPlan& p);
