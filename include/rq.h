@@ -222,11 +222,12 @@ int rq_weight_device_ptrs(rq_weight w, const void** qdata, const void** scales);
  *    m <= 8); the MFMA decode kernel when a slice of x would not fit two
  *    workgroups' LDS, and further until the grid covers about 85% of the CUs,
  *    rounded up to a power of two while each slice keeps 8 blocks (at most
- *    in / 32 slices; Q4_0 at m <= 4, and Q8_0 at m <= 8 or with n * in above
- *    32 Mi, grow it under capture too, and where they cannot have it (device
- *    memory full, rq_qmatmul_noalloc past RQ_NOALLOC_SCRATCH_MAX) take the
- *    slices one after another, slower, with the same results); the
- *    weight-stream GEMM (bf16 x, 16 < m <= 64) on a thin grid (up to 8 slices);
+ *    in / 32 slices; Q4_0 at m <= 4, and Q8_0 at m <= 8, with n * in above
+ *    32 Mi, or with in < 3072 and m * in < 5 n, grow it under capture too, and
+ *    where they cannot have it (device memory full, rq_qmatmul_noalloc past
+ *    RQ_NOALLOC_SCRATCH_MAX) take the slices one after another, slower, with
+ *    the same results); the weight-stream GEMM (bf16 x, 16 < m <= 64) on a
+ *    thin grid (up to 8 slices);
  *  - Q4_K / Q6_K: the q8_K activations, m * (in + in/256*4 + in/sub*4)
  *    bytes (each part rounded up to 256), sub = 32 for Q4_K, 16 for Q6_K.
  * Under HIP graph capture nothing else can be allocated: run the same (or a

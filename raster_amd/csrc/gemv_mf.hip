@@ -626,7 +626,7 @@ MfPlan plan_gemv_mf(int64_t m, int64_t k, int64_t npad, int x_dtype, int format,
     while (n > ks && (n - 1) * ((nkb + n - 1) / n) >= nkb) --n;  // no empty slice
     p.ks = (int)n;
     if (p.gcols * n > INT32_MAX) return p;
-    p.scratch = m >= 9 && npad * k <= (int64_t(32) << 20);
+    p.scratch = m >= 9 && npad * k <= (int64_t(32) << 20) && (k >= 3072 || m * k >= 5 * npad);
     p.ok = true;
     return p;
   }

@@ -210,8 +210,8 @@ __global__ __launch_bounds__(64 * kKqWaves) void kquant_gemv_kernel(
   float* ls = reinterpret_cast<float*>(smem + MT * K + MT * nsub * 4);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  // ---- this wave's work: row groups gi = 0 .. ng-1 (rows o0 = 4 (gw + gi
-  // nwaves) ..), each swept in nit steps (lane: sub-block lane + 64 si). The
+  // ---- this wave's work: row groups gi = 0 .. ng-1 (kKqRows rows from o0 =
+  // kKqRows (gw + gi nwaves)), each swept in nit steps (lane: sub-block lane + 64 si). The
   // steps stream through a D-step register ring of raw code and scale bits
   // across row groups (steps padded to whole ring turns); nothing converts or
   // tests loaded bits before the step computes, and refills are unconditional
@@ -220,7 +220,8 @@ __global__ __launch_bounds__(64 * kKqWaves) void kquant_gemv_kernel(
   // 15.5 us and Q6_K 16.9 / 17.4 / 18.9 / 19.0 us at D = 1 .. 4; before this
   // stream, loading each step only when it was computed: 15.0 and 16.3 us).
   const int nthr = (int)blockDim.x;
-  const int gw = XF ? wave * (int)gridDim.x + (int)blockIdx.x : (int)blockIdx.x * (nthr / 64) + wave, nwaves = (int)gridDim.x * (nthr / 64);
+  const int gw = XF ? wave * (int)gridDim.x + (int)blockIdx.x : (int)blockIdx.x * (nthr / 64) + wave;
+  const int nwaves = (int)gridDim.x * (nthr / 64);
   const int ngrp = (N + kKqRows - 1) / kKqRows;
   const int ng = gw < ngrp ? (ngrp - 1 - gw) / nwaves + 1 : 0;
   const int nit = (nsub + 63) / 64, nitp = (nit + D - 1) / D * D;

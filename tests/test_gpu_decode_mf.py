@@ -235,7 +235,8 @@ def test_mf_lines_and_large_values(torch, ctx, orc, fmt, m, out, in_, kernel, xd
 @pytest.mark.parametrize("fmt,m,out,in_,xdt,ydt", [("q4", 4, 2048, 5632, "f32", "f32"), ("q4f", 2, 300, 8224, "f32", "bf16"),
                                                    ("q4", 3, 2801, 5632, "bf16", "f32"), ("q8", 6, 1024, 4096, "f32", "f32"),
                                                    ("q8", 5, 37, 14336, "bf16", "bf16"), ("q8", 16, 6200, 8192, "f32", "bf16"),
-                                                   ("q8", 8, 1500, 3104, "f32", "f32")])
+                                                   ("q8", 8, 1500, 3104, "f32", "f32"), ("q8", 9, 5632, 2048, "f32", "f32"),
+                                                   ("q8", 16, 7000, 2048, "bf16", "bf16")])
 def test_mf_captured_first(torch, orc, fmt, m, out, in_, xdt, ydt):
     """A first call under graph capture grows the K-slices' scratch there: the bits of
     the eager call on every replay (a row of 2^112 and more among them)."""
