@@ -84,23 +84,22 @@ struct Src<true> {
 // Blocks past the last one, which fill up a step, add zeros: rereading the last
 // block and scaling its sum by 0 would make NaN where y is infinite. f32
 // activations, whose sums can overflow, read as zero there, out of a resource of
-// no bytes; the int8 sums cannot, so the codes are the last block's again, with
-// scales from the zeros that the packed scales end with.
-template <bool WIDE, bool I8>
+// no bytes; the int8 sums cannot, so the codes there are the next tile's (zeros
+// after the last), with scales from the zeros that each tile's scales end with.
+template <bool WIDE>
 struct ActBlock {
   using Off = typename Src<WIDE>::Off;
   Src<WIDE> x;
   Off off;  // of the block
   __device__ __forceinline__ ActBlock(const void* p, uint32_t x_bytes, int kb, int nkb, uint32_t block_bytes)
-      : x(p, I8 || kb < nkb ? x_bytes : 0u),
-        off(I8 ? (Off)min(kb, nkb - 1) * block_bytes : kb < nkb ? (Off)kb * block_bytes : 0u) {}
+      : x(p, kb < nkb ? x_bytes : 0u), off(kb < nkb ? (Off)kb * block_bytes : 0u) {}
 };
 
-// bytes of the packed activations: bf16 hi + lo, or (int8) bf16 codes and f32 block
-// scales, of one block more
+// bytes of the packed activations: bf16 hi + lo, or (int8) f32 block scales, of one
+// block more per tile, and bf16 codes, of one block more
 int64_t packed_bytes(int x_dtype, int64_t m, int64_t k) {
   const int64_t m32 = (m + 31) / 32 * 32;
-  return x_dtype == kXtI8 ? m32 * k * 2 + m32 * (k / 32 + 1) * 4 : m32 * k * 4;
+  return x_dtype == kXtI8 ? m32 * (k / 32 + 1) * 4 + m32 * k * 2 + 2048 : m32 * k * 4;
 }
 
 }  // namespace
@@ -129,9 +128,9 @@ __global__ __launch_bounds__(256) void pack_x32_split_kernel(const float* __rest
   dst[128] = lo;
 }
 
-// int8 codes xq[M][K] and their block scales xs[M][K/32] -> the same fragments
-// (codes as bf16, exact) and, after them, the scales as [M/32][K/32 + 1][32], the
-// last block's zero.
+// int8 codes xq[M][K] and their block scales xs[M][K/32] -> the scales as
+// [M/32][K/32 + 1][32], a tile's last block zero, and after them the same fragments
+// (codes as bf16, exact) and a block of zeros.
 __global__ __launch_bounds__(256) void pack_x32_i8_kernel(const int8_t* __restrict__ xq, const float* __restrict__ xs,
                                                           uint16_t* __restrict__ xf, int M, int K) {
   const int nkb = K / 32, nq = (nkb + 1) / 2;
@@ -143,10 +142,16 @@ __global__ __launch_bounds__(256) void pack_x32_i8_kernel(const int8_t* __restri
   if (m < M) v = *reinterpret_cast<const u32x2*>(xq + (int64_t)m * K + 32 * kb + 8 * cc);
   const u32x2 p = q8_dword_bf16(v[0], 1.0f), q = q8_dword_bf16(v[1], 1.0f);
   const int64_t at = (int64_t)tile * nkb + kb;
-  reinterpret_cast<u32x4*>(xf)[(at * 2 + (cc & 1)) * 64 + row + 32 * (cc >> 1)] = u32x4{p[0], p[1], q[0], q[1]};
-  float* sf = reinterpret_cast<float*>(xf + (int64_t)((M + 31) / 32) * nkb * 1024) + (at + tile) * 32 + row;
+  const int tiles = (M + 31) / 32;
+  float* sf = reinterpret_cast<float*>(xf) + (at + tile) * 32 + row;
+  u32x4* cf = reinterpret_cast<u32x4*>(reinterpret_cast<float*>(xf) + (int64_t)tiles * (nkb + 1) * 32) +
+              (at * 2 + (cc & 1)) * 64 + row + 32 * (cc >> 1);
+  cf[0] = u32x4{p[0], p[1], q[0], q[1]};
   if (cc == 0) sf[0] = m < M ? xs[(int64_t)m * nkb + kb] : 0.0f;
-  if (cc == 1 && kb == nkb - 1) sf[32] = 0.0f;
+  if (kb == nkb - 1) {
+    if (cc == 1) sf[32] = 0.0f;
+    if (tile == tiles - 1) cf[128] = u32x4{0u, 0u, 0u, 0u};
+  }
 }
 
 // Workgroup: WM x KG waves; tile 32 MF WM rows x 32 NF columns, a wave 32 MF x
@@ -267,27 +272,35 @@ gemm_blk_kernel(const uint8_t* __restrict__ q, const ST* __restrict__ sc, const 
 
   // ---- this wave's activation fragments: rows m0 + 32 f + lane % 32
   const int r32_last = (M + 31) / 32 - 1;
-  const Off xs_base = (Off)(r32_last + 1) * (Off)nkb * 2048u;  // I8: the scales' region
+  const Off xc = I8 ? (Off)(r32_last + 1) * (Off)(nkb + 1) * 128u : 0u;  // I8: the codes, after the scales
   Off xo[MF], so[MF];
 #pragma unroll
   for (int f = 0; f < MF; f++) {
     const Off t32 = (Off)min(m0 / 32 + f, r32_last);
-    xo[f] = PK ? t32 * (Off)nkb * (1024u * AF) + 16u * (Off)lane
+    xo[f] = PK ? xc + t32 * (Off)nkb * (1024u * AF) + 16u * (Off)lane
                : (Off)min(m0 + 32 * f + l32, M - 1) * (Off)nkb * 128u + 64u * (Off)g;
-    so[f] = xs_base + t32 * (Off)(nkb + 1) * 128u + 16u * (Off)g;
+    so[f] = t32 * (Off)(nkb + 1) * 128u + 16u * (Off)g;
   }
   u32x4 a[2][MF][AF];     // PK: hi j 0, 1, f32: lo j 0, 1; else the 16 f32
   f32x4 xs[2][I8 ? MF : 1][4];  // I8: the scales of rows 8 q + 4 g + 0..3
   auto aload = [&](int slot, int kb) {
-    const ActBlock<WIDE, I8> b(x, x_bytes, kb, nkb, PK ? 1024u * AF : 128u);
+    if constexpr (I8) {
+      const Src<WIDE> src(x, x_bytes);
+      const Off k = (Off)min(kb, nkb);
 #pragma unroll
-    for (int f = 0; f < MF; f++) {
+      for (int f = 0; f < MF; f++) {
 #pragma unroll
-      for (int i = 0; i < AF; i++) a[slot][f][i] = b.x.b128(xo[f] + (PK ? 1024u : 16u) * i, b.off);
-      if (I8)
+        for (int i = 0; i < AF; i++) a[slot][f][i] = src.b128(xo[f] + 1024u * i, k * 2048u);
 #pragma unroll
         for (int i = 0; i < 4; i++)
-          xs[slot][f][i] = __builtin_bit_cast(f32x4, b.x.b128(so[f] + 32u * i, (Off)min(kb, nkb) * 128u));
+          xs[slot][f][i] = __builtin_bit_cast(f32x4, src.b128(so[f] + 32u * i, k * 128u));
+      }
+    } else {
+      const ActBlock<WIDE> b(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
+#pragma unroll
+      for (int f = 0; f < MF; f++)
+#pragma unroll
+        for (int i = 0; i < AF; i++) a[slot][f][i] = b.x.b128(xo[f] + (PK ? 1024u : 16u) * i, b.off);
     }
   };
 
@@ -530,20 +543,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
     // cost about 70 beside the FMAs that wait for them), issued ahead of the next
     // pair's MFMAs, beside which the pair before is scaled
     const uint32_t t32 = (uint32_t)min(m0 / 32, r32_last);
-    const uint32_t xo = t32 * (uint32_t)nkb * 2048u + 16u * (uint32_t)lane;
-    const uint32_t so = ((uint32_t)(r32_last + 1) * (uint32_t)nkb * 512u + t32 * (uint32_t)(nkb + 1) * 32u + (uint32_t)l32) * 4u;
+    const uint32_t so = t32 * (uint32_t)(nkb + 1) * 128u + 4u * (uint32_t)l32;
+    const uint32_t xo = (uint32_t)(r32_last + 1) * (uint32_t)(nkb + 1) * 128u + t32 * (uint32_t)nkb * 2048u +
+                        16u * (uint32_t)lane;
     constexpr int NP = NF / 2, TP = NB * NP;  // pairs per block and step
-    const __amdgpu_buffer_rsrc_t xr = buffer_rsrc(x, x_bytes);
+    const Src<false> xr(x, x_bytes);
     u32x4 a[RA][2];
     float xs[RA];
     auto aload = [&](int slot, int kb) {
-      const int ka = min(kb, nkb - 1);
+      const uint32_t k = (uint32_t)min(kb, nkb);
 #pragma unroll
-      for (int i = 0; i < 2; i++)
-        a[slot][i] = __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, (int)(xo + 1024u * i), (int)((uint32_t)ka * 2048u), 0));
-      xs[slot] =
-          __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(xr, (int)so, (int)((uint32_t)min(kb, nkb) * 128u), 0));
+      for (int i = 0; i < 2; i++) a[slot][i] = xr.b128(xo + 1024u * i, k * 2048u);
+      xs[slot] = __uint_as_float(xr.b32(so, k * 128u));
     };
     f32x16 p[2][2];
 #pragma unroll
@@ -605,7 +616,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(512, 512), amdgpu_waves_pe
                            : (uint32_t)min(m0 + l32, M - 1) * (uint32_t)nkb * 128u + 64u * (uint32_t)g;
     u32x4 a[RA][4];
     auto aload = [&](int slot, int kb) {
-      const ActBlock<false, false> b(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
+      const ActBlock<false> b(x, x_bytes, kb, nkb, PK ? 4096u : 128u);
 #pragma unroll
       for (int i = 0; i < 4; i++) a[slot][i] = b.x.b128(xo + (PK ? 1024u : 16u) * i, b.off);
     };
@@ -797,7 +808,7 @@ hipError_t launch_tile(int tile, const MatmulArgs& a, const void* x, void* y, in
 // elements) and the least rows of packed int8 activations (32) stay within 32-bit
 // offsets
 constexpr int64_t kMaxK32 = (int64_t)1 << 24;
-static_assert(192 * kMaxK32 <= UINT32_MAX && 32 * (2 * kMaxK32 + (kMaxK32 / 32 + 1) * 4) <= UINT32_MAX,
+static_assert(192 * kMaxK32 <= UINT32_MAX && 32 * (2 * kMaxK32 + (kMaxK32 / 32 + 1) * 4) + 2048 <= UINT32_MAX,
               "32-bit offsets");
 
 // Rows per launch: the packed copy within rq_qmatmul_noalloc's scratch, x within
