@@ -576,15 +576,15 @@ namespace rq {
 //    16.0 / 15.5; 28672 x 8192 m = 4 35.2 / 35.5; 4096 x 4096 m = 4 9.4 / 10.4).
 //  * Q8_0, weights to 32 Mi codes, m >= 9: always. This kernel carries x to 2^-17
 //    per element, that one to 2^-15 of its block's largest (2-norm error 2.5e-6
-//    against 3.2e-5), and the calls where that one is the faster are close (2048 x
-//    2048 m = 9 11.1 / 9.9; 4096 x 4096 m = 12 / 16 26.9 / 15.1; 6144 x 2048 m =
-//    12 / 16 14.9 / 17.3, 17.6 / 17.2; 11264 x 2048 m = 9 15.0 / 19.4).
+//    against 3.2e-5), and is the faster or close (in a graph, weights warm: 5632 x
+//    2048 m = 9 / 16 12.4 / 10.0, 16.4 / 10.7; 11264 x 2048 14.0 / 14.0, 18.6 / 14.6;
+//    16384 x 2048 16.6 / 14.8, 21.1 / 15.2; 4096 x 1024 8.7 / 9.4, 11.8 / 9.7).
 //  * Q8_0, rows of 3072 and more, weights to 64 Mi codes: m >= 6 with m k >= 9/4
-//    n, m = 5 with m k >= 6 n (14336 x 4096 m = 6 / 8 / 16 22.5 / 22.8, 24.3 /
-//    22.8, 37.4 / 28.7; 4096 x 14336 m = 5 / 16 28.0 / 22.8, 40.0 / 28.4; 4096 x
-//    4096 m = 5 / 6 / 8 12.4 / 12.8, 13.5 / 13.0, 16.2 / 13.1; 8192 x 8192 m = 12
-//    35.9 / 28.1; 8192 x 3072 m = 6 15.8 / 15.1; past the line 11008 x 8192 m =
-//    9 38.3 / 43.4, 28672 x 8192 m = 16 72.9 / 87.9).
+//    n, m = 5 with m k >= 6 n (14336 x 4096 m = 8 / 16 23.0 / 21.9, 36.2 / 26.7;
+//    4096 x 14336 m = 5 / 16 27.0 / 21.2, 38.5 / 27.6; 4096 x 4096 m = 6 / 8 13.0 /
+//    10.5, 15.6 / 10.6; 11008 x 4096 m = 8 / 9 20.3 / 21.2, 24.1 / 22.2, warm; cold
+//    8192 x 8192 m = 12 35.9 / 28.1; past the line 11008 x 8192 m = 9 38.3 / 43.4,
+//    28672 x 8192 m = 16 72.9 / 87.9).
 static bool mf_takes(int64_t m, int64_t k, int64_t npad, int format) {
   if (format == RQ_Q4_0) return m >= 5 || (k >= 5632 && m * k > 2 * npad);
   if (m >= 9 && npad * k <= (int64_t(32) << 20)) return true;
@@ -592,9 +592,10 @@ static bool mf_takes(int64_t m, int64_t k, int64_t npad, int format) {
          (m >= 6 ? 4 * m * k >= 9 * npad : m == 5 && m * k >= 6 * npad);
 }
 
-// Plan. The waves of a workgroup take different groups (splitting K between them measured slower at m = 16): Q4_0 16 waves with
-// an 8-step ring (two quads; at that shape 17.9 us against 18.8 for 8 waves
-// and 16 steps, and at K = 8192, N = 28672, bf16 x, 40.6 against 45.8),
+// Plan. The waves of a workgroup take different groups (splitting K between them
+// measured slower at m = 16): Q4_0 16 waves with an 8-step ring (two quads; at
+// 14336 x 4096 17.9 us against 18.8 for 8 waves and 16 steps, and at K = 8192,
+// N = 28672, bf16 x, 40.6 against 45.8),
 // Q8_0 8 waves with a 16-step ring (32 steps: 30 us with 8-byte Q4 loads);
 // ks: at least the fewest K-slices whose LDS fits two workgroups per CU, and
 // enough workgroups for ~85% of the CUs (slices of at least 8 steps): at
